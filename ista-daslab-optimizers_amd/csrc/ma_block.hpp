@@ -91,9 +91,9 @@ struct FusedParams {
     int32_t spin_limit;
 };
 
-// Extras of a block kernel (template parameter AUX, a set of bits).  Kernels with extras run
-// rarely or on request, and are compiled for any quantisation group with the register budget
-// of two workgroups per CU.
+// Extras of a block kernel (template parameter AUX, a set of bits).  Logging steps are rare: their
+// kernels are compiled for any quantisation group with the register budget of two workgroups
+// per CU.
 //   kAuxLog: a logging step (MA:155-156, :271-272, :306-308, :320-324): every block leaves the
 //            sums of its elements in its metrics slot, in the order of the reference's return
 //            value (MA:328): |quant_err|^2, |g|^2, |u|^2, |Qinv(e)|^2, zeros of u, zeros of
@@ -151,9 +151,31 @@ struct RawChunk<RegsBF16<C>> {
             v[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
         }
     }
-    __device__ __forceinline__ void from_float(const float (&v)[8]) {
-        q = make_uint4(f2bf_pair(v[0], v[1]), f2bf_pair(v[2], v[3]), f2bf_pair(v[4], v[5]),
-                       f2bf_pair(v[6], v[7]));
+    // elements 2i and 2i + 1; from_pair rounds to the element type
+    __device__ __forceinline__ void to_pair(int i, float &a, float &b) const {
+        const uint32_t w = i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w;
+        a = __uint_as_float(w << 16);
+        b = __uint_as_float(w & 0xffff0000u);
+    }
+    __device__ __forceinline__ void from_pair(int i, float a, float b) {
+        uint32_t w = f2bf_pair(a, b);
+        // (packed here and now: left to itself the compiler moves the packing to where the
+        // words are used and keeps the two floats instead)
+        asm volatile("" : "+v"(w));
+        (i == 0 ? q.x : i == 1 ? q.y : i == 2 ? q.z : q.w) = w;
+    }
+    // stores what load would read back
+    __device__ __forceinline__ void store(uint16_t *base, int off, int n, bool full) const {
+        if (full || off + kChunk <= n) {
+            typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+            const u4 t = {q.x, q.y, q.z, q.w};
+            __builtin_nontemporal_store(t, reinterpret_cast<u4 *>(base + off));
+        } else {
+            const uint32_t r[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (off + i < n) base[off + i] = (uint16_t)(r[i >> 1] >> (16 * (i & 1)));
+        }
     }
 };
 template <int C>
@@ -173,9 +195,16 @@ struct RawChunk<RegsF32<C>> {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = v_[i];
     }
-    __device__ __forceinline__ void from_float(const float (&v)[8]) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v_[i] = v[i];
+    __device__ __forceinline__ void to_pair(int i, float &a, float &b) const {
+        a = v_[2 * i];
+        b = v_[2 * i + 1];
+    }
+    __device__ __forceinline__ void from_pair(int i, float a, float b) {
+        v_[2 * i] = a;
+        v_[2 * i + 1] = b;
+    }
+    __device__ __forceinline__ void store(float *base, int off, int n, bool full) const {
+        store8(base, off, full ? 0x7fffffff : n, true, v_);
     }
 };
 
@@ -343,6 +372,10 @@ struct FusedBlock {
     // ---- parameters and the older window rows: requested early, consumed last
     __device__ __forceinline__ void load_params_window(const BlockGeo &G) {
         load_params(G);
+        load_older_rows(G);
+    }
+
+    __device__ __forceinline__ void load_older_rows(const BlockGeo &G) {
         wide = wide_window(G);
         if (wide)
             load_window_wide(G);
@@ -653,7 +686,7 @@ struct FusedBlock {
                     for (int j = 0; j < nbytes; ++j)
                         err[(off >> 1) + j] = (uint8_t)(codes >> (8 * j));
                 }
-                if constexpr (LOG || QE) quant_err_chunk(G, c, off, n, x, cf, mnf, u);
+                if constexpr (LOG || QE) quant_err_chunk(G, c, off, n, codes, mnf, u);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -663,36 +696,45 @@ struct FusedBlock {
     // gradient's type receives it (MA:267-268, :321-322): its squares for a logging step, and
     // with alpha == -2 the parameter steps p = p * decay (MA:234-235), p = p - a (MA:264),
     // p = p + d (MA:269) on the parameters held in praw, and quant_err = a - d (MA:259-270).
+    // Taken two elements at a time straight from the packed registers and the packed codes:
+    // with the chunk's values, codes, parameters and losses unpacked side by side the stage
+    // needs 40 registers more than the 80 of three workgroups per CU.
     __device__ __forceinline__ void quant_err_chunk(const BlockGeo &G, int c, int off, int n,
-                                                    const float (&x)[8], const float (&cf)[8],
-                                                    float mnf, float u) {
-        float pv[8], lost[8];
-        if constexpr (QE) praw[c].to_float(pv);
+                                                    uint32_t codes, float mnf, float u) {
+        const float decay = G.D.apply_decay != 0 ? G.D.decay : 1.0f;  // (p * 1 is p)
+        RawChunk<R> lost;
 #pragma unroll
-        for (int e = 0; e < kChunk; ++e) {
-            float deq = cf[e] * u;
-            deq = deq + mnf;
-            const float d = to_elem(0.0f + deq);
-            const bool valid = FULL || off + e < n;
-            if (valid) log_square(kMtError, d);
-            lost[e] = 0.0f;
-            if constexpr (QE) {
-                if (G.D.apply_decay != 0) pv[e] = to_elem(pv[e] * G.D.decay);
-                pv[e] = to_elem(pv[e] + (-1.0f) * x[e]);
-                pv[e] = to_elem(pv[e] + d);
-                if (valid) {
-                    lost[e] = to_elem(x[e] - d);
-                    log_square(kMtQuantErr, lost[e]);
-                    log_zero(kMtQuantErrZeros, lost[e]);
+        for (int i = 0; i < kChunk / 2; ++i) {
+            float pv[2], lo[2];
+            if constexpr (QE) praw[c].to_pair(i, pv[0], pv[1]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int e = 2 * i + j;
+                const uint32_t code = (codes >> (8 * i + (j ? 0 : 4))) & 15u;
+                float deq = (float)code * u;
+                deq = deq + mnf;
+                const float d = to_elem(0.0f + deq);
+                const bool valid = FULL || off + e < n;
+                if (valid) log_square(kMtError, d);
+                if constexpr (QE) {
+                    const float x = r.val(c, e);
+                    pv[j] = to_elem(pv[j] * decay);
+                    pv[j] = to_elem(pv[j] + (-1.0f) * x);
+                    pv[j] = pv[j] + d;
+                    lo[j] = to_elem(x - d);
+                    if (valid) {
+                        log_square(kMtQuantErr, lo[j]);
+                        log_zero(kMtQuantErrZeros, lo[j]);
+                    }
                 }
             }
+            if constexpr (QE) {
+                praw[c].from_pair(i, pv[0], pv[1]);
+                lost.from_pair(i, lo[0], lo[1]);
+            }
         }
-        if constexpr (QE) {
-            praw[c].from_float(pv);
-            // st['quant_err'] = a - Qinv(e) (MA:259-271)
-            store8(reinterpret_cast<elem_t *>(G.D.ws) + G.e0, off, FULL ? 0x7fffffff : n, true,
-                   lost);
-        }
+        // st['quant_err'] = a - Qinv(e) (MA:259-271)
+        if constexpr (QE) lost.store(reinterpret_cast<elem_t *>(G.D.ws) + G.e0, off, n, FULL);
     }
 
     // the weight decay of the update stages: with alpha == -2 it has been applied already
@@ -2173,6 +2215,13 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
             fb.load_window(G);
             fb.window_stage(G);
             fb.param_stage_dense(G);
+        } else if constexpr ((AUX & kAuxQuantErr) != 0) {
+            // the quantisation steps the parameters; the window is asked for behind it (with
+            // its entries in flight through that stage the kernel spills 74 registers)
+            fb.load_params(G);
+            fb.quantize(G);
+            fb.load_older_rows(G);
+            fb.update(G);
         } else {
             // parameters and window entries are asked for before the quantisation, which
             // hides their latency (the selection runs with more registers free without them)
@@ -2236,8 +2285,7 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
             }
         } else if constexpr (PASS == 2) {
             fb.span_load_row(G);
-            fb.wide = fb.wide_window(G);
-            if (fb.wide) fb.load_window_wide(G); else fb.load_window(G);
+            fb.load_older_rows(G);
             fb.span_load_residual(G);
             fb.span_row_to_lds(G);
             fb.template span_statistics<true>(G, S);
@@ -2623,9 +2671,9 @@ constexpr int kMinWaves = kWG / 128;  // waves per SIMD the block kernels are co
 template <class R, int QL, bool DENSE = false, int WIN = kWinFused, int AUX = 0>
 static int launch_fused_one(unsigned grid, int lds_bytes, hipStream_t s, const FusedParams &P) {
     // bf16 blocks of up to 20480 elements fit 80 registers and a third of the LDS: three
-    // workgroups per CU; the kernels with extras take the budget of two
+    // workgroups per CU; the kernels of logging steps take the budget of two
     constexpr int kWaves_ =
-        (R::kBF16 && R::kC <= kClass2 && AUX == 0) ? kWavesThreeWG : kMinWaves;
+        (R::kBF16 && R::kC <= kClass2 && (AUX & kAuxLog) == 0) ? kWavesThreeWG : kMinWaves;
     // grid == 0: the preparation of the launch only (whatever may fail apart from the launch
     // itself), so that a call can prepare all its launches before the first one starts
     if (grid == 0) return allow_big_lds(fused_step_kernel<R, kWaves_, QL, DENSE, WIN, AUX>, lds_bytes);
@@ -2633,10 +2681,19 @@ static int launch_fused_one(unsigned grid, int lds_bytes, hipStream_t s, const F
                          lds_bytes, s, P);
 }
 
-// the kernels with extras (logging, alpha == -2): one per class, any quantisation group
+// the kernels with extras (logging, alpha == -2)
 template <template <int> class RT, bool DENSE, int AUX>
 static int launch_fused_aux(int C, unsigned grid, int lds_bytes, hipStream_t s,
                             const FusedParams &P) {
+    // alpha == -2 without logging is a training step like any other and bound by memory: with the
+    // quantisation group compiled in and three workgroups per CU the 542 M-parameter bf16 list
+    // (q = 64, weight decay) takes 0.98 ms = 5.3 TB/s, with a run-time group at two 1.26 ms.
+    if constexpr (AUX == kAuxQuantErr) {
+        if (C == kClass2 && P.q_shift == 6)
+            return launch_fused_one<RT<kClass2>, 8, DENSE, kWinFused, AUX>(grid, lds_bytes, s, P);
+        if (C == kClass2 && P.q_shift == 5)
+            return launch_fused_one<RT<kClass2>, 4, DENSE, kWinFused, AUX>(grid, lds_bytes, s, P);
+    }
     switch (C) {
         case kClass0: return launch_fused_one<RT<kClass0>, 0, DENSE, kWinFused, AUX>(grid, lds_bytes, s, P);
         case kClass1: return launch_fused_one<RT<kClass1>, 0, DENSE, kWinFused, AUX>(grid, lds_bytes, s, P);
