@@ -1436,8 +1436,6 @@ struct FusedBlock {
             const uint32_t mnb = f2bf(mn), mxb = f2bf(mx);
             dstat[c] = mnb | mxb << 16;
             dcodes[c] = 0;
-            float r2[8];
-            float mn2 = INFINITY, mx2 = -INFINITY;
             const float mnf = bf2f(mnb);
             const float u = div15(bf2f(mxb) - mnf, d15);
             if (FULL || off < n) {
@@ -1447,52 +1445,31 @@ struct FusedBlock {
                 for (int e = 0; e < kChunk; ++e)
                     if (!FULL && off + e >= n) cf[e] = 0.0f;
                 dcodes[c] = pack_codes(cf);
-#pragma unroll
-                for (int e = 0; e < kChunk; ++e) {
-                    float deq = cf[e] * u;
-                    deq = deq + mnf;
-                    const float keep = P.keep * deq;
-                    r2[e] = to_elem(0.0f + keep);
-                    if (FULL || off + e < n) {
-                        mn2 = fmin_raw(mn2, r2[e]);
-                        mx2 = fmax_raw(mx2, r2[e]);
-                    }
-                }
             }
-            if (long_q) {
-                // r2 does not decrease with the code, nor the code with the element: the
-                // extremes of r2 over the quantisation block are r2 at the codes of the
-                // extremes of r, which every chunk of the block knows
-                float ext[8], ce[8];
-#pragma unroll
-                for (int e = 0; e < kChunk; ++e) ext[e] = (e & 1) ? mx : mn;
-                codes8(ext, mnf, u, ce);
-                float lo = ce[0] * u, hi = ce[1] * u;
-                lo = lo + mnf;
-                hi = hi + mnf;
-                lo = P.keep * lo;
-                hi = P.keep * hi;
-                mn2 = to_elem(0.0f + lo);
-                mx2 = to_elem(0.0f + hi);
+            // (packed here and now: left to itself the compiler moves the packing to the update
+            // and keeps the floats instead, which costs 42 spilled registers)
+            asm volatile("" : "+v"(dcodes[c]), "+v"(dstat[c]));
+            uint32_t mn2b, mx2b, codes;
+            if (requantised_alike(mn, mx, mnf, u, FULL || off < n, mn2b, mx2b)) {
+                codes = dcodes[c];
             } else {
-                group_minmax<QL>(mn2, mx2, ql);
+                requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
             }
-            const uint32_t mn2b = f2bf(mn2), mx2b = f2bf(mx2);
+            asm volatile("" : "+v"(codes), "+v"(mn2b), "+v"(mx2b));
             if (FULL || off < n) {
                 if ((lane & (ql - 1)) == 0) {
                     const unsigned qb = (unsigned)off >> q_shift;
                     mnp[qb] = (uint16_t)mn2b;
                     mxp[qb] = (uint16_t)mx2b;
                 }
-                const float m2f = bf2f(mn2b);
-                const float u2 = div15(bf2f(mx2b) - m2f, d15);
-                float cf[8];
-                codes8(r2, m2f, u2, cf);
-                log_error(cf, m2f, u2, FULL ? kChunk : n - off);
+                if constexpr (LOG) {
+                    const float m2f = bf2f(mn2b);
+                    float cf[8];
 #pragma unroll
-                for (int e = 0; e < kChunk; ++e)
-                    if (!FULL && off + e >= n) cf[e] = 0.0f;
-                const uint32_t codes = pack_codes(cf);
+                    for (int e = 0; e < kChunk; ++e)
+                        cf[e] = (float)((codes >> (8 * (e >> 1) + ((e & 1) ? 0 : 4))) & 15u);
+                    log_error(cf, m2f, div15(bf2f(mx2b) - m2f, d15), FULL ? kChunk : n - off);
+                }
                 if (FULL || off + kChunk <= n) {
                     *reinterpret_cast<uint32_t *>(err + ((unsigned)off >> 1)) = codes;
                 } else {
@@ -1502,6 +1479,96 @@ struct FusedBlock {
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    // The second quantisation of alpha > 0 maps the 16 values r2(code) = (1 - alpha) * Qinv(code)
+    // to codes again, and as r2 is linear in the code up to its rounding, code c nearly always
+    // maps to c: the rounding of r2 (2^-9 of it for bf16) would have to reach half a step, i.e.
+    // the block's values to lie many times its range away from zero.  So a quantisation block's
+    // lanes try the 16 codes between them instead of requantising their 8 elements each (q = 64:
+    // two divisions a lane instead of eight, and no second min / max).  True, for the whole
+    // wave, if every block maps every code to itself; the statistics of r2 are then r2 at the
+    // codes of the block's extremes, 0 and 15.  `valid`: this lane's chunk belongs to the block.
+    __device__ __forceinline__ bool requantised_alike(float mn, float mx, float mnf, float u,
+                                                      bool valid, uint32_t &mn2b,
+                                                      uint32_t &mx2b) const {
+        if (QL == 0 && ql < 16) return false;
+        constexpr int kPer = QL > 0 ? 16 / (QL > 0 ? QL : 1) : 1;  // codes a lane tries
+        mn2b = f2bf(kept_value(0.0f, mnf, u));
+        mx2b = f2bf(kept_value(15.0f, mnf, u));
+        const float m2f = bf2f(mn2b);
+        const float u2 = div15(bf2f(mx2b) - m2f, d15);
+        bool alike = divisor_is_plain(u) && divisor_is_plain(u2);
+        const Divisor dv2 = make_divisor(u2);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const float code = (float)((lane & ((QL > 0 ? QL : 16) - 1)) + i * (QL > 0 ? QL : 16));
+            const float y = kept_value(code, mnf, u) - m2f;
+            alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
+        }
+        if constexpr (!R::kBF16) {
+            // (bf16 extremes are their own statistics and get the codes 0 and 15)
+            const Divisor dv = make_divisor(u);
+            alike = alike && div_shared(mn - mnf, dv) + 0.5f < 1.0f &&
+                    div_shared(mx - mnf, dv) + 0.5f >= 15.0f;
+        }
+        // a range of zero: every code is 0, before and after
+        alike = alike || (u == 0.0f && fabsf(mnf) <= 3.0e38f);
+        return __builtin_amdgcn_ballot_w64(valid && !alike) == 0;
+    }
+
+    // r2 of a code: what of Qinv(code) stays in the error feedback, in the element type
+    __device__ __forceinline__ float kept_value(float code, float mnf, float u) const {
+        float deq = code * u;
+        deq = deq + mnf;
+        const float keep = P.keep * deq;
+        return to_elem(0.0f + keep);
+    }
+
+    // The second quantisation element by element: r2 from the codes of the chunk, its statistics,
+    // its codes.  Loops that stay loops: the stage is rare, and unrolled its registers are what
+    // the whole kernel would be short of.
+    __device__ __forceinline__ void requantise_chunk(int c, int off, int n, bool long_q, float mn,
+                                                     float mx, float mnf, float u, uint32_t &mn2b,
+                                                     uint32_t &mx2b, uint32_t &codes) const {
+        const int valid = FULL ? kChunk : off < n ? min(n - off, kChunk) : 0;
+        float mn2 = INFINITY, mx2 = -INFINITY;
+        auto r2_at = [&](int e) {
+            const uint32_t code = (dcodes[c] >> ((e ^ 1) * 4)) & 15u;
+            return kept_value((float)code, mnf, u);
+        };
+        if (long_q) {
+            // r2 does not decrease with the code, nor the code with the element: the
+            // extremes of r2 over the quantisation block are r2 at the codes of the
+            // extremes of r, which every chunk of the block knows
+            float ext[8], ce[8];
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e) ext[e] = (e & 1) ? mx : mn;
+            codes8(ext, mnf, u, ce);
+            mn2 = kept_value(ce[0], mnf, u);
+            mx2 = kept_value(ce[1], mnf, u);
+        } else {
+#pragma unroll 1
+            for (int e = 0; e < valid; ++e) {
+                const float v = r2_at(e);
+                mn2 = fmin_raw(mn2, v);
+                mx2 = fmax_raw(mx2, v);
+            }
+            group_minmax<QL>(mn2, mx2, ql);
+        }
+        mn2b = f2bf(mn2);
+        mx2b = f2bf(mx2);
+        codes = 0;
+        const float m2f = bf2f(mn2b);
+        const float u2 = div15(bf2f(mx2b) - m2f, d15);
+#pragma unroll 1
+        for (int e = 0; e < valid; ++e) {
+            float v[8], cf[8];
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i) v[i] = r2_at(e);  // (eight times the same)
+            codes8(v, m2f, u2, cf);
+            codes |= (uint32_t)cf[0] << ((e ^ 1) * 4);
         }
     }
 
@@ -2210,10 +2277,14 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
         fb.topk_and_row(G);
         if constexpr (WIN == kWinApart) fb.file_row_cuts(G);
         if constexpr (DENSE) {
+            // 1.07 G bf16 parameters, q = 64: 2.67 ms with codes and statistics of e1 left to the
+            // compiler (42 spilled registers), the narrow window stage and all elements
+            // quantised twice; 1.90 ms so.  (The parameters asked for before the window: the same
+            // 1.89 ms and five spilled registers.)
             fb.quantize_dense(G);
+            fb.load_older_rows(G);
+            fb.window_cells(G);
             fb.load_params(G);
-            fb.load_window(G);
-            fb.window_stage(G);
             fb.param_stage_dense(G);
         } else if constexpr ((AUX & kAuxQuantErr) != 0) {
             // the quantisation steps the parameters; the window is asked for behind it (with

@@ -179,6 +179,33 @@ def test_step_fused_densified_route(oracle, sizes, dtype, m, q, k_init, alpha, w
          expect_route=use_fused)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q,DB", [(16, 4096), (32, 20480), (64, 20480), (128, 20480), (1024, 20480)])
+def test_densified_second_quantisation(oracle, q, DB, dtype):
+    """Codes of (1 - alpha) * Qinv(code) where a code maps to itself and where it does not:
+    quantisation blocks around zero, blocks at 3, 30 and 300 times their range from zero (the
+    rounding of the kept share then moves codes) and blocks of zeros, side by side in a wave."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(23)
+    d = DB + 5 * q + 24
+    offset = torch.tensor([0.0, 0.03, 0.3, 3.0, 0.0])[torch.arange(d) // q % 5]
+    params = [(torch.randn(d, generator=gen) * 0.02).to(dtype)]
+    oparams = [to_np(params[0])]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=DB)
+    gp = torch.nn.Parameter(params[0].clone().cuda())
+    opt = MicroAdam([gp], m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
+    opt.d_block_size = DB
+    for step in range(3):
+        g = offset + torch.randn(d, generator=gen) * 0.003
+        g[torch.arange(d) // q % 5 == 4] = 0.0
+        gp.grad = g.to(dtype).cuda()
+        opt.step()
+        assert opt._fusable(gp, opt.state[gp]) == 3
+        oref.step([to_np(g.to(dtype))])
+        assert_state_equal(opt.state[gp], oref.state[0], f"step {step + 1}")
+        assert np.array_equal(to_np(gp.data), oparams[0]), f"step {step + 1}: parameters"
+
+
 @pytest.mark.parametrize("use_fused", [True, False], ids=["fused", "opbyop"])
 @pytest.mark.parametrize("scale", [1e-36, 3e-38, 1e-39])
 def test_denormal_scale_gradients(oracle, scale, use_fused):
