@@ -232,6 +232,19 @@ int64_t ma_spanning_step_workspace(const ma_tensor *tensors /* host */, int n_te
 int ma_spanning_step_check(const ma_tensor *tensor /* host */, const ma_hyper *hyper /* host */,
                             double alpha);
 
+/* One step with alpha == 0 for quantisation blocks that are a multiple of 8, at least 512 elements
+ * long and shorter than hyper->d_block_size (a tensor may be shorter than a quantisation block).
+ * p, g: contiguous, same dtype, 16-byte aligned.  g is overwritten with the residual in blocks
+ * whose neighbours were late, and left as it is elsewhere.  workspace: device memory, 16-byte
+ * aligned, at least ma_spanning_step_workspace() bytes, in no particular state.  Every array is
+ * read and written once (micro_adam.py:186-304). */
+int ma_segmented_step(const ma_tensor *tensors /* host */, int n_tensors,
+                      const ma_hyper *hyper /* host */, void *workspace, int64_t workspace_bytes,
+                      void *stream);
+
+/* 0 if ma_segmented_step would accept this tensor, else the MA_ERR_* it would return. */
+int ma_segmented_step_check(const ma_tensor *tensor /* host */, const ma_hyper *hyper /* host */);
+
 /* ma_spanning_step for callers that cannot allocate device memory or hand over a workspace
  * (tight serving loops, harnesses that forbid hipMalloc, code under HIP graph capture).  No
  * counterpart in the reference.  Same arguments, conditions and results as ma_spanning_step;

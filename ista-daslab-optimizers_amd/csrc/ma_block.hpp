@@ -2224,6 +2224,258 @@ struct FusedBlock {
         }
         span_store_statistics(G, S);
     }
+
+    // =========================================================================================
+    // Segmented route, alpha == 0: quantisation blocks of q_span elements (a multiple of 8, at
+    // least a stretch of 512) that are shorter than the top-k blocks and do not divide them.  A
+    // top-k block holds several of them whole and shares its first and its last one with the
+    // block before and behind it, with no other: only the extremes of these two parts are
+    // exchanged, the way the one-pass form of the spanning route exchanges its pairs (publish,
+    // bounded wait, deferred blocks to a second launch).  Everything else is the fused step:
+    // every array crosses HBM once, where the op-by-op sequence crosses the gradient buffer
+    // nine times and pays 8 launches per tensor (124 M bf16 parameters in 148 tensors,
+    // q = 10000, the refill of the gradient buffer included: 3.70 ms op by op, 0.32 ms so).
+    // Bound by memory like the fused step; 80 registers, three workgroups per CU.
+    // A wave's stretch of 512 elements meets at most two quantisation blocks.
+    // =========================================================================================
+    struct Segments {
+        int64_t qb0;  // quantisation block of the block's first element
+        int rem;      // elements of it in the block before
+        int count;    // quantisation blocks the block meets
+        float rq;     // 1 / q
+        int q;
+        // which of them holds offset o: (x + 0.5) / q is at least 0.5 / q away from an integer,
+        // for x < 2^17 far more than the rounding of the two operations
+        __device__ __forceinline__ int of(int o) const {
+            return (int)(((float)(rem + o) + 0.5f) * rq);
+        }
+    };
+
+    __device__ __forceinline__ Segments make_segments(const BlockGeo &G) const {
+        const int n = FULL ? C * kRound : G.n;
+        Segments S;
+        S.q = P.q_span;
+        S.qb0 = G.e0 / S.q;
+        S.rem = (int)(G.e0 - S.qb0 * S.q);
+        S.rq = __builtin_amdgcn_rcpf((float)S.q);
+        S.count = S.of(n - 1) + 1;
+        return S;
+    }
+
+    // chunk c of this wave: its first quantisation block, and whether this lane's elements
+    // belong to the next one
+    __device__ __forceinline__ int seg_chunk(const Segments &S, int c, bool &second,
+                                             bool &split) const {
+        const int first = (__builtin_amdgcn_readfirstlane(wave) * C + c) * kRowCutStep;
+        const int s0 = __builtin_amdgcn_readfirstlane(S.of(first));
+        const int bnd = (s0 + 1) * S.q - S.rem - first;  // a multiple of 8
+        second = lane * kChunk >= bnd;
+        split = bnd < kRowCutStep;
+        return s0;
+    }
+
+    __device__ __forceinline__ void seg_load_grad_inputs(const BlockGeo &G, const Segments &S) {
+        load_hint(G);
+        const int n = FULL ? C * kRound : G.n;
+        const elem_t *g = reinterpret_cast<const elem_t *>(G.D.g) + G.e0;
+        const uint8_t *err = G.D.err + (G.e0 >> 1);
+        const uint16_t *mnp = G.D.mn + S.qb0, *mxp = G.D.mx + S.qb0;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int off = chunk_off<C>(wave, c, lane);
+            graw[c].load(g, off, n, FULL);
+            cw[c] = smn[c] = smx[c] = 0;
+            if (FULL || off < n) {
+                if (FULL || off + kChunk <= n) {
+                    cw[c] = *reinterpret_cast<const uint32_t *>(err + ((unsigned)off >> 1));
+                } else {
+                    const int nbytes = (n - off + 1) >> 1;
+                    for (int j = 0; j < nbytes; ++j)
+                        cw[c] |= (uint32_t)err[(off >> 1) + j] << (8 * j);
+                }
+                bool second, split;
+                const unsigned at = (unsigned)(seg_chunk(S, c, second, split) + (second ? 1 : 0));
+                smn[c] = mnp[at];
+                smx[c] = mxp[at];
+            }
+        }
+    }
+
+    // LDS of the exchange, where the selection's histograms were: the extremes of the two parts
+    // of every (wave, chunk), then the extremes of every quantisation block, which
+    // become its (min, step)
+    static constexpr int kSegMax = 32768 / kRowCutStep + 2;
+    __device__ __forceinline__ float4 *seg_parts() const { return reinterpret_cast<float4 *>(hist); }
+    __device__ __forceinline__ float2 *seg_table() const {
+        return reinterpret_cast<float2 *>(seg_parts() + kWaves * C);
+    }
+
+    // extremes of the residual (in the registers) per quantisation block, as far as this block
+    // holds it, to seg_table; the shared ones to the workspace.  Ends with a barrier.
+    __device__ __forceinline__ void seg_extremes(const BlockGeo &G, const Segments &S) {
+        const int n = FULL ? C * kRound : G.n;
+        __syncthreads();  // the selection may still be reading its lists there
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int off = chunk_off<C>(wave, c, lane);
+            float x[8];
+            float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e) x[e] = r.val(c, e);
+            if (FULL) {
+                minmax8(x, mn, mx);
+            } else {
+#pragma unroll
+                for (int e = 0; e < kChunk; ++e) {
+                    if (off + e < n) {
+                        mn = fmin_raw(mn, x[e]);
+                        mx = fmax_raw(mx, x[e]);
+                    }
+                }
+            }
+            bool second, split;
+            seg_chunk(S, c, second, split);
+            float4 part = make_float4(second ? INFINITY : mn, second ? -INFINITY : mx,
+                                      INFINITY, -INFINITY);
+            group_minmax<0>(part.x, part.y, kWave);
+            if (split) {
+                part.z = second ? mn : INFINITY;
+                part.w = second ? mx : -INFINITY;
+                group_minmax<0>(part.z, part.w, kWave);
+            }
+            if (lane == 0) seg_parts()[wave * C + c] = part;
+        }
+        __syncthreads();
+        static_assert(kWaves * C <= kWave, "a lane per stretch");
+        for (int s = __builtin_amdgcn_readfirstlane(wave); s < S.count; s += kWaves) {
+            float mn = INFINITY, mx = -INFINITY;
+            if (lane < kWaves * C) {
+                const float4 part = seg_parts()[lane];
+                const int s0 = S.of(lane * kRowCutStep);
+                if (s0 == s) {
+                    mn = part.x;
+                    mx = part.y;
+                } else if (s0 + 1 == s) {
+                    mn = part.z;
+                    mx = part.w;
+                }
+            }
+            group_minmax<0>(mn, mx, kWave);
+            if (lane == 0) seg_table()[s] = make_float2(mn, mx);
+        }
+        __syncthreads();
+    }
+
+    // pair 0 of the block's slot: its part of its first quantisation block, pair 1: of its last
+    // (the words and the order of accesses as in span_publish)
+    __device__ __forceinline__ void seg_publish(const BlockGeo &G, const Segments &S) {
+        if (tid < 2) {
+            const float2 e = seg_table()[tid == 0 ? 0 : S.count - 1];
+            uint64_t *w = reinterpret_cast<uint64_t *>(G.D.ws + block_id(G) * kSpanWords);
+            __hip_atomic_store(w + tid,
+                               (uint64_t)__float_as_uint(e.x) |
+                                   (uint64_t)__float_as_uint(e.y) << 32,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+
+    // Takes the neighbours' parts of the shared quantisation blocks (polling at most `limit`
+    // times), then leaves (min, step) of every quantisation block in seg_table and stores the
+    // statistics of those that begin in this block.  False, for every thread and with nothing
+    // stored, if a neighbour did not publish in time (never with MUST: everything has been).
+    // Two barriers.  The statistics a block stores are read, as the last step's, by the block
+    // behind it alone, which has published, and so read them, by then.
+    template <bool MUST>
+    __device__ __forceinline__ bool seg_await(const BlockGeo &G, const Segments &S, int limit) {
+        const int n = FULL ? C * kRound : G.n;
+        const int64_t end = G.e0 + n;
+        if (wave == 0) {
+            const bool before = lane == 0 && S.rem != 0;
+            const bool behind = lane == 1 && end < G.D.d && (S.qb0 + S.count) * S.q > end;
+            bool ok = true;
+            if (before || behind) {
+                const int64_t b = block_id(G) + (before ? -1 : 1);
+                uint64_t *w = reinterpret_cast<uint64_t *>(G.D.ws + b * kSpanWords) +
+                              (before ? 1 : 0);
+                uint64_t pair = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!MUST) {
+                    while ((uint32_t)pair == 0xffffffffu && limit > 0) {
+                        __builtin_amdgcn_s_sleep(8);
+                        --limit;
+                        pair = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    ok = (uint32_t)pair != 0xffffffffu;
+                }
+                // (a full block meets two quantisation blocks at least and the last block of a
+                // tensor has no block behind it: never both lanes on one entry)
+                float2 *e = seg_table() + (before ? 0 : S.count - 1);
+                *e = make_float2(fmin_raw(e->x, __uint_as_float((uint32_t)pair)),
+                                 fmax_raw(e->y, __uint_as_float((uint32_t)(pair >> 32))));
+            }
+            const bool all_ok = __builtin_amdgcn_ballot_w64(!ok) == 0;
+            if (lane == 0) sh[kShTies] = all_ok ? 1u : 0u;
+        }
+        __syncthreads();
+        const bool all_ok = sh[kShTies] != 0;
+        if (all_ok && tid < S.count) {
+            const float2 e = seg_table()[tid];
+            const uint32_t mnb = f2bf(e.x), mxb = f2bf(e.y);
+            const float mnf = bf2f(mnb);
+            seg_table()[tid] = make_float2(mnf, div15(bf2f(mxb) - mnf, d15));
+            if (tid > 0 || S.rem == 0) {
+                G.D.mn[S.qb0 + tid] = (uint16_t)mnb;
+                G.D.mx[S.qb0 + tid] = (uint16_t)mxb;
+            }
+        }
+        __syncthreads();
+        return all_ok;
+    }
+
+    // e = Q(r) against seg_table.  Ends with a barrier: the window stage takes the LDS over.
+    __device__ __forceinline__ void seg_codes(const BlockGeo &G, const Segments &S) {
+        const int n = FULL ? C * kRound : G.n;
+        uint8_t *err = G.D.err + (G.e0 >> 1);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int off = chunk_off<C>(wave, c, lane);
+            if (FULL || off < n) {
+                bool second, split;
+                const int s0 = seg_chunk(S, c, second, split);
+                const float2 st = seg_table()[s0 + (second ? 1 : 0)];
+                float x[8], cf[8];
+                residual8<true>(c, x);
+                codes8(x, st.x, st.y, cf);
+                // an undefined element gets code 0, as asymm_block_quant gives it (left as it is
+                // it would spread over the codes it is packed with)
+#pragma unroll
+                for (int e = 0; e < kChunk; ++e) {
+                    if (R::kBF16) cf[e] = fmax_raw(cf[e], 0.0f);
+                    if (!FULL && off + e >= n) cf[e] = 0.0f;
+                }
+                const uint32_t codes = pack_codes(cf);
+                if (FULL || off + kChunk <= n) {
+                    *reinterpret_cast<uint32_t *>(err + ((unsigned)off >> 1)) = codes;
+                } else {
+                    const int nbytes = (n - off + 1) >> 1;
+                    for (int j = 0; j < nbytes; ++j)
+                        err[(off >> 1) + j] = (uint8_t)(codes >> (8 * j));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+    }
+
+    // the residual a deferred block left in the gradient buffer, back into the registers
+    __device__ __forceinline__ void seg_reload(const BlockGeo &G) {
+        span_load_residual(G);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            float v[8];
+            graw[c].to_float(v);
+            r.set_chunk(c, v);
+        }
+    }
 };
 
 // Work item of this workgroup.  The hardware hands consecutive workgroups of a launch to the
@@ -2324,6 +2576,8 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
 // (the slot of block 0 of the launch's first tensor), the i-th deferred work item is word
 // kSpanDeferItem of the i-th slot from there (the launch has at most as many work items as
 // there are slots from its first to the end of the workspace).
+// Segmented route (quantisation blocks shorter than the top-k blocks), alpha == 0, no logging:
+// PASS 7 the step, PASS 9 the codes and statistics of the blocks it deferred, listed the same way.
 // (With alpha > 0 the one-pass form was built as well and measured slower than the two passes:
 // its second half needs the registers of the second pass on top of the residual, which costs
 // the third workgroup per CU or spills, and neither pass is short of memory bandwidth by
@@ -2333,7 +2587,7 @@ constexpr int kSpanDeferItem = 4, kSpanDeferCount = 6;
 template <class R, int MIN_WAVES, int PASS, int AUX = 0>
 __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P) {
     extern __shared__ __align__(16) unsigned char lds[];
-    constexpr bool kSweep = PASS == 8;
+    constexpr bool kSweep = PASS == 8 || PASS == 9, kSegmented = PASS == 7 || PASS == 9;
     uint32_t *slots = reinterpret_cast<uint32_t *>(P.t[0].ws);
     uint32_t *defer_count = slots + kSpanDeferCount;
     // (PASS 6) this block gives up: listed for the sweep
@@ -2343,7 +2597,34 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
             slots[(int64_t)at * kSpanWords + kSpanDeferItem] = (uint32_t)item;
         }
     };
+    auto run_segmented = [&](auto &fb, const BlockGeo &G, int item) {
+        const auto S = fb.make_segments(G);
+        if constexpr (kSweep) {
+            fb.seg_reload(G);
+            fb.seg_extremes(G, S);
+            fb.template seg_await<true>(G, S, 0);
+            fb.seg_codes(G, S);
+        } else {
+            fb.seg_load_grad_inputs(G, S);
+            fb.dequant(G);
+            fb.topk_and_row(G);
+            fb.seg_extremes(G, S);
+            fb.seg_publish(G, S);
+            if (fb.template seg_await<false>(G, S, P.spin_limit)) {
+                fb.seg_codes(G, S);
+            } else {
+                fb.span_defer(G);
+                list_deferred(item);
+            }
+            fb.load_params_window(G);
+            fb.update(G);
+        }
+    };
     auto run = [&](auto &fb, const BlockGeo &G, int item) {
+        if constexpr (kSegmented) {
+            run_segmented(fb, G, item);
+            return;
+        }
         const auto S = fb.make_span(G);
         if constexpr (PASS == 1 || PASS == 4) {
             fb.span_load_grad_inputs(G, S);
@@ -2849,6 +3130,8 @@ static int launch_span_one(int pass, unsigned grid, int lds_bytes, hipStream_t s
         switch (pass) {
             MA_SPAN_CASE(6, kFirst, lds_bytes)
             MA_SPAN_CASE(8, kMinWaves, kMiscBytes)
+            MA_SPAN_CASE(7, kFirst, lds_bytes)
+            MA_SPAN_CASE(9, kMinWaves, lds_bytes)
         }
     }
 #undef MA_SPAN_CASE

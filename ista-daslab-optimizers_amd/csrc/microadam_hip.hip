@@ -518,6 +518,9 @@ static int fused_check(const ma_tensor *t, const ma_hyper *h, bool dense = false
 }
 
 constexpr int kSpanMaxBlocks = 64;  // top-k blocks one quantisation block may touch
+// LDS the segmented route's exchange takes in the union: a quadruple per stretch of 512 elements,
+// a pair per quantisation block
+constexpr int kSegmentBytes = 64 * 16 + (MA_MAX_D_BLOCK / kRowCutStep + 2) * 8;
 constexpr unsigned kSweepGroups = 256;  // workgroups of the sweep behind a one-pass launch
 
 // Polls a workgroup of the one-pass form spends at most on one neighbour's flag (each a sleep
@@ -543,6 +546,24 @@ static int span_check(const ma_tensor *t, const ma_hyper *h, double alpha) {
     const int64_t q = h->quant_block_size;
     if (q % 8 != 0 || q < g.dbs || q >= (1LL << 30)) return MA_ERR_NOT_FUSABLE;
     if ((q + g.dbs - 1) / g.dbs + 1 > kSpanMaxBlocks) return MA_ERR_NOT_FUSABLE;
+    const bool single = t->d <= h->d_block_size;
+    if (!single && g.dbs % 8 != 0) return MA_ERR_NOT_FUSABLE;
+    if (plan_lds((int)g.dbs, (int)g.k_many, h->m, h->dtype == MA_BF16 ? 2 : 4, true, false).total >
+        kLdsLimit)
+        return MA_ERR_LDS;
+    return 0;
+}
+
+// the segmented route, alpha == 0: quantisation blocks a multiple of 8, at least the 512 elements
+// of a wave's stretch and shorter than the hardware's top-k block, that the fused step does not
+// take.  A tensor shorter than a quantisation block is one.  (Below 512 a wave's stretch would meet
+// three quantisation blocks; such sizes keep the op-by-op sequence.)
+static int segmented_check(const ma_tensor *t, const ma_hyper *h) {
+    Geometry g;
+    const int rc = common_check(t, h, &g);
+    if (rc) return rc;
+    const int64_t q = h->quant_block_size;
+    if (q % 8 != 0 || q < kRowCutStep || q >= h->d_block_size) return MA_ERR_NOT_FUSABLE;
     const bool single = t->d <= h->d_block_size;
     if (!single && g.dbs % 8 != 0) return MA_ERR_NOT_FUSABLE;
     if (plan_lds((int)g.dbs, (int)g.k_many, h->m, h->dtype == MA_BF16 ? 2 : 4, true, false).total >
@@ -815,16 +836,18 @@ __global__ __launch_bounds__(kReduceThreads) void metrics_reduce_kernel(const fl
 }
 
 // aux: kAux* bits.  With kAuxLog, metrics holds kMetricSlots floats per block of the call.
+// segmented: with span, quantisation blocks shorter than the top-k blocks (alpha == 0, aux == 0).
 static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h, void *stream,
                      bool span, double alpha, void *ws, int64_t ws_bytes, int aux = 0,
-                     float *metrics = nullptr) {
+                     float *metrics = nullptr, bool segmented = false) {
     const bool dense = !span && alpha > 0.0;
     if (!tensors || !h || n_tensors < 0) return MA_ERR_ARG;
     if ((aux & kAuxQuantErr) && (span || dense)) return MA_ERR_NOT_FUSABLE;
     if ((aux & kAuxLog) && !metrics) return MA_ERR_ARG;
     for (int i = 0; i < n_tensors; ++i) {
-        const int rc =
-            span ? span_check(&tensors[i], h, alpha) : fused_check(&tensors[i], h, alpha > 0.0);
+        const int rc = segmented ? segmented_check(&tensors[i], h)
+                       : span    ? span_check(&tensors[i], h, alpha)
+                                 : fused_check(&tensors[i], h, alpha > 0.0);
         if (rc) return rc;
         if (aux & kAuxQuantErr) {  // st['quant_err'] is written with 16-byte stores
             if (!tensors[i].quant_err) return MA_ERR_ARG;
@@ -916,6 +939,7 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             P.spin_limit = span_spin_limit();
             plan.back().kind = kWholeStep;
             int rc = P.L.total > kLdsLimit ? MA_ERR_LDS : 0;
+            if (segmented && P.L.total - P.L.off_union < kSegmentBytes) rc = MA_ERR_LDS;
             if (!span && !dense && !aux && P.L.cell_bytes == 0) {
                 // a window too large for the one-pass stage: the block kernel ends with the
                 // quantisation, a second launch over the same blocks forms the update
@@ -1019,8 +1043,8 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
         } else {
             // alpha > 0 and logging steps: two passes; else one pass and the sweep over the
             // blocks it deferred
-            const int passes[2] = {alpha > 0.0 ? 1 : one_pass ? 6 : 4,
-                                   alpha > 0.0 ? 2 : one_pass ? 8 : 3};
+            const int passes[2] = {segmented ? 7 : alpha > 0.0 ? 1 : one_pass ? 6 : 4,
+                                   segmented ? 9 : alpha > 0.0 ? 2 : one_pass ? 8 : 3};
             for (int i = 0; i < 2 && rc == 0; ++i) {
                 unsigned g2 = grid;
                 if (one_pass && i == 1 && grid > kSweepGroups) g2 = kSweepGroups;
@@ -1112,6 +1136,16 @@ int64_t ma_spanning_step_workspace(const ma_tensor *tensors, int n_tensors, cons
 int ma_spanning_step(const ma_tensor *tensors, int n_tensors, const ma_hyper *h, double alpha,
                       void *workspace, int64_t workspace_bytes, void *stream) {
     return step_impl(tensors, n_tensors, h, stream, true, alpha, workspace, workspace_bytes);
+}
+
+int ma_segmented_step_check(const ma_tensor *tensor, const ma_hyper *hyper) {
+    return segmented_check(tensor, hyper);
+}
+
+int ma_segmented_step(const ma_tensor *tensors, int n_tensors, const ma_hyper *h, void *workspace,
+                      int64_t workspace_bytes, void *stream) {
+    return step_impl(tensors, n_tensors, h, stream, true, 0.0, workspace, workspace_bytes, 0,
+                     nullptr, true);
 }
 
 // ---- ma_spanning_step without a caller workspace and without any allocation -----------------

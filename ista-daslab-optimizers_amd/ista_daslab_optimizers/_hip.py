@@ -78,6 +78,9 @@ def _load():
                                                          ctypes.POINTER(MaHyper)]),
         "ma_spanning_step_check": (ci, [ctypes.POINTER(MaTensor), ctypes.POINTER(MaHyper),
                                          ctypes.c_double]),
+        "ma_segmented_step": (ci, [ctypes.POINTER(MaTensor), ci, ctypes.POINTER(MaHyper), vp, i64,
+                                   vp]),
+        "ma_segmented_step_check": (ci, [ctypes.POINTER(MaTensor), ctypes.POINTER(MaHyper)]),
         "ma_sparse_scalar_products": (ci, [i64, i64, i64, i64, i64, vp, ci, vp, vp, ci, vp, vp,
                                            i64, vp]),
         "ma_sparse_scalar_products_workspace": (ci, [i64, i64, i64, i64, i64,
@@ -101,7 +104,8 @@ EXPORTS = ("ma_error_string", "ma_get_sm_count",
            "ma_fused_step_densified",
            "ma_fused_step_quant_err", "ma_logged_step", "ma_logged_step_partials",
            "ma_spanning_step", "ma_spanning_step_static", "ma_spanning_step_workspace",
-           "ma_spanning_step_check", "ma_sparse_scalar_products",
+           "ma_spanning_step_check", "ma_segmented_step", "ma_segmented_step_check",
+           "ma_sparse_scalar_products",
            "ma_sparse_scalar_products_workspace", "ma_sparse_linear_combination",
            "ma_copy_values_typed")
 

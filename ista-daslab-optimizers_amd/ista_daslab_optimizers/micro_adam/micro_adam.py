@@ -3,12 +3,15 @@
 Same class name, constructor, attributes and per-parameter state as the optimizer of
 ista_daslab_optimizers/micro_adam/micro_adam.py (constructor :14, state :61-94); the step itself
 is carried out by gfx950 HIP kernels of libmicroadam_hip.so.  Every tensor of a step takes one
-of four routes, all of which compute micro_adam.py:146-328:
+of five routes, all of which compute micro_adam.py:146-328:
 
   fused            ma_fused_step            alpha == 0, quantisation blocks inside the top-k blocks
   fused, densified ma_fused_step_densified  0 < alpha < 1, same layout
   spanning         ma_spanning_step         0 <= alpha < 1, quantisation blocks at least as long
                                             as the top-k blocks
+  segmented        ma_segmented_step        alpha == 0, quantisation blocks of 512 elements or more
+                                            that are shorter than the top-k blocks without
+                                            dividing them
   op by op         one kernel per call of the reference's sequence: everything else
                    (alpha == -2, other quantisation block sizes, unaligned or strided tensors)
 
@@ -36,7 +39,7 @@ try:  # logging is optional here; the reference imports wandb unconditionally (m
 except Exception:  # pragma: no cover
     wandb = None
 
-OP_BY_OP, FUSED, SPANNING, FUSED_DENSIFIED, FUSED_QUANT_ERR = 0, 1, 2, 3, 4
+OP_BY_OP, FUSED, SPANNING, FUSED_DENSIFIED, FUSED_QUANT_ERR, SEGMENTED = 0, 1, 2, 3, 4, 5
 _LOGGED_ROUTE = {FUSED: _hip.MA_ROUTE_FUSED, FUSED_DENSIFIED: _hip.MA_ROUTE_DENSIFIED,
                  SPANNING: _hip.MA_ROUTE_SPANNING, FUSED_QUANT_ERR: _hip.MA_ROUTE_QUANT_ERR}
 
@@ -240,10 +243,20 @@ class MicroAdam(torch.optim.Optimizer):
             return FUSED_DENSIFIED
         if self.alpha == -2:
             return OP_BY_OP
+        if self.alpha == 0 and self._q_is_segmented() and _hip.lib.ma_segmented_step_check(
+                ctypes.byref(probe), ctypes.byref(h)) == 0:
+            return SEGMENTED
         if _hip.lib.ma_spanning_step_check(ctypes.byref(probe), ctypes.byref(h),
                                            float(self.alpha)) == 0:
             return SPANNING
         return OP_BY_OP
+
+    def _q_is_segmented(self):
+        """Quantisation blocks ma_fused_step does not take whatever the tensor's size: a list's
+        tensors shorter than one of them then ride along with the others instead of taking the
+        spanning route's launches for themselves."""
+        q = self.quant_block_size
+        return q > 4096 or q & (q - 1) != 0
 
     def _probe(self, p, st):
         """A record of p's state (with stand-ins for the buffers of a step) and the
@@ -258,7 +271,7 @@ class MicroAdam(torch.optim.Optimizer):
 
     def _fusable(self, p, st):
         """Route p takes in a step with its current gradient: 0 op by op, 1 fused, 2 spanning,
-        3 fused densified, 4 fused with alpha == -2."""
+        3 fused densified, 4 fused with alpha == -2, 5 segmented."""
         g = p.grad
         if g.dtype != p.dtype or not p.is_contiguous() or not g.is_contiguous():
             return OP_BY_OP
@@ -312,6 +325,8 @@ class MicroAdam(torch.optim.Optimizer):
                     e.p_addr, e.g_addr = p.data_ptr(), g.data_ptr()
                     if not (e.p_addr | e.g_addr) & 15:
                         route = e.route
+                        if logging_step and route == SEGMENTED:
+                            route = OP_BY_OP  # its kernels do not form the logged sums
                 if route == OP_BY_OP:
                     for key, value in self.update_step(p, lr, wd, logging_step).items():
                         totals[key] += value
@@ -362,7 +377,7 @@ class MicroAdam(torch.optim.Optimizer):
         n, h, stream = len(entries), self._hyper(dtype, self.steps), _hip.stream_ptr()
         device = entries[0].p.device
         alpha, ws_ptr, ws_len = float(self.alpha), None, 0
-        if route == SPANNING:
+        if route in (SPANNING, SEGMENTED):
             need = _hip.lib.ma_spanning_step_workspace(table.records, n, ctypes.byref(h))
             ws = self._workspace
             if ws is None or ws.numel() < need or ws.device != device:
@@ -389,6 +404,10 @@ class MicroAdam(torch.optim.Optimizer):
         elif route == FUSED_QUANT_ERR:
             rc = _hip.lib.ma_fused_step_quant_err(table.records, n, ctypes.byref(h), stream)
             _hip.check(rc, "ma_fused_step_quant_err")
+        elif route == SEGMENTED:
+            rc = _hip.lib.ma_segmented_step(table.records, n, ctypes.byref(h), ws_ptr, ws_len,
+                                            stream)
+            _hip.check(rc, "ma_segmented_step")
         else:
             rc = _hip.lib.ma_spanning_step(table.records, n, ctypes.byref(h), alpha, ws_ptr,
                                            ws_len, stream)

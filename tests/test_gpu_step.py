@@ -157,6 +157,61 @@ def test_step_spanning_route(oracle, sizes, dtype, m, q, k_init, alpha, wd, DB, 
          expect_route=use_fused)
 
 
+SEGMENTED_CASES = [
+    # quantisation blocks shorter than the top-k blocks that do not divide them: edges at every
+    # place of a wave's 512-element stretch (q = 520), more than forty of them (q = 512 with a top-k
+    # block that it does not divide), powers of two above 4096, one element of the last block in
+    # a quantisation block of its own, tensors shorter than one and tensors of one top-k block
+    ([20480 * 2 + 4096, 768, 10000, 20480], torch.bfloat16, 10, 10000, 0.01, 0.0, 0.0, 20480, 12),
+    ([20480 * 3 + 1, 1001], torch.bfloat16, 4, 1000, 0.01, 0.0, 0.01, 20480, 7),
+    ([20480 * 2 + 77, 20480 + 20000], torch.float32, 4, 16384, 0.01, 0.0, 0.01, 20480, 6),
+    ([20480 * 3 + 4096], torch.bfloat16, 4, 8192, 0.02, 0.0, 0.0, 20480, 6),
+    ([20480 * 4], torch.bfloat16, 4, 520, 0.01, 0.0, 0.0, 20480, 6),
+    ([20480 * 2 + 9], torch.float32, 3, 20472, 0.01, 0.0, 0.0, 20480, 5),
+    ([1032 * 5 + 3, 700, 24], torch.bfloat16, 3, 1000, 0.03, 0.0, 0.0, 1032, 7),
+    ([4096 * 3 + 11], torch.float32, 3, 520, 0.02, 0.0, 0.0, 4096, 6),
+    ([12288 * 2 + 8], torch.bfloat16, 3, 5000, 0.01, 0.0, 0.0, 12288, 5),
+    ([32768 * 2 + 520], torch.bfloat16, 3, 520, 0.01, 0.0, 0.0, 32768, 5),
+    ([20480 + 8192], torch.bfloat16, 20, 10000, 0.05, 0.0, 0.0, 20480, 22),
+]
+
+
+@pytest.mark.parametrize("spin", [None, "0"], ids=["exchange", "deferred"])
+@pytest.mark.parametrize("sizes,dtype,m,q,k_init,alpha,wd,DB,steps", SEGMENTED_CASES)
+def test_step_segmented_route(oracle, monkeypatch, sizes, dtype, m, q, k_init, alpha, wd, DB, steps,
+                              spin):
+    """spin "0": no block waits for its neighbours, every block that has one takes the sweep."""
+    if spin is not None:
+        monkeypatch.setenv("MA_SPAN_SPIN_LIMIT", spin)
+    opt = _run(oracle, sizes, dtype, m, q, k_init, alpha, wd, DB, steps, True, zero_step=2)
+    for p in opt.param_groups[0]["params"]:
+        assert opt._fusable(p, opt.state[p]) == 5
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_segmented_route_takes_what_the_op_by_op_route_takes(value):
+    """Infinite and undefined gradients, more of them than a top-k block selects: the same state
+    and parameters as the op-by-op sequence leaves, bit for bit."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(3)
+    d = 20480 * 2 + 4096
+    start = (torch.randn(d, generator=gen) * 0.02).to(torch.bfloat16)
+    g = (torch.randn(d, generator=gen) * 0.01).to(torch.bfloat16)
+    g[25000:25300] = value
+    states = []
+    for fused in (True, False):
+        p = torch.nn.Parameter(start.clone().cuda())
+        opt = MicroAdam([p], m=3, lr=1e-3, quant_block_size=10000)
+        opt.use_fused = fused
+        for _ in range(2):
+            p.grad = g.clone().cuda()
+            opt.step()
+        st = opt.state[p]
+        states.append([to_np(p.data)] + [to_np(st[key]) for key in ("error", "min_vals", "max_vals")])
+    for got, want in zip(*states):
+        assert np.array_equal(got, want)
+
+
 FUSED_DENSIFIED_CASES = [
     # 0 < alpha < 1 with quantisation blocks inside the top-k blocks: one pass
     ([20480 * 2 + 4096, 768, 4096], torch.bfloat16, 10, 64, 0.01, 0.5, 0.0, 20480, 12),
