@@ -17,7 +17,8 @@ namespace ma {
 namespace {
 
 constexpr int kLdsBytes = 160 * 1024;
-constexpr int kBatchRows = 16;         // rows the linear combination requests ahead
+constexpr int kRingRows = 32;          // rows the linear combination requests ahead
+constexpr int kCombineThreads = 256;  // of a workgroup in which one wave applies the rows
 constexpr int kDotUnroll = 4;          // entries a lane requests ahead in the scalar products
 
 __device__ __forceinline__ float widen(float x) { return x; }
@@ -41,6 +42,60 @@ __device__ __forceinline__ BlockSpan block_span(int64_t d, int dbs, int kbs, int
     s.len = (int)(len < dbs ? len : dbs);
     s.kb = (int)(kb < kbs ? kb : kbs);
     return s;
+}
+
+// Four window entries as they lie in memory, from any boundary an entry can lie on (the hardware
+// takes unaligned loads).
+struct __attribute__((packed, aligned(2))) IndexQuad {
+    uint32_t w[2];
+    __device__ __forceinline__ uint32_t index(int e) const {
+        return (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu;
+    }
+    // both halves: the larger of `top` and the indices in that half
+    __device__ __forceinline__ uint32_t largest(uint32_t top) const {
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        const u16x2 t = __builtin_bit_cast(u16x2, top), a = __builtin_bit_cast(u16x2, w[0]),
+                    b = __builtin_bit_cast(u16x2, w[1]);
+        return __builtin_bit_cast(
+            uint32_t, __builtin_elementwise_max(__builtin_elementwise_max(t, a), b));
+    }
+};
+template <typename TV>
+struct ValueQuad;
+template <>
+struct __attribute__((packed, aligned(2))) ValueQuad<uint16_t> {
+    uint32_t w[2];
+    __device__ __forceinline__ float value(int e) const {
+        return __uint_as_float((e & 1) ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16);
+    }
+};
+template <>
+struct __attribute__((packed, aligned(4))) ValueQuad<float> {
+    float f[4];
+    __device__ __forceinline__ float value(int e) const { return f[e]; }
+};
+
+// First of the four entries that lane l holds of a row of kb >= 4: every entry is some lane's and
+// no lane reads past the row; the last lanes hold entries that others hold too.
+__device__ __forceinline__ int quad_start(int kb, int l) { return min(4 * l, kb - 4); }
+// lanes' worth of quads, in wavefronts, that rows of kbs entries take
+inline int quad_groups(int64_t kbs) { return (int)((kbs + 255) / 256); }
+
+// 16 bytes of the dense vector += as many accumulators
+__device__ __forceinline__ void add_sixteen_bytes(float *dst, const float *acc) {
+    float4 o = *reinterpret_cast<const float4 *>(dst);
+    const float4 a = *reinterpret_cast<const float4 *>(acc);
+    o.x = o.x + a.x; o.y = o.y + a.y; o.z = o.z + a.z; o.w = o.w + a.w;
+    *reinterpret_cast<float4 *>(dst) = o;
+}
+__device__ __forceinline__ void add_sixteen_bytes(uint16_t *dst, const float *acc) {
+    uint4 o = *reinterpret_cast<const uint4 *>(dst);
+    uint32_t *w = &o.x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        w[i] = f2bf_pair(__uint_as_float(w[i] << 16) + acc[2 * i],
+                         __uint_as_float(w[i] & 0xffff0000u) + acc[2 * i + 1]);
+    *reinterpret_cast<uint4 *>(dst) = o;
 }
 
 // ---- scalar products ------------------------------------------------------------------------
@@ -133,58 +188,197 @@ __global__ __launch_bounds__(kWG) void sparse_dot_reduce_kernel(const float *par
 
 // ---- linear combination ---------------------------------------------------------------------
 // acc[c] (fp32, LDS) takes the terms coef[r] * V[r][j] of the block's coordinates row by row in
-// increasing r: the entries of one row name distinct coordinates, so a row is applied without
-// atomics, and a barrier separates rows.  With at most 512 entries per row a thread holds one
-// column of kBatchRows rows, the next batch requested before the current one is applied.
-template <typename TO, typename TV, int WG>
+// increasing r; the entries of one row name distinct coordinates, so a row is applied without
+// atomics.  The accumulators fill the LDS (two 20480-element blocks per CU), so what bounds the
+// kernel is the chain of rows.  ONE wave applies all rows of a block: the LDS operations of a wave
+// execute in program order, so a row needs no barrier behind it, only its own reads; the next
+// row's addresses and terms are formed while those are under way.  The window comes in through a
+// ring of registers, four entries a request.
+typedef __attribute__((address_space(3))) float LdsFloat;
+
+// LDS address of cell `half` (16 bits) of w: one instruction, as the kernel's dynamic LDS, which
+// the accumulators begin, is all the LDS it has and so begins at address 0
+template <int HALF>
+__device__ __forceinline__ uint32_t cell_address(uint32_t w, uint32_t two) {
+    uint32_t a;
+    if (HALF == 0)
+        asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD "
+            "src1_sel:WORD_0" : "=v"(a) : "v"(two), "v"(w));
+    else
+        asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD "
+            "src1_sel:WORD_1" : "=v"(a) : "v"(two), "v"(w));
+    return a;
+}
+
+template <typename TV, int G, int RING>
+__device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int64_t k, int m_rows,
+                                             const float *coef, const int16_t *I, const TV *V,
+                                             int lane) {
+    static_assert(RING <= 64, "a lane holds one coefficient of the ring");
+    constexpr int kStep = 4;  // rows whose indices are checked together
+    constexpr uint32_t kWide = sizeof(TV) / 2;
+    // byte offset in a row of the indices of this lane's entries
+    uint32_t start[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) start[g] = 2u * (uint32_t)quad_start(S.kb, lane + g * 64);
+    IndexQuad ix[RING][G];
+    ValueQuad<TV> v[RING][G];
+    // Requests are made in row order and at every round alike (the last row again and again
+    // behind the window's end), so that at any time the same number of them is under way and
+    // the compiler can wait for the oldest ones alone.  Rows of a round are addressed from its
+    // first one in 32 bits (the host checks that RING rows fit).
+    const uint32_t row_bytes = (uint32_t)k * 2u;
+    const int16_t *Ir = I + S.col0;
+    const TV *Vr = V + S.col0;
+    uint32_t row_at = 0, last_at = 0;
+    auto aim = [&](int first) {  // the next RING requests are for the rows from `first` on
+        const int row = first < m_rows ? first : m_rows - 1;
+        const int more = m_rows - 1 - row;
+        Ir = I + ((int64_t)row * k + S.col0);
+        Vr = V + ((int64_t)row * k + S.col0);
+        row_at = 0;
+        last_at = (uint32_t)(more < RING ? more : RING) * row_bytes;
+    };
+    auto request = [&](int slot) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            uint32_t at = start[g] + row_at;
+            asm volatile("" : "+v"(at));  // (kept a 32-bit offset from the scalar address)
+            ix[slot][g] = *reinterpret_cast<const IndexQuad *>(
+                reinterpret_cast<const char *>(Ir) + at);
+            v[slot][g] = *reinterpret_cast<const ValueQuad<TV> *>(
+                reinterpret_cast<const char *>(Vr) + (at * kWide));
+        }
+        row_at = min(row_at + row_bytes, last_at);
+    };
+    uint32_t cell[2][G][4];  // LDS addresses
+    float term[2][G][4];
+    uint32_t two = 2;
+    asm volatile("" : "+v"(two));
+    auto prepare = [&](int which, int slot, float c) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            cell[which][g][0] = cell_address<0>(ix[slot][g].w[0], two);
+            cell[which][g][1] = cell_address<1>(ix[slot][g].w[0], two);
+            cell[which][g][2] = cell_address<0>(ix[slot][g].w[1], two);
+            cell[which][g][3] = cell_address<1>(ix[slot][g].w[1], two);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                term[which][g][e] = c * v[slot][g].value(e);
+                // (formed here: left to itself the compiler moves it to where it is used,
+                // behind the wait for the reads)
+                asm volatile("" : "+v"(term[which][g][e]));
+            }
+        }
+    };
+    float x[G][4];
+    auto read = [&](int which) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[g][e] = *(LdsFloat *)(uintptr_t)cell[which][g][e];
+    };
+    // (lanes that hold the same entry write the same sum)
+    auto add_write = [&](int which) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[g][e] = x[g][e] + term[which][g][e];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) *(LdsFloat *)(uintptr_t)cell[which][g][e] = x[g][e];
+    };
+    // (the first round only requests: a request is made at one place of the code, in one order,
+    // whatever the round)
+#pragma unroll
+    for (int u = 0; u < RING; ++u)
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            ix[u][g] = IndexQuad{};
+            v[u][g] = ValueQuad<TV>{};
+        }
+    float next_coef = 0.0f;
+    for (int r0 = -RING; r0 < m_rows; r0 += RING) {
+        const float cs = next_coef;
+        next_coef = coef[r0 + RING + lane < m_rows ? r0 + RING + lane : m_rows - 1];
+        aim(r0 + RING);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s0 = 0; s0 < RING; s0 += kStep) {
+            const int row = r0 + s0;
+            uint32_t top = 0;
+#pragma unroll
+            for (int u = 0; u < kStep; ++u)
+#pragma unroll
+                for (int g = 0; g < G; ++g) top = ix[s0 + u][g].largest(top);
+            const bool stray =
+                (top & 0xffffu) >= (uint32_t)S.len || (top >> 16) >= (uint32_t)S.len;
+            const bool in_block = __builtin_amdgcn_ballot_w64(stray) == 0;
+            auto coef_of = [&](int u) {
+                return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), s0 + u));
+            };
+            if (r0 >= 0 && in_block && row + kStep <= m_rows) {
+                prepare(0, s0, coef_of(0));
+#pragma unroll
+                for (int u = 0; u < kStep; ++u) {
+                    read(u & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (u + 1 < kStep) prepare((u + 1) & 1, s0 + u + 1, coef_of(u + 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    add_write(u & 1);
+                }
+            } else if (r0 >= 0 && in_block) {  // the window's last rows
+#pragma unroll
+                for (int u = 0; u < kStep - 1; ++u) {
+                    if (row + u < m_rows) {
+                        prepare(0, s0 + u, coef_of(u));
+                        read(0);
+                        add_write(0);
+                    }
+                }
+            } else if (r0 >= 0) {
+                // an index outside the block, which is skipped: these rows entry by entry
+                for (int r = row; r < row + kStep && r < m_rows; ++r) {
+                    const int64_t first = (int64_t)r * k + S.col0;
+                    for (int j = lane; j < S.kb; j += 64) {
+                        const int i = I[first + j];
+                        const float t = coef[r] * widen(V[first + j]);
+                        if ((unsigned)i < (unsigned)S.len) acc[i] = acc[i] + t;
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kStep; ++u) {
+                request(s0 + u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+}
+
+// G == 0: rows of any length, all threads, a barrier behind every row
+template <typename TO, typename TV, int G, int WG>
 __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, int kbs,
                                                              int64_t k, int m_rows,
-                                                             const float *coef, const int16_t *I,
-                                                             const TV *V, TO *out) {
+                                                             const float *__restrict__ coef,
+                                                             const int16_t *__restrict__ I,
+                                                             const TV *__restrict__ V,
+                                                             TO *__restrict__ out) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float *acc = (float *)lds_raw;
     const BlockSpan S = block_span(d, dbs, kbs, k);
     const int tid = threadIdx.x;
-    for (int i = tid; i < S.len; i += WG) acc[i] = 0.0f;
+    for (int i = tid; i < S.len / 4; i += WG)
+        ((float4 *)acc)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (tid < (S.len & 3)) acc[(S.len & ~3) + tid] = 0.0f;
     __syncthreads();
 
-    if (S.kb <= WG) {
-        // thread tid holds column tid of kBatchRows consecutive rows.  Requests are
-        // unconditional (row and column clamped into the window) and their results stay as
-        // loaded until they are applied, so that all of a batch is in flight at once.
-        const bool mine = tid < S.kb;
-        const int16_t *Ic = I + S.col0 + (mine ? tid : 0);
-        const TV *Vc = V + S.col0 + (mine ? tid : 0);
-        int nix[kBatchRows];
-        TV nraw[kBatchRows];
-        float ncoef[kBatchRows];
-        auto request = [&](int r0) {
-#pragma unroll
-            for (int u = 0; u < kBatchRows; ++u) {
-                const int row = r0 + u < m_rows ? r0 + u : m_rows - 1;
-                nix[u] = Ic[(int64_t)row * k];
-                nraw[u] = Vc[(int64_t)row * k];
-                ncoef[u] = coef[row];
-            }
-        };
-        request(0);
-        for (int r0 = 0; r0 < m_rows; r0 += kBatchRows) {
-            int ix[kBatchRows];
-            float term[kBatchRows];
-#pragma unroll
-            for (int u = 0; u < kBatchRows; ++u) {
-                ix[u] = (mine && (unsigned)nix[u] < (unsigned)S.len) ? nix[u] : -1;
-                term[u] = ncoef[u] * widen(nraw[u]);
-            }
-            if (r0 + kBatchRows < m_rows) request(r0 + kBatchRows);
-#pragma unroll
-            for (int u = 0; u < kBatchRows; ++u) {
-                if (r0 + u < m_rows) {
-                    if (ix[u] >= 0) acc[ix[u]] = acc[ix[u]] + term[u];
-                    __syncthreads();
-                }
-            }
-        }
+    if (G > 0 && S.kb >= 4) {
+        if (tid < 64)
+            combine_rows<TV, (G > 0 ? G : 1), kRingRows / (G > 0 ? G : 1)>(acc, S, k, m_rows, coef,
+                                                                          I, V, tid);
+        __syncthreads();
     } else {
         for (int r = 0; r < m_rows; ++r) {
             const float c = coef[r];
@@ -199,7 +393,15 @@ __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, 
     }
 
     TO *dst = out + S.e0;
-    for (int i = tid; i < S.len; i += WG) narrow(dst + i, widen(dst[i]) + acc[i]);
+    int done = 0;
+    if ((((uintptr_t)dst) & 15) == 0) {
+        constexpr int kPer = 16 / sizeof(TO);
+        const int n = S.len / kPer;
+#pragma unroll 4
+        for (int i = tid; i < n; i += WG) add_sixteen_bytes(dst + i * kPer, acc + i * kPer);
+        done = n * kPer;
+    }
+    for (int i = done + tid; i < S.len; i += WG) narrow(dst + i, widen(dst[i]) + acc[i]);
 }
 
 // ---- copy_values with typed window values ---------------------------------------------------
@@ -310,18 +512,22 @@ int ma_sparse_linear_combination(int64_t d, int64_t m_rows, int64_t k, int64_t d
     const int lds = (int)(d_block_size * 4);
     if (lds > kLdsBytes) return MA_ERR_LDS;
     hipStream_t s = (hipStream_t)stream;
-    // rows of at most 256 entries go to 256-thread workgroups: a row's barrier then joins four
-    // waves instead of eight
-#define CALL_WG(TO, TV, WG)                                                                     \
-    if ((rc = allow_lds(sparse_combine_kernel<TO, TV, WG>, lds))) return rc;                    \
-    rc = launch_kernel(sparse_combine_kernel<TO, TV, WG>, dim3((unsigned)nblocks), WG, lds, s,  \
-                       d, (int)d_block_size, (int)k_block_size, k, (int)m_rows, coef, indices,  \
-                       (const TV *)values, (TO *)out);
+    // Rows of up to 512 entries per block: one wave applies them.  1248 blocks of 20480, 1024 rows
+    // of 205 bf16: 360 us against 590 with four waves and a barrier per row.  Longer rows give a
+    // barrier more to do, and a row of more than 2^25 entries does not fit the wave's offsets.
+    const int groups = k <= (1 << 25) ? quad_groups(k_block_size) : 0;
+#define CALL_G(TO, TV, G, WG)                                                                   \
+    if ((rc = allow_lds(sparse_combine_kernel<TO, TV, G, WG>, lds))) return rc;                 \
+    rc = launch_kernel(sparse_combine_kernel<TO, TV, G, WG>, dim3((unsigned)nblocks), WG, lds,  \
+                       s, d, (int)d_block_size, (int)k_block_size, k, (int)m_rows, coef,        \
+                       indices, (const TV *)values, (TO *)out);
 #define CALL(TO, TV)                                                                            \
-    if (k_block_size <= 256) { CALL_WG(TO, TV, 256) } else { CALL_WG(TO, TV, kWG) }
+    if (groups == 1) { CALL_G(TO, TV, 1, kCombineThreads) }                                     \
+    else if (groups == 2) { CALL_G(TO, TV, 2, kCombineThreads) }                                \
+    else { CALL_G(TO, TV, 0, kWG) }
     MA_DISPATCH2(out_dtype, values_dtype, CALL)
 #undef CALL
-#undef CALL_WG
+#undef CALL_G
     return rc;
 }
 
