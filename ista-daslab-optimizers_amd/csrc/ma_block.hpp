@@ -421,12 +421,12 @@ struct FusedBlock {
 
     __device__ __forceinline__ void load_hint(const BlockGeo &G) {
         hint = 0x7fffu;
-        if constexpr (FULL && R::kBF16) {
+        {
             const int prev = (G.D.row == 0 ? P.W.rows_total : G.D.row) - 1;
             const uint16_t *Vp = G.D.V + ((int64_t)prev * G.D.k + G.col0);
             if (G.kb <= kWG) {
                 if (tid < G.kb) hint = Vp[tid] & 0x7fffu;
-            } else if (G.kb <= kHintLongRow) {
+            } else if (FULL && R::kBF16 && G.kb <= kHintLongRow) {
                 for (int j = tid; j < G.kb; j += kWG) hint = min(hint, Vp[j] & 0x7fffu);
             }
         }
@@ -543,6 +543,11 @@ struct FusedBlock {
                 // the block was parked in the slot cells and every thread cleared its own
                 slot_clear = topk_done && P.L.slot_cells == C * kRound;
             }
+        } else if (kb <= kWG && P.win_apart == 0 &&
+                   P.L.total - P.L.off_union >= kHintRegBytes) {
+            // (the window kernel of the two-launch form wants its rows by coordinate)
+            topk_done = hint_topk_registers(r, kb, hint, hist, sh, sel_idx, sel_val);
+            launder(r);
         }
         row_sorted = !topk_done;  // the selections below list their entries by coordinate
         if constexpr (FULL && R::kBF16) {

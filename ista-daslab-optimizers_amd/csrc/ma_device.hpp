@@ -652,6 +652,180 @@ __device__ __forceinline__ bool hint_topk_bf16(R &r, int kb, uint32_t hint, uint
                                        L);
 }
 
+// The top-k with a lower bound known beforehand for blocks that are not parked in LDS: fp32 data,
+// and partial blocks of either type (elements past the block's end are zeros, which no bound
+// admits).  `hint` as in hint_topk_bf16; the fewer entries a block has the further its threshold
+// moves from step to step, so the bound is lowered by a thirty-second, a sixteenth, an eighth or
+// a quarter: error feedback over 300 steps, fresh gradients and recurring ones, blocks of 67 to
+// 20480 elements, had under 1 % refusals from kb = 3 on (lowered too far, the elements that pile
+// up just below the threshold overflow the lists).  Every wave lists its elements of at least L (ballots; 128 slots), a pass over the
+// listed keys in bins of 2^15 above L's finds the bin of the kb-th largest, the few entries of
+// that bin are ranked against each other by (magnitude, lowest index), and every lane clears
+// its elements from the threshold that gives.  False (uniformly, r unchanged) if the bound
+// finds fewer than kb elements, a list overflows, the kb-th largest is an octave or more above
+// L, or there is no usable hint; any hint gives the same selection or a refusal.  Entries are
+// listed above the threshold's bin in (wave, chunk, element, lane) order, then by rank.
+//   hist: kHintRegBytes of LDS; sh: the kSh* words.  Ends with a barrier.
+constexpr int kHintRegCap = 128;   // list slots per wave: two per lane
+constexpr int kHintRegTies = 256;  // entries of the threshold's bin
+constexpr int kHintRegBytes = 256 * 4 + kHintRegTies * 8 + kWaves * kHintRegCap * 6;
+template <class R>
+__device__ __forceinline__ bool hint_topk_registers(R &r, int kb, uint32_t hint, uint32_t *hist,
+                                                    uint32_t *sh, uint16_t *sel_idx,
+                                                    uint16_t *sel_val) {
+    constexpr int C = R::kC;
+    const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+    uint32_t *bins = hist, *tie_key = hist + 256, *tie_idx = tie_key + kHintRegTies;
+    uint32_t *bits = tie_idx + kHintRegTies + wave * kHintRegCap;
+    uint16_t *idx = reinterpret_cast<uint16_t *>(tie_idx + kHintRegTies + kWaves * kHintRegCap) +
+                    wave * kHintRegCap;
+    const uint32_t wmin = wave_min_to_last(hint);
+    if (lane == kWave - 1) sh[kShScan + wave] = wmin;
+    if (tid < 256) bins[tid] = 0;
+    if (tid == 0) {
+        sh[kShTies] = 0;
+        sh[kShSel + 2] = 0xffffffffu;
+    }
+    __syncthreads();
+    uint32_t hmin = 0x7fffu;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) hmin = min(hmin, sh[kShScan + w]);
+    const float lf = __uint_as_float(hmin << 16) *
+                     (kb >= 128 ? 0.96875f : kb >= 12 ? 0.9375f : kb >= 3 ? 0.875f : 0.75f);
+    // (a fresh window's rows are all zero; nothing is taken to be said by infinities)
+    if (!(lf > 1e-30f) || hmin >= 0x7f00u) return false;
+    const uint32_t L = (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(lf));
+    uint32_t filled = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int off = chunk_off<C>(wave, c, lane);
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            const float v = r.val(c, e);
+            const bool in = !(__builtin_fabsf(v) < __uint_as_float(L));  // (NaN: largest of all)
+            const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
+            if (mask != 0) {
+                const uint32_t pos = filled + mbcnt(mask);
+                if (in && pos < (uint32_t)kHintRegCap) {
+                    bits[pos] = __float_as_uint(v);
+                    idx[pos] = (uint16_t)(off + e);
+                }
+                filled += (uint32_t)__builtin_popcountll(mask);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (lane == 0) sh[kShCnts + wave] = filled;
+    // a lane takes slots 2 * lane and 2 * lane + 1 of its wave's list
+    uint32_t key[2], bin[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t p = (uint32_t)(2 * lane + i);
+        key[i] = 0;
+        bin[i] = 0;
+        if (p < filled && p < (uint32_t)kHintRegCap) {
+            key[i] = bits[p] & 0x7fffffffu;
+            bin[i] = min((key[i] - L) >> 15, 255u) + 1;  // 0: no entry
+            atomicAdd(&bins[bin[i] - 1], 1u);
+        }
+    }
+    __syncthreads();
+    uint32_t total = 0, most = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t n = sh[kShCnts + w];
+        total += n;
+        most = max(most, n);
+    }
+    if (most > (uint32_t)kHintRegCap || total < (uint32_t)kb) return false;
+    // every wave walks the bins from the top: lane l has bins 255 - 4l down to 252 - 4l
+    const uint4 four = reinterpret_cast<const uint4 *>(bins)[63 - lane];
+    const uint32_t cnt[4] = {four.w, four.z, four.y, four.x};
+    const uint32_t sum = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    const uint32_t incl = wave_incl_scan(sum, lane);
+    uint32_t above = incl - sum, pivot = 0, inside = 0, higher = 0;
+    const uint64_t here =
+        __builtin_amdgcn_ballot_w64(above < (uint32_t)kb && (uint32_t)kb <= incl);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (above < (uint32_t)kb && (uint32_t)kb <= above + cnt[i]) {
+            pivot = (uint32_t)(255 - 4 * lane - i);
+            inside = cnt[i];
+            higher = above;
+        }
+        above += cnt[i];
+    }
+    const int src = __builtin_ctzll(here);  // (total >= kb: exactly one lane)
+    pivot = (uint32_t)__builtin_amdgcn_readlane((int)pivot, src);
+    inside = (uint32_t)__builtin_amdgcn_readlane((int)inside, src);
+    higher = (uint32_t)__builtin_amdgcn_readlane((int)higher, src);
+    if (pivot == 255u || inside > (uint32_t)kHintRegTies) {
+        __syncthreads();  // other waves may still be reading the bins, which the caller takes over
+        return false;
+    }
+    const uint32_t need = (uint32_t)kb - higher;
+    // ---- the entries above the pivot's bin take places in list order; the bin's go to a list
+    uint32_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) mine += bin[i] > pivot + 1 ? 1u : 0u;
+    const uint32_t upto = wave_incl_scan(mine, lane);
+    if (lane == kWave - 1) sh[kShScan + wave] = upto;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (bin[i] == pivot + 1) {
+            const uint32_t at = atomicAdd(&sh[kShTies], 1u);
+            tie_key[at] = bits[2 * lane + i];
+            tie_idx[at] = idx[2 * lane + i];
+        }
+    }
+    __syncthreads();
+    uint32_t place = upto - mine;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+        if (w < wave) place += sh[kShScan + w];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (bin[i] > pivot + 1) {
+            sel_idx[place] = idx[2 * lane + i];
+            sel_val[place] = (uint16_t)f2bf(__uint_as_float(bits[2 * lane + i]));
+            ++place;
+        }
+    }
+    if ((uint32_t)tid < inside) {
+        const uint32_t b = tie_key[tid], k = b & 0x7fffffffu, x = tie_idx[tid];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < inside; ++j) {
+            const uint32_t kj = tie_key[j] & 0x7fffffffu;
+            rank += (kj > k || (kj == k && tie_idx[j] < x)) ? 1u : 0u;
+        }
+        if (rank < need) {
+            sel_idx[higher + rank] = (uint16_t)x;
+            sel_val[higher + rank] = (uint16_t)f2bf(__uint_as_float(b));
+        }
+        if (rank == need - 1) {
+            sh[kShSel] = k;
+            sh[kShSel + 1] = x;
+        }
+        if (rank == need) sh[kShSel + 2] = k;  // the largest that is not taken
+    }
+    __syncthreads();
+    const float T = __uint_as_float(
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)sh[kShSel]));
+    const int last = __builtin_amdgcn_readfirstlane((int)sh[kShSel + 1]);
+    const bool tied = sh[kShSel + 2] == sh[kShSel];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e)
+            if (!(__builtin_fabsf(r.val(c, e)) < T)) {
+                const int off = chunk_off<C>(wave, c, lane) + e;
+                if (!tied || __builtin_fabsf(r.val(c, e)) != T || off <= last) r.zero(c, e);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    return true;
+}
+
 // The threshold of a full bf16 block's kb largest magnitudes from a lower bound known
 // beforehand, for selections too long for the candidate lists of hint_topk_bf16 (which then
 // take compact_selected).  `hint` as there.  The elements with key >= L are counted by key - L,

@@ -719,3 +719,40 @@ def test_quantisation_rounding_boundaries(oracle, dtype, DB, q, alpha, use_fused
         assert np.array_equal(to_np(gp.data), oparams[0]), f"step {step + 1}: parameters"
     codes = oracle.unpack_codes(to_np(opt.state[gp]["error"]), d)
     assert set(np.unique(codes)) == set(range(16))
+
+
+@pytest.mark.parametrize("kind", ["ties", "jumps", "one_wave", "few"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_selection_from_the_previous_threshold(oracle, dtype, kind):
+    """fp32 blocks and partial blocks, whose selection starts from the previous row's threshold:
+    magnitudes that tie at the threshold and at every bin edge, thresholds that jump past the
+    bins in either direction, all large elements in one wave's stretch (its list overflows), and
+    fewer non-zero elements than are selected."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(17)
+    sizes = [20480 * 2 + 4096, 12288 + 700, 768, 300, 67, 9]
+    params = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in params]
+    oref = oracle.OracleMicroAdam(oparams, 4, 1e-3, 8, 0.01, 0.0, d_block_size=20480)
+    gparams = [torch.nn.Parameter(p.clone().cuda()) for p in params]
+    opt = MicroAdam(gparams, m=4, lr=1e-3, quant_block_size=8, k_init=0.01)
+    for step in range(9):
+        grads = []
+        for n in sizes:
+            g = torch.randn(n, generator=gen) * 0.01
+            if kind == "ties":
+                g = torch.randint(-4, 5, (n,), generator=gen) * 2.0 ** -8
+            elif kind == "jumps":
+                g = g * [1.0, 1.0, 3.0, 3.0, 0.3, 1.0, 1000.0, 1000.0, 1.0][step]
+            elif kind == "one_wave":
+                g[:min(n, 600)] *= 50.0
+            else:
+                g[torch.rand(n, generator=gen) > 0.005] = 0.0
+            grads.append(g.to(dtype))
+        for p, g in zip(gparams, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        oref.step([to_np(g) for g in grads])
+        for i, p in enumerate(gparams):
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
