@@ -33,9 +33,19 @@ struct BlockSpan {
     int kb;        // window entries per row in the block
 };
 
-__device__ __forceinline__ BlockSpan block_span(int64_t d, int dbs, int kbs, int64_t k) {
+// Work item of this workgroup, of `total`: the hardware deals consecutive workgroups to the 8
+// XCDs in turn, the items are dealt so that every XCD, with its own L2, walks one contiguous
+// eighth.  Neighbouring blocks' stretches of a window row share cache lines (410 bytes of 205
+// bf16 entries touch 4.2 lines of 128).
+__device__ __forceinline__ int xcd_item(int total) {
+    constexpr int kXcds = 8;
+    const int x = (int)blockIdx.x % kXcds, j = (int)blockIdx.x / kXcds;
+    const int q = total / kXcds, r = total % kXcds;
+    return x * q + (x < r ? x : r) + j;
+}
+
+__device__ __forceinline__ BlockSpan block_span(int64_t d, int dbs, int kbs, int64_t k, int64_t b) {
     BlockSpan s;
-    const int64_t b = blockIdx.x;
     s.e0 = b * dbs;
     s.col0 = b * kbs;
     const int64_t len = d - s.e0, kb = k - s.col0;
@@ -99,91 +109,197 @@ __device__ __forceinline__ void add_sixteen_bytes(uint16_t *dst, const float *ac
 }
 
 // ---- scalar products ------------------------------------------------------------------------
-// partial[b][r] = sum over the entries of row r in block b of V * g; a wave per row, the lanes'
-// sums folded by a butterfly.  The second kernel adds the blocks' partial sums in a fixed order.
-template <typename TG, typename TV>
-__global__ __launch_bounds__(kWG) void sparse_dot_kernel(int64_t d, int dbs, int kbs, int64_t k,
-                                                         int m_rows, const TG *g,
-                                                         const int16_t *I, const TV *V,
-                                                         float *partial) {
+// partial[b][r] = sum over the entries of row r in block b of V * g.  The block of g is staged in
+// LDS in its own type and is all the LDS the kernel uses, so that four workgroups with a
+// 20480-element bf16 block share a CU.  The second kernel adds the blocks' partial sums in a
+// fixed order.
+
+// Which entries of a row of kb >= 4 a lane sums: lane l < kb / 4 the four it loads, each of the
+// kb % 4 lanes behind them the last of the four it loads.  No lane reads past the row.
+struct DotQuad {
+    int start;  // first entry loaded
+    bool four;  // the first three are this lane's
+    bool last;  // the last one is
+};
+__device__ __forceinline__ DotQuad dot_quad(int kb, int l) {
+    const int full = kb >> 2, rest = kb & 3;
+    DotQuad q;
+    q.four = l < full;
+    q.last = l < full + rest;
+    q.start = q.four ? 4 * l : q.last ? 3 * full + l - 3 : 0;
+    return q;
+}
+// wavefronts of lanes that rows of up to kbs entries take (a shorter row may leave more single
+// entries: 251 take 62 + 3 lanes)
+inline int dot_groups(int64_t kbs) { return (int)((kbs + 6 + 255) / 256); }
+
+// sum over the 64 lanes, in lane 63
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ float add_from(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK,
+                                                          0xF, true));
+}
+__device__ __forceinline__ float wave_sum_to_last(float v) {
+    v = add_from<0x111>(v);       // row_shr 1, 2, 4, 8: the last lane of every 16
+    v = add_from<0x112>(v);
+    v = add_from<0x114>(v);
+    v = add_from<0x118>(v);
+    v = add_from<0x142, 0xA>(v);  // the rows' sums into the rows behind them
+    return add_from<0x143, 0xC>(v);
+}
+
+// A wave sums ROWS rows at a time, four entries a request, the next ROWS rows requested before;
+// 16 two-byte requests a lane instead took 320 us for 1 GB of window (25.6 M coordinates, 1024 rows
+// of 1 %, bf16).  The workgroups that share a block are neighbours on one XCD: 260 us, 291 with all
+// blocks' first shares before their second ones, 318 with blocks dealt to the XCDs in turn.  The
+// gathers from LDS are free (without them 291 stays 291); more rows at a time, more shares and
+// a block staged with five requests under way were slower (300, 325, 349).  G: as dot_groups; 0: rows
+// of any length, entry by entry.
+template <typename TG, typename TV, int G>
+__global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, int kbs, int64_t k,
+                                                         int m_rows, int nblocks, int shares,
+                                                         const TG *g, const int16_t *I,
+                                                         const TV *V, float *partial) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const BlockSpan S = block_span(d, dbs, kbs, k);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int item = xcd_item(nblocks * shares), block = item / shares;
+    const BlockSpan S = block_span(d, dbs, kbs, k, block);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TG *gl = (TG *)lds_raw;
 
-    const TG *src = g + S.e0;
-    constexpr int kPer16 = 16 / sizeof(TG);
-    int staged = 0;
-    if ((((uintptr_t)src) & 15) == 0) {
-        const int n16 = S.len / kPer16;
-        for (int i = tid; i < n16; i += kWG) ((uint4 *)gl)[i] = ((const uint4 *)src)[i];
-        staged = n16 * kPer16;
-    }
-    for (int i = staged + tid; i < S.len; i += kWG) gl[i] = src[i];
-    __syncthreads();
-
-    // the workgroups of one block (gridDim.y of them) share its rows; a wave takes two rows at
-    // a time so that both rows' entries are in flight together
+    // `shares` workgroups share the rows of a block
     constexpr int kWaves = kWG / 64;
-    const int per = (m_rows + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int row_lo = (int)blockIdx.y * per;
+    const int per = (m_rows + shares - 1) / shares;
+    const int row_lo = item % shares * per;
     const int row_hi = row_lo + per < m_rows ? row_lo + per : m_rows;
-    for (int r = row_lo + wave; r < row_hi; r += 2 * kWaves) {
-        const int r2 = r + kWaves;
-        const bool two = r2 < row_hi;
-        const int64_t atA = (int64_t)r * k + S.col0, atB = (int64_t)(two ? r2 : r) * k + S.col0;
-        float accA = 0.0f, accB = 0.0f;
-        for (int j0 = 0; j0 < S.kb; j0 += 64 * kDotUnroll) {
-            int ixA[kDotUnroll], ixB[kDotUnroll];
-            TV vA[kDotUnroll], vB[kDotUnroll];
+    float *dst = partial + (int64_t)block * m_rows;
+
+    auto stage = [&]() {
+        const TG *src = g + S.e0;
+        constexpr int kPer16 = 16 / sizeof(TG);
+        int staged = 0;
+        if ((((uintptr_t)src) & 15) == 0) {
+            const int n16 = S.len / kPer16;
+            for (int i = tid; i < n16; i += kWG) ((uint4 *)gl)[i] = ((const uint4 *)src)[i];
+            staged = n16 * kPer16;
+        }
+        for (int i = staged + tid; i < S.len; i += kWG) gl[i] = src[i];
+        __syncthreads();
+    };
+
+    if (G > 0 && S.kb >= 4) {
+        constexpr int GG = G > 0 ? G : 1;
+        constexpr int ROWS = 2;
+        DotQuad at[GG];
 #pragma unroll
-            for (int u = 0; u < kDotUnroll; ++u) {
-                const int j = j0 + u * 64 + lane;
-                ixA[u] = ixB[u] = -1;
-                vA[u] = vB[u] = (TV)0;
-                if (j < S.kb) {
-                    ixA[u] = I[atA + j];
-                    vA[u] = V[atA + j];
-                    if (two) {
-                        ixB[u] = I[atB + j];
-                        vB[u] = V[atB + j];
-                    }
+        for (int q = 0; q < GG; ++q) at[q] = dot_quad(S.kb, lane + q * 64);
+        IndexQuad nix[ROWS][GG];
+        ValueQuad<TV> nv[ROWS][GG];
+        auto request = [&](int r) {
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                const int row = r + u * kWaves < row_hi ? r + u * kWaves : row_hi - 1;
+                const int64_t first = (int64_t)row * k + S.col0;
+#pragma unroll
+                for (int q = 0; q < GG; ++q) {
+                    nix[u][q] = *reinterpret_cast<const IndexQuad *>(I + first + at[q].start);
+                    nv[u][q] = *reinterpret_cast<const ValueQuad<TV> *>(V + first + at[q].start);
                 }
             }
+        };
+        if (row_lo < row_hi) request(row_lo + wave);
+        stage();
+        for (int r = row_lo + wave; r < row_hi; r += ROWS * kWaves) {
+            IndexQuad ix[ROWS][GG];
+            ValueQuad<TV> v[ROWS][GG];
+            uint32_t top = 0;
 #pragma unroll
-            for (int u = 0; u < kDotUnroll; ++u) {
-                if ((unsigned)ixA[u] < (unsigned)S.len) accA += widen(vA[u]) * widen(gl[ixA[u]]);
-                if ((unsigned)ixB[u] < (unsigned)S.len) accB += widen(vB[u]) * widen(gl[ixB[u]]);
+            for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+                for (int q = 0; q < GG; ++q) {
+                    ix[u][q] = nix[u][q];
+                    v[u][q] = nv[u][q];
+                    top = ix[u][q].largest(top);
+                }
+            request(r + ROWS * kWaves);
+            const bool stray =
+                (top & 0xffffu) >= (uint32_t)S.len || (top >> 16) >= (uint32_t)S.len;
+            const bool in_block = __builtin_amdgcn_ballot_w64(stray) == 0;
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                float sum = 0.0f;
+#pragma unroll
+                for (int q = 0; q < GG; ++q) {
+                    float t[4];
+                    if (in_block) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            t[e] = v[u][q].value(e) * widen(gl[ix[u][q].index(e)]);
+                    } else {  // an index outside the block contributes nothing
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t i = ix[u][q].index(e);
+                            t[e] = 0.0f;
+                            if (i < (uint32_t)S.len) t[e] = v[u][q].value(e) * widen(gl[i]);
+                        }
+                    }
+                    const float three = t[0] + t[1] + t[2];
+                    sum += (at[q].four ? three : 0.0f) + (at[q].last ? t[3] : 0.0f);
+                }
+                sum = wave_sum_to_last(sum);
+                if (lane == 63 && r + u * kWaves < row_hi) dst[r + u * kWaves] = sum;
             }
         }
+    } else {
+        stage();
+        for (int r = row_lo + wave; r < row_hi; r += kWaves) {
+            const int64_t first = (int64_t)r * k + S.col0;
+            float acc = 0.0f;
+            for (int j0 = 0; j0 < S.kb; j0 += 64 * kDotUnroll) {
+                int ix[kDotUnroll];
+                TV v[kDotUnroll];
 #pragma unroll
-        for (int s = 32; s > 0; s >>= 1) {
-            accA += __shfl_xor(accA, s, 64);
-            accB += __shfl_xor(accB, s, 64);
-        }
-        // straight to the workspace: LDS holds the block of g and nothing else, so that four
-        // workgroups with a 20480-element bf16 block share a CU
-        if (lane == 0) {
-            float *dst = partial + (int64_t)blockIdx.x * m_rows;
-            dst[r] = accA;
-            if (two) dst[r2] = accB;
+                for (int u = 0; u < kDotUnroll; ++u) {
+                    const int j = j0 + u * 64 + lane;
+                    ix[u] = -1;
+                    v[u] = (TV)0;
+                    if (j < S.kb) {
+                        ix[u] = I[first + j];
+                        v[u] = V[first + j];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kDotUnroll; ++u)
+                    if ((unsigned)ix[u] < (unsigned)S.len) acc += widen(v[u]) * widen(gl[ix[u]]);
+            }
+            acc = wave_sum_to_last(acc);
+            if (lane == 63) dst[r] = acc;
         }
     }
 }
 
-// out[r] += sum over blocks of partial[b][r]: a wave per row, lane l adds blocks l, l + 64, ...
-// in increasing order, then the butterfly
+// out[r] += sum over blocks of partial[b][r]: 16 rows per workgroup (a read covers 64 contiguous
+// bytes), thread (part, row) adds blocks part, part + 32, ..., then the parts in order.
+constexpr int kReduceRows = 16, kReduceParts = kWG / kReduceRows;
 __global__ __launch_bounds__(kWG) void sparse_dot_reduce_kernel(const float *partial,
                                                                 int64_t nblocks, int m_rows,
                                                                 float *out) {
-    const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * (kWG / 64) + (threadIdx.x >> 6);
-    if (r >= m_rows) return;
+    __shared__ float part[kReduceParts][kReduceRows];
+    const int rl = threadIdx.x % kReduceRows, p = threadIdx.x / kReduceRows;
+    const int r = (int)blockIdx.x * kReduceRows + rl;
     float acc = 0.0f;
-    for (int64_t b = lane; b < nblocks; b += 64) acc += partial[b * m_rows + r];
+    if (r < m_rows) {
+#pragma unroll 8
+        for (int64_t b = p; b < nblocks; b += kReduceParts) acc += partial[b * m_rows + r];
+    }
+    part[p][rl] = acc;
+    __syncthreads();
+    if (p == 0 && r < m_rows) {
+        float sum = 0.0f;
 #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s, 64);
-    if (lane == 0) out[r] = out[r] + acc;
+        for (int i = 0; i < kReduceParts; ++i) sum += part[i][rl];
+        out[r] = out[r] + sum;
+    }
 }
 
 // ---- linear combination ---------------------------------------------------------------------
@@ -367,7 +483,7 @@ __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, 
                                                              TO *__restrict__ out) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     float *acc = (float *)lds_raw;
-    const BlockSpan S = block_span(d, dbs, kbs, k);
+    const BlockSpan S = block_span(d, dbs, kbs, k, xcd_item((int)gridDim.x));
     const int tid = threadIdx.x;
     for (int i = tid; i < S.len / 4; i += WG)
         ((float4 *)acc)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -486,15 +602,22 @@ int ma_sparse_scalar_products(int64_t d, int64_t m_rows, int64_t k, int64_t d_bl
     int64_t gy = (4096 + nblocks - 1) / nblocks, gy_max = m_rows / 64;
     gy = gy > gy_max ? gy_max : gy;
     gy = gy < 1 ? 1 : gy;
+    const int groups = dot_groups(k_block_size);
+#define CALL_G(TG, TV, G)                                                                       \
+    if ((rc = allow_lds(sparse_dot_kernel<TG, TV, G>, lds))) return rc;                         \
+    rc = launch_kernel(sparse_dot_kernel<TG, TV, G>, dim3((unsigned)(nblocks * gy)), kWG, lds,  \
+                       s, d, (int)d_block_size, (int)k_block_size, k, (int)m_rows,              \
+                       (int)nblocks, (int)gy, (const TG *)g, indices, (const TV *)values,       \
+                       partial);
 #define CALL(TG, TV)                                                                            \
-    if ((rc = allow_lds(sparse_dot_kernel<TG, TV>, lds))) return rc;                            \
-    rc = launch_kernel(sparse_dot_kernel<TG, TV>, dim3((unsigned)nblocks, (unsigned)gy), kWG,   \
-                       lds, s, d, (int)d_block_size, (int)k_block_size, k, (int)m_rows,         \
-                       (const TG *)g, indices, (const TV *)values, partial);
+    if (groups == 1) { CALL_G(TG, TV, 1) }                                                      \
+    else if (groups == 2) { CALL_G(TG, TV, 2) }                                                 \
+    else { CALL_G(TG, TV, 0) }
     MA_DISPATCH2(g_dtype, values_dtype, CALL)
 #undef CALL
+#undef CALL_G
     if (rc) return rc;
-    const unsigned rgrid = (unsigned)((m_rows + kWG / 64 - 1) / (kWG / 64));
+    const unsigned rgrid = (unsigned)((m_rows + kReduceRows - 1) / kReduceRows);
     return launch_kernel(sparse_dot_reduce_kernel, dim3(rgrid), kWG, 0, s, partial, nblocks,
                          (int)m_rows, out);
 }

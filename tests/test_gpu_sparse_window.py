@@ -196,3 +196,44 @@ def test_resnet50_sized_window_properties(mods, hip_lib):
     assert torch.allclose(torch.diagonal(gram), diag, rtol=1e-5)
     scale = torch.sqrt(diag[:, None] * diag[None, :])
     assert torch.all((gram - gram.T).abs() <= 1e-5 * scale)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kb", [1, 3, 4, 5, 250, 251, 255, 256, 257, 506, 507, 512, 513])
+def test_row_lengths_at_the_edges(mods, oracle, dtype, kb):
+    """Block rows at the edges of what a wave takes four entries at a time, with a shorter last
+    block, row counts off the batches of four and thirty-two, and indices outside the block
+    (skipped) in some rows: first and last entries among them."""
+    _, smf = mods
+    dbs, rows, m = 1024, 39, 41
+    tail = max(1, kb - 2)
+    d, k = dbs * 2 + max(tail, 600), 2 * kb + tail
+    gen = torch.Generator().manual_seed(kb)
+    lens = [dbs, dbs, d - 2 * dbs]
+    cols = [torch.rand(m, ln, generator=gen).argsort(dim=1)[:, :kk]
+            for ln, kk in zip(lens, (kb, kb, tail))]
+    I = torch.cat(cols, dim=1).to(torch.int16)
+    V = torch.randn(I.shape, generator=gen).to(dtype)
+    clean = I.clone()
+    for r, c in ((0, 0), (5, kb - 1), (13, k - 1), (38, kb)):
+        I[r, c] = -3 if r % 2 else 1500  # outside every block
+    coef = torch.randn(m, generator=gen)
+    g = torch.randn(d, generator=gen).to(dtype)
+    bf16 = int(dtype == torch.bfloat16)
+    # the oracle takes no such index: it gets the row's own index and a value of zero
+    Vz = V.clone()
+    Vz[I != clean] = 0
+    want = to_np(torch.zeros(d, dtype=dtype))
+    oracle.sparse_linear_combination(d, rows, k, dbs, kb, coef.numpy(), to_np(clean), to_np(Vz), want)
+    out = torch.zeros(d, dtype=dtype, device="cuda")
+    smf.LCG(0, 0, 51, d, rows, k, dbs, kb, coef.cuda(), I.cuda(), V.cuda(), out, bf16)
+    assert np.array_equal(to_np(out), want)
+    want = np.zeros(m)
+    oracle.sparse_scalar_products(d, rows, k, dbs, kb, to_np(g), to_np(clean), to_np(Vz), want)
+    pos = (torch.arange(k) // kb) * dbs + clean.long()
+    mass = (Vz.double().abs() * g.double()[pos].abs()).sum(dim=1).numpy()
+    dots = torch.zeros(m, dtype=torch.float32, device="cuda")
+    smf.SP(0, 0, 23, d, rows, k, dbs, kb, g.cuda(), I.cuda(), V.cuda(), dots, bf16)
+    got = dots.cpu().numpy()
+    assert np.all(np.abs(got[:rows] - want[:rows]) <= SP_TOL * mass[:rows] + 1e-30)
+    assert np.all(got[rows:] == 0)
