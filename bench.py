@@ -290,7 +290,7 @@ class LaunchEvents:
     whole also count the host's work of a step whenever the stream is empty, which is the case
     for the first steps after the synchronisation that starts the timed region."""
     ENTRY_POINTS = ("ma_fused_step", "ma_fused_step_densified", "ma_fused_step_quant_err",
-                    "ma_spanning_step", "ma_logged_step")
+                    "ma_spanning_step", "ma_segmented_step", "ma_logged_step")
 
     def __init__(self):
         import torch

@@ -756,3 +756,53 @@ def test_selection_from_the_previous_threshold(oracle, dtype, kind):
         for i, p in enumerate(gparams):
             assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
             assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+
+
+def test_steps_of_one_table_follow_what_changes_between_them(oracle):
+    """Once all tensors of a list took one table, the next step refreshes it in whole columns;
+    what may change between steps is followed all the same: new gradient tensors, lr and weight
+    decay per group, a missing gradient, a gradient that is not 16-byte aligned, a parameter whose
+    storage moved, state cast to another type, an op-by-op step in between."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(29)
+    sizes = [20480 + 4096, 768, 4096, 1024]
+    cpu = [(torch.randn(n, generator=gen) * 0.02).to(torch.bfloat16) for n in sizes]
+    oparams = [to_np(p) for p in cpu]
+    gparams = [torch.nn.Parameter(p.clone().cuda()) for p in cpu]
+    opt = MicroAdam([dict(params=gparams[:2]), dict(params=gparams[2:], weight_decay=0.1)], m=3,
+                    lr=1e-3, quant_block_size=64)
+    orefs = [oracle.OracleMicroAdam(oparams[:2], 3, 1e-3, 64, 0.01, 0.0, d_block_size=20480),
+             oracle.OracleMicroAdam(oparams[2:], 3, 1e-3, 64, 0.01, 0.0, weight_decay=0.1,
+                                    d_block_size=20480)]
+    for s in range(12):
+        grads = [(torch.randn(n, generator=gen) * 1e-2).to(torch.bfloat16) for n in sizes]
+        lrs = [1e-3 * (1 + s), 2e-3]
+        for group, lr in zip(opt.param_groups, lrs):
+            group['lr'] = lr
+        if s == 3:
+            grads[1] = None
+        for i, (p, g) in enumerate(zip(gparams, grads)):
+            if g is None:
+                p.grad = None
+                continue
+            p.grad = g.clone().cuda()
+            if s == 6 and i == 0:  # an address 2 bytes off
+                buf = torch.zeros(sizes[0] + 1, dtype=torch.bfloat16, device="cuda")
+                buf[1:] = p.grad
+                p.grad = buf[1:]
+        if s == 7:
+            gparams[3].data = gparams[3].data.clone()
+        if s == 8:
+            opt.state[gparams[0]]['I'] = opt.state[gparams[0]]['I'].to(torch.int32)
+        opt.use_fused = s != 9
+        opt.step()
+        want = [None if g is None else to_np(g) for g in grads]
+        for ref, lo, hi, lr in ((orefs[0], 0, 2, lrs[0]), (orefs[1], 2, 4, lrs[1])):
+            ref.step(want[lo:hi], lr=lr)
+        for i, p in enumerate(gparams):
+            ref = orefs[i // 2].state[i % 2]
+            if ref is not None:
+                assert_state_equal(opt.state[p], ref, f"step {s + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (s, i)
+        if s in (2, 4, 11):
+            assert opt._uniform is not None
