@@ -114,24 +114,8 @@ __device__ __forceinline__ void add_sixteen_bytes(uint16_t *dst, const float *ac
 // 20480-element bf16 block share a CU.  The second kernel adds the blocks' partial sums in a
 // fixed order.
 
-// Which entries of a row of kb >= 4 a lane sums: lane l < kb / 4 the four it loads, each of the
-// kb % 4 lanes behind them the last of the four it loads.  No lane reads past the row.
-struct DotQuad {
-    int start;  // first entry loaded
-    bool four;  // the first three are this lane's
-    bool last;  // the last one is
-};
-__device__ __forceinline__ DotQuad dot_quad(int kb, int l) {
-    const int full = kb >> 2, rest = kb & 3;
-    DotQuad q;
-    q.four = l < full;
-    q.last = l < full + rest;
-    q.start = q.four ? 4 * l : q.last ? 3 * full + l - 3 : 0;
-    return q;
-}
-// wavefronts of lanes that rows of up to kbs entries take (a shorter row may leave more single
-// entries: 251 take 62 + 3 lanes)
-inline int dot_groups(int64_t kbs) { return (int)((kbs + 6 + 255) / 256); }
+// wavefronts of lanes that rows of up to kbs entries take, with one entry before the first
+inline int dot_groups(int64_t kbs) { return (int)((kbs + 1 + 255) / 256); }
 
 // sum over the 64 lanes, in lane 63
 template <int CTRL, int ROW_MASK = 0xF>
@@ -148,13 +132,13 @@ __device__ __forceinline__ float wave_sum_to_last(float v) {
     return add_from<0x143, 0xC>(v);
 }
 
-// A wave sums ROWS rows at a time, four entries a request, the next ROWS rows requested before;
-// 16 two-byte requests a lane instead took 320 us for 1 GB of window (25.6 M coordinates, 1024 rows
-// of 1 %, bf16).  The workgroups that share a block are neighbours on one XCD: 260 us, 291 with all
-// blocks' first shares before their second ones, 318 with blocks dealt to the XCDs in turn.  The
-// gathers from LDS are free (without them 291 stays 291); more rows at a time, more shares and
-// a block staged with five requests under way were slower (300, 325, 349).  G: as dot_groups; 0: rows
-// of any length, entry by entry.
+// A wave sums ROWS rows at a time, four entries a request, the next ROWS rows requested before.
+// What bounds it is how the window's 1 GB (25.6 M coordinates, 1024 rows of 1 %, bf16) is asked for:
+// 16 two-byte requests a lane took 309 us; eight bytes a request with the workgroups of a block
+// and of its neighbours on one XCD 260; the same from 4-byte boundaries 223 (4.7 TB/s).  The
+// gathers from LDS are hidden behind it; four rows at a time and more or fewer workgroups a
+// block were no faster (225 to 237), a block of g staged with five requests under way slower.
+// G: as dot_groups; 0: rows of any length, entry by entry.
 template <typename TG, typename TV, int G>
 __global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, int kbs, int64_t k,
                                                          int m_rows, int nblocks, int shares,
@@ -190,20 +174,46 @@ __global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, 
     if (G > 0 && S.kb >= 4) {
         constexpr int GG = G > 0 ? G : 1;
         constexpr int ROWS = 2;
-        DotQuad at[GG];
+        // Lane l takes the entries 4l .. 4l + 3 of a row's stretch, all one less if the stretch
+        // begins on an odd entry: every load is 4-byte aligned then, where unaligned ones kept the
+        // kernel at 260 us.  The outermost loads reach up to three entries into the neighbouring
+        // stretches, whose terms are dropped; where the array may end behind the block the lanes
+        // load from the stretch's own boundaries, aligned or not.
+        const bool exact = S.col0 + S.kb + 3 > k;
+        uint32_t from[GG];     // entry the lane's loads start at, from the row's first one
+        bool own[2][GG][4];    // by the row's parity: which of the four are this lane's
 #pragma unroll
-        for (int q = 0; q < GG; ++q) at[q] = dot_quad(S.kb, lane + q * 64);
+        for (int q = 0; q < GG; ++q) {
+            const int l = lane + q * 64;
+            from[q] = (uint32_t)(exact ? min(4 * l, S.kb - 4) : 4 * l < S.kb + 1 ? 4 * l : 0);
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int at = (int)from[q] - odd + e, lo = 4 * l - odd;
+                    own[odd][q][e] = at >= lo && at < lo + 4 && at >= 0 && at < S.kb;
+                }
+        }
+        auto first_of = [&](int r, int u) {
+            const int row = r + u * kWaves < row_hi ? r + u * kWaves : row_hi - 1;
+            return (int64_t)row * k + S.col0;
+        };
         IndexQuad nix[ROWS][GG];
         ValueQuad<TV> nv[ROWS][GG];
         auto request = [&](int r) {
 #pragma unroll
             for (int u = 0; u < ROWS; ++u) {
-                const int row = r + u * kWaves < row_hi ? r + u * kWaves : row_hi - 1;
-                const int64_t first = (int64_t)row * k + S.col0;
+                int64_t first = first_of(r, u);
+                if (!exact) first &= ~(int64_t)1;
 #pragma unroll
                 for (int q = 0; q < GG; ++q) {
-                    nix[u][q] = *reinterpret_cast<const IndexQuad *>(I + first + at[q].start);
-                    nv[u][q] = *reinterpret_cast<const ValueQuad<TV> *>(V + first + at[q].start);
+                    uint32_t at = from[q] * 2u;
+                    asm volatile("" : "+v"(at));  // (kept a 32-bit offset from the scalar address)
+                    nix[u][q] = *reinterpret_cast<const IndexQuad *>(
+                        reinterpret_cast<const char *>(I + first) + at);
+                    nv[u][q] = *reinterpret_cast<const ValueQuad<TV> *>(
+                        reinterpret_cast<const char *>(V + first) +
+                        at * (uint32_t)(sizeof(TV) / 2));
                 }
             }
         };
@@ -225,29 +235,39 @@ __global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, 
             const bool stray =
                 (top & 0xffffu) >= (uint32_t)S.len || (top >> 16) >= (uint32_t)S.len;
             const bool in_block = __builtin_amdgcn_ballot_w64(stray) == 0;
+            float sum[ROWS];
+            if (in_block) {
 #pragma unroll
-            for (int u = 0; u < ROWS; ++u) {
-                float sum = 0.0f;
+                for (int u = 0; u < ROWS; ++u) {
+                    const bool odd = !exact && (first_of(r, u) & 1) != 0;
+                    sum[u] = 0.0f;
 #pragma unroll
-                for (int q = 0; q < GG; ++q) {
-                    float t[4];
-                    if (in_block) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            t[e] = v[u][q].value(e) * widen(gl[ix[u][q].index(e)]);
-                    } else {  // an index outside the block contributes nothing
+                    for (int q = 0; q < GG; ++q) {
+                        float t[4];
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const uint32_t i = ix[u][q].index(e);
-                            t[e] = 0.0f;
-                            if (i < (uint32_t)S.len) t[e] = v[u][q].value(e) * widen(gl[i]);
+                            t[e] = v[u][q].value(e) * widen(gl[ix[u][q].index(e)]);
+                            t[e] = (odd ? own[1][q][e] : own[0][q][e]) ? t[e] : 0.0f;
                         }
+                        sum[u] += (t[0] + t[1]) + (t[2] + t[3]);
                     }
-                    const float three = t[0] + t[1] + t[2];
-                    sum += (at[q].four ? three : 0.0f) + (at[q].last ? t[3] : 0.0f);
                 }
-                sum = wave_sum_to_last(sum);
-                if (lane == 63 && r + u * kWaves < row_hi) dst[r + u * kWaves] = sum;
+            } else {  // an index outside the block contributes nothing
+#pragma unroll
+                for (int u = 0; u < ROWS; ++u) {
+                    const int64_t first = first_of(r, u);
+                    sum[u] = 0.0f;
+                    for (int j = lane; j < S.kb; j += 64) {
+                        const int i = I[first + j];
+                        if ((unsigned)i < (unsigned)S.len)
+                            sum[u] += widen(V[first + j]) * widen(gl[i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                const float all = wave_sum_to_last(sum[u]);
+                if (lane == 63 && r + u * kWaves < row_hi) dst[r + u * kWaves] = all;
             }
         }
     } else {
@@ -602,7 +622,9 @@ int ma_sparse_scalar_products(int64_t d, int64_t m_rows, int64_t k, int64_t d_bl
     int64_t gy = (4096 + nblocks - 1) / nblocks, gy_max = m_rows / 64;
     gy = gy > gy_max ? gy_max : gy;
     gy = gy < 1 ? 1 : gy;
-    const int groups = dot_groups(k_block_size);
+    // (arrays of two-byte elements that do not begin on four bytes: entry by entry)
+    const int groups =
+        (((uintptr_t)indices | (uintptr_t)values) & 3) == 0 ? dot_groups(k_block_size) : 0;
 #define CALL_G(TG, TV, G)                                                                       \
     if ((rc = allow_lds(sparse_dot_kernel<TG, TV, G>, lds))) return rc;                         \
     rc = launch_kernel(sparse_dot_kernel<TG, TV, G>, dim3((unsigned)(nblocks * gy)), kWG, lds,  \
