@@ -215,8 +215,8 @@ int ma_fused_step_densified(const ma_tensor *tensors /* host */, int n_tensors,
  * MA:190-316).
  * The caller advances st['index'] itself.  Conditions (else MA_ERR_NOT_FUSABLE, nothing
  * launched): 0 <= alpha < 1 (MA:18); quant_block_size a multiple of 8, not below
- * min(d, d_block_size), below 2^30 and covering at most 62 top-k blocks; alignment as for
- * ma_fused_step.
+ * min(d, d_block_size), below 2^30 and covering at most 62 of the tensor's top-k blocks
+ * (any number of lengths of a tensor that is one block); alignment as for ma_fused_step.
  * workspace: device memory, 16-byte aligned, at least ma_spanning_step_workspace() bytes,
  * owned by the caller; its contents need not survive between calls. */
 int ma_spanning_step(const ma_tensor *tensors /* host */, int n_tensors,

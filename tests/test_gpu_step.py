@@ -806,3 +806,14 @@ def test_steps_of_one_table_follow_what_changes_between_them(oracle):
             assert np.array_equal(to_np(p.data), oparams[i]), (s, i)
         if s in (2, 4, 11):
             assert opt._uniform is not None
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.5])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q", [50000, 100000, 1 << 20])
+def test_spanning_route_takes_short_vectors(oracle, q, dtype, alpha):
+    """Tensors of a single top-k block under quantisation blocks more than 62 times as long: all
+    the quantisation block covers is that one block (q = 2^20 with single-block tensors only)."""
+    sizes = [768, 125, 80, 9, 20480] + ([20480 * 2 + 77] if q < 1 << 20 else [])
+    _run(oracle, sizes, dtype, 3, q, 0.01, alpha, 0.01, 20480, 5, True, zero_step=2,
+         expect_route=True)
