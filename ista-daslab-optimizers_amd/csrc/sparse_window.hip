@@ -5,8 +5,8 @@
 //   linear combination of the rows into a dense vector
 //     (ista_daslab_cuda_sparse_mfac.LCG, sparse_core_mfac_w_ef.py:205-221),
 //   copy_values with fp32 window values (sparse_core_mfac_w_ef.py:105-124, use_bf16 = False).
-// One 512-thread workgroup per top-k block: the block of the dense vector lives in LDS, the
-// window entries of the block stream past it once.  Part of libmicroadam_hip.so.
+// A workgroup works on one top-k block: the block of the dense vector lives in LDS, the window
+// entries of the block stream past it once.  Part of libmicroadam_hip.so.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
