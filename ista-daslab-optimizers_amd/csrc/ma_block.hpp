@@ -1455,7 +1455,10 @@ struct FusedBlock {
             // and keeps the floats instead, which costs 42 spilled registers)
             asm volatile("" : "+v"(dcodes[c]), "+v"(dstat[c]));
             uint32_t mn2b, mx2b, codes;
-            if (requantised_alike(mn, mx, mnf, u, FULL || off < n, mn2b, mx2b)) {
+            // (a quantisation block that begins inside the block counts with all its lanes: those
+            // past the end hold no elements, but try codes that the others' elements may have)
+            const bool begun = FULL || (off & -(1 << q_shift)) < n;
+            if (requantised_alike(mn, mx, mnf, u, begun, mn2b, mx2b)) {
                 codes = dcodes[c];
             } else {
                 requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
@@ -1494,9 +1497,10 @@ struct FusedBlock {
     // lanes try the 16 codes between them instead of requantising their 8 elements each (q = 64:
     // two divisions a lane instead of eight, and no second min / max).  True, for the whole
     // wave, if every block maps every code to itself; the statistics of r2 are then r2 at the
-    // codes of the block's extremes, 0 and 15.  `valid`: this lane's chunk belongs to the block.
+    // codes of the block's extremes, 0 and 15.  `counts`: this lane's quantisation block has
+    // elements, be they other lanes' alone.
     __device__ __forceinline__ bool requantised_alike(float mn, float mx, float mnf, float u,
-                                                      bool valid, uint32_t &mn2b,
+                                                      bool counts, uint32_t &mn2b,
                                                       uint32_t &mx2b) const {
         if (QL == 0 && ql < 16) return false;
         constexpr int kPer = QL > 0 ? 16 / (QL > 0 ? QL : 1) : 1;  // codes a lane tries
@@ -1520,7 +1524,7 @@ struct FusedBlock {
         }
         // a range of zero: every code is 0, before and after
         alike = alike || (u == 0.0f && fabsf(mnf) <= 3.0e38f);
-        return __builtin_amdgcn_ballot_w64(valid && !alike) == 0;
+        return __builtin_amdgcn_ballot_w64(counts && !alike) == 0;
     }
 
     // r2 of a code: what of Qinv(code) stays in the error feedback, in the element type

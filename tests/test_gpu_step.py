@@ -261,6 +261,39 @@ def test_densified_second_quantisation(oracle, q, DB, dtype):
         assert np.array_equal(to_np(gp.data), oparams[0]), f"step {step + 1}: parameters"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q", [32, 64, 128, 512, 1024])
+def test_densified_second_quantisation_of_a_short_block(oracle, q, dtype):
+    """A tensor's last quantisation block with 1 to q - 1 of its q elements, at 30 times its range
+    from zero, where the second quantisation moves some of the 16 codes: which of them the block's
+    few elements have must not matter.  The blocks in front of it lie around zero, where every code
+    maps to itself, and hold the largest elements, so that the top-k leaves the short one alone."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(q)
+    tails = sorted({1, 7, 8, 16, 24, q // 2, q - 8, q - 1}) * 6
+    sizes = [(4096 if i % 2 else 0) + 2 * q + t for i, t in enumerate(tails)]
+    params = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in params]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=4096)
+    gparams = [torch.nn.Parameter(p.clone().cuda()) for p in params]
+    opt = MicroAdam(gparams, m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
+    opt.d_block_size = 4096
+    for step in range(3):
+        grads = []
+        for n, t in zip(sizes, tails):
+            g = torch.randn(n, generator=gen) * 0.3
+            g[n - t:] = 0.1 + torch.randn(t, generator=gen) * 0.003
+            grads.append(g.to(dtype))
+        for p, g in zip(gparams, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        oref.step([to_np(g) for g in grads])
+        for i, p in enumerate(gparams):
+            assert opt._fusable(p, opt.state[p]) == 3
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tail {tails[i]}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, tails[i])
+
+
 @pytest.mark.parametrize("use_fused", [True, False], ids=["fused", "opbyop"])
 @pytest.mark.parametrize("scale", [1e-36, 3e-38, 1e-39])
 def test_denormal_scale_gradients(oracle, scale, use_fused):
