@@ -176,10 +176,11 @@ __global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, 
         constexpr int ROWS = 2;
         // Lane l takes the entries 4l .. 4l + 3 of a row's stretch, all one less if the stretch
         // begins on an odd entry: every load is 4-byte aligned then, where unaligned ones kept the
-        // kernel at 260 us.  The outermost loads reach up to three entries into the neighbouring
-        // stretches, whose terms are dropped; where the array may end behind the block the lanes
+        // kernel at 260 us.  The outermost loads reach up to four entries into the neighbouring
+        // stretches (a lane may start at entry kb: it is needed when the stretch begins one entry
+        // earlier), whose terms are dropped; where the array may end behind the block the lanes
         // load from the stretch's own boundaries, aligned or not.
-        const bool exact = S.col0 + S.kb + 3 > k;
+        const bool exact = S.col0 + S.kb + 4 > k;
         uint32_t from[GG];     // entry the lane's loads start at, from the row's first one
         bool own[2][GG][4];    // by the row's parity: which of the four are this lane's
 #pragma unroll

@@ -237,3 +237,35 @@ def test_row_lengths_at_the_edges(mods, oracle, dtype, kb):
     got = dots.cpu().numpy()
     assert np.all(np.abs(got[:rows] - want[:rows]) <= SP_TOL * mass[:rows] + 1e-30)
     assert np.all(got[rows:] == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kb", [4, 16, 204, 308, 508])
+@pytest.mark.parametrize("full,m", [(1, 1), (1, 3), (2, 1), (2, 6)])
+def test_scalar_products_take_nothing_from_behind_the_window(mods, dtype, kb, full, m):
+    """Block rows of a multiple of four entries in front of a last block of three: the outermost
+    lane of the last row may not reach past the window's end.  What lies there, an index outside
+    every block once and a valid one once, must not change a bit of the sums."""
+    _, smf = mods
+    dbs, tail = 1024, 3
+    d, k = dbs * full + 200, full * kb + tail
+    gen = torch.Generator().manual_seed(kb)
+    cols = [torch.rand(m, ln, generator=gen).argsort(dim=1)[:, :kk]
+            for ln, kk in zip([dbs] * full + [200], [kb] * full + [tail])]
+    I = torch.cat(cols, dim=1).to(torch.int16)
+    V = torch.randn(I.shape, generator=gen).to(dtype)
+    g = torch.randn(d, generator=gen).to(dtype).cuda()
+    outs = []
+    for behind in (30000, 0):
+        Ib = torch.full((m * k + 64,), behind, dtype=torch.int16, device="cuda")
+        Vb = torch.full((m * k + 64,), 7.0, dtype=dtype, device="cuda")
+        Ib[:m * k], Vb[:m * k] = I.view(-1).cuda(), V.view(-1).cuda()
+        out = torch.zeros(m, dtype=torch.float32, device="cuda")
+        smf.SP(0, 0, 23, d, m, k, dbs, kb, g, Ib[:m * k].view(m, k), Vb[:m * k].view(m, k), out,
+               int(dtype == torch.bfloat16))
+        outs.append(to_np(out))
+    assert np.array_equal(outs[0], outs[1])
+    pos = (torch.arange(k) // kb) * dbs + I.long()
+    terms = V.double() * g.cpu().double()[pos]
+    assert np.all(np.abs(outs[0] - terms.sum(dim=1).numpy())
+                  <= SP_TOL * terms.abs().sum(dim=1).numpy())
