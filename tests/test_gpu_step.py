@@ -271,13 +271,12 @@ def test_densified_second_quantisation_of_a_short_block(oracle, q, dtype):
     from ista_daslab_optimizers import MicroAdam
     gen = torch.Generator().manual_seed(q)
     tails = sorted({1, 7, 8, 16, 24, q // 2, q - 8, q - 1}) * 6
-    sizes = [(4096 if i % 2 else 0) + 2 * q + t for i, t in enumerate(tails)]
+    sizes = [(20480 if i % 2 else 0) + 2 * q + t for i, t in enumerate(tails)]
     params = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
     oparams = [to_np(p) for p in params]
-    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=4096)
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=20480)
     gparams = [torch.nn.Parameter(p.clone().cuda()) for p in params]
     opt = MicroAdam(gparams, m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
-    opt.d_block_size = 4096
     for step in range(3):
         grads = []
         for n, t in zip(sizes, tails):
