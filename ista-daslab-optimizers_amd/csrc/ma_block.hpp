@@ -84,7 +84,8 @@ struct FusedParams {
     float keep;       // (float)(1 - alpha): share that stays in the error feedback
     // logging steps (kernels compiled with kAuxLog): kMetricSlots floats per work item
     float *metrics;
-    // the block kernel ends with the quantisation; window_param_kernel does the rest
+    // the window is window_param_kernel's: the block kernel ends with the quantisation (but not
+    // a logging step's) and lists its rows by coordinate where it can
     int32_t win_apart;
     // one-pass form of the two-pass route: polls a workgroup spends at most on waiting for the
     // extremes of the blocks that share its quantisation blocks (0: it does not wait at all)
@@ -545,7 +546,8 @@ struct FusedBlock {
             }
         } else if (kb <= kWG && P.win_apart == 0 &&
                    P.L.total - P.L.off_union >= kHintRegBytes) {
-            // (the window kernel of the two-launch form wants its rows by coordinate)
+            // (the window kernel of the two-launch form wants its rows by coordinate, those that
+            // logging steps write among them)
             topk_done = hint_topk_registers(r, kb, hint, hist, sh, sel_idx, sel_val);
             launder(r);
         }

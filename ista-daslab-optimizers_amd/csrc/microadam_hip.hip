@@ -938,7 +938,9 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             P.alpha = (float)alpha;
             P.keep = (float)(1.0 - alpha);
             P.metrics = (aux & kAuxLog) ? metrics + items_before * kMetricSlots : nullptr;
-            P.win_apart = 0;
+            // (a logging step of windows that the ordinary step takes in two launches runs in one,
+            // but leaves its rows as the second launch of the next steps wants them)
+            P.win_apart = !span && !dense && aux == kAuxLog && P.L.cell_bytes == 0 ? 1 : 0;
             P.spin_limit = span_spin_limit();
             plan.back().kind = kWholeStep;
             int rc = P.L.total > kLdsLimit ? MA_ERR_LDS : 0;

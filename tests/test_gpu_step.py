@@ -849,3 +849,30 @@ def test_spanning_route_takes_short_vectors(oracle, q, dtype, alpha):
     sizes = [768, 125, 80, 9, 20480] + ([20480 * 2 + 77] if q < 1 << 20 else [])
     _run(oracle, sizes, dtype, 3, q, 0.01, alpha, 0.01, 20480, 5, True, zero_step=2,
          expect_route=True)
+
+
+@pytest.mark.parametrize("sizes,dtype,m,k_init", [
+    ([20480 * 2 + 8192], torch.bfloat16, 20, 0.03),        # partial block: 246 entries
+    ([20480 + 4096, 20480], torch.float32, 20, 0.025),     # 512 entries a block
+])
+def test_logging_steps_write_dense_windows_rows_by_coordinate(sizes, dtype, m, k_init):
+    """Windows that the ordinary step takes in two launches: the second one counts on block rows
+    in coordinate order, those of the logging steps among them."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(41)
+    params = [torch.nn.Parameter((torch.randn(n, generator=gen) * 0.02).to(dtype).cuda())
+              for n in sizes]
+    opt = MicroAdam(params, m=m, lr=1e-3, quant_block_size=32, k_init=k_init)
+    opt.log_interval = 2
+    opt._logging_active = lambda: True
+    opt._log = lambda *a: None
+    for step in range(16):
+        for p in params:
+            p.grad = (torch.randn(p.numel(), generator=gen) * 0.01).to(dtype).cuda()
+        opt.step()
+        for p in params:
+            st = opt.state[p]
+            row, many = st["I"][step % m].long().cpu(), st["k_block_size_many"]
+            # (full bf16 blocks of at most 512 entries are not listed by coordinate by any step)
+            for part in row.split(many):
+                assert torch.all(part[1:] > part[:-1]), (step, len(part))
