@@ -420,7 +420,8 @@ class MicroAdam(torch.optim.Optimizer):
         if sums is not None:
             for key, value in zip(('norm_qe', 'norm_g', 'norm_u', 'norm_e', 'sparsity_u',
                                    'sparsity_qe'), sums.tolist()):
-                totals[key] += value
+                # (a tensor of the gradient's type, or of whole numbers, where tensors went op by op)
+                totals[key] = float(totals[key]) + value
 
         if logging_step:
             self._log(totals['norm_qe'], totals['norm_g'], totals['norm_u'], totals['norm_e'],

@@ -876,3 +876,33 @@ def test_logging_steps_write_dense_windows_rows_by_coordinate(sizes, dtype, m, k
             # (full bf16 blocks of at most 512 entries are not listed by coordinate by any step)
             for part in row.split(many):
                 assert torch.all(part[1:] > part[:-1]), (step, len(part))
+
+
+def test_logging_step_of_a_list_on_several_routes(oracle):
+    """A tensor whose gradient is not 16-byte aligned goes op by op beside the others: its sums and
+    the kernels' are added."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(47)
+    sizes = [20480 + 4096, 768]
+    cpu = [(torch.randn(n, generator=gen) * 0.02).to(torch.bfloat16) for n in sizes]
+    oparams = [to_np(p) for p in cpu]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, 64, 0.01, 0.0, d_block_size=20480)
+    params = [torch.nn.Parameter(p.clone().cuda()) for p in cpu]
+    opt = MicroAdam(params, m=3, lr=1e-3, quant_block_size=64)
+    opt.log_interval = 1
+    opt._logging_active = lambda: True
+    logged = []
+    opt._log = lambda *a: logged.append([float(x) for x in a[:6]])
+    for step in range(2):
+        grads = [(torch.randn(n, generator=gen) * 0.01).to(torch.bfloat16) for n in sizes]
+        buf = torch.zeros(sizes[1] + 1, dtype=torch.bfloat16, device="cuda")
+        buf[1:] = grads[1].cuda()
+        params[0].grad, params[1].grad = grads[0].cuda(), buf[1:]
+        opt.step()
+        want = oref.step([to_np(g) for g in grads], metrics=True)
+        for key, value in zip(("norm_qe", "norm_g", "norm_u", "norm_e"), logged[step]):
+            # (the op-by-op sums are bf16's: 2^-9 a rounding, a few of them)
+            assert value == pytest.approx(want[key], rel=3e-2, abs=0), key
+        assert logged[step][4:] == [want["sparsity_u"], want["sparsity_qe"]]
+        for i, p in enumerate(params):
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
