@@ -309,6 +309,14 @@ class MicroAdam(torch.optim.Optimizer):
             return SPANNING
         return OP_BY_OP
 
+    def _logged_segmented(self, p, st):
+        """Route of a logging step of a tensor on the segmented route, whose kernels do not form
+        the logged sums: the spanning route's do, for the tensors it takes."""
+        probe, h = self._probe(p, st)
+        taken = _hip.lib.ma_spanning_step_check(ctypes.byref(probe), ctypes.byref(h),
+                                                float(self.alpha)) == 0
+        return SPANNING if taken else OP_BY_OP
+
     def _q_is_segmented(self):
         """Quantisation blocks ma_fused_step does not take whatever the tensor's size: a list's
         tensors shorter than one of them then ride along with the others instead of taking the
@@ -399,7 +407,7 @@ class MicroAdam(torch.optim.Optimizer):
                     if not (e.p_addr | e.g_addr) & 15:
                         route = e.route
                         if logging_step and route == SEGMENTED:
-                            route = OP_BY_OP  # its kernels do not form the logged sums
+                            route = self._logged_segmented(p, e.st)
                 if route == OP_BY_OP:
                     for key, value in self.update_step(p, lr, wd, logging_step).items():
                         totals[key] += value

@@ -906,3 +906,42 @@ def test_logging_step_of_a_list_on_several_routes(oracle):
         assert logged[step][4:] == [want["sparsity_u"], want["sparsity_qe"]]
         for i, p in enumerate(params):
             assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_logging_steps_of_the_segmented_route(oracle, dtype):
+    """Its kernels do not form the logged sums: on a logging step the tensors that the spanning
+    route takes go there, only the others op by op, and the state stays the oracle's."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(43)
+    sizes = [20480 + 4096, 768, 10000, 33, 12288]
+    cpu = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in cpu]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, 10000, 0.01, 0.0, d_block_size=20480)
+    params = [torch.nn.Parameter(p.clone().cuda()) for p in cpu]
+    opt = MicroAdam(params, m=3, lr=1e-3, quant_block_size=10000)
+    opt.log_interval = 2
+    opt._logging_active = lambda: True
+    logged, wanted = [], []
+    opt._log = lambda *a: logged.append([float(x) for x in a[:6]])
+    one_by_one, inner = [], opt.update_step
+    opt.update_step = lambda p, *a: (one_by_one.append((opt.steps, p.numel())), inner(p, *a))[1]
+    for step in range(5):
+        grads = [(torch.randn(n, generator=gen) * 0.01).to(dtype) for n in sizes]
+        for p, g in zip(params, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        out = oref.step([to_np(g) for g in grads], metrics=step % 2 == 1)
+        if out is not None:
+            wanted.append(out)
+        for i, p in enumerate(params):
+            assert opt._fusable(p, opt.state[p]) == 5
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+    assert one_by_one == [(s, n) for s in (2, 4) for n in (24576, 12288)]
+    assert len(logged) == 2 == len(wanted)
+    rel = 3e-2 if dtype == torch.bfloat16 else 1e-4  # as in test_logged_sums_match_oracle, op by op
+    for got, want in zip(logged, wanted):
+        for key, value in zip(("norm_qe", "norm_g", "norm_u", "norm_e"), got):
+            assert value == pytest.approx(want[key], rel=rel, abs=0), key
+        assert got[4:] == [want["sparsity_u"], want["sparsity_qe"]]
