@@ -318,11 +318,11 @@ class MicroAdam(torch.optim.Optimizer):
         return SPANNING if taken else OP_BY_OP
 
     def _q_is_segmented(self):
-        """Quantisation blocks ma_fused_step does not take whatever the tensor's size: a list's
-        tensors shorter than one of them then ride along with the others instead of taking the
-        spanning route's launches for themselves."""
+        """Quantisation blocks ma_fused_step does not take in a tensor of several top-k blocks: a
+        list's tensors shorter than one of them then ride along with the others instead of
+        taking the spanning route's launches for themselves."""
         q = self.quant_block_size
-        return q > 4096 or q & (q - 1) != 0
+        return q > 4096 or q & (q - 1) != 0 or self.d_block_size % q != 0
 
     def _probe(self, p, st):
         """A record of p's state (with stand-ins for the buffers of a step) and the

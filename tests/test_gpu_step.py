@@ -173,6 +173,9 @@ SEGMENTED_CASES = [
     ([12288 * 2 + 8], torch.bfloat16, 3, 5000, 0.01, 0.0, 0.0, 12288, 5),
     ([32768 * 2 + 520], torch.bfloat16, 3, 520, 0.01, 0.0, 0.0, 32768, 5),
     ([20480 + 8192], torch.bfloat16, 20, 10000, 0.05, 0.0, 0.0, 20480, 22),
+    # powers of two up to 4096 that do not divide the top-k block
+    ([10240 * 2 + 4104, 10240 * 3], torch.bfloat16, 3, 4096, 0.01, 0.0, 0.0, 10240, 5),
+    ([1032 * 4 + 3], torch.float32, 3, 512, 0.02, 0.0, 0.0, 1032, 5),
 ]
 
 
