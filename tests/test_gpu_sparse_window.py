@@ -269,3 +269,31 @@ def test_scalar_products_take_nothing_from_behind_the_window(mods, dtype, kb, fu
     terms = V.double() * g.cpu().double()[pos]
     assert np.all(np.abs(outs[0] - terms.sum(dim=1).numpy())
                   <= SP_TOL * terms.abs().sum(dim=1).numpy())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dbs,kb,tail", [(13653, 3, 1), (13653, 137, 2), (13654, 137, 3),
+                                         (13654, 2, 2), (4096, 300, 1), (20480, 512, 3)])
+def test_linear_combination_of_short_rows_and_small_blocks(mods, oracle, dtype, dbs, kb, tail):
+    """Blocks of one to three entries a row behind longer ones and alone, on both sides of the block
+    length below which one wave makes a workgroup, with indices outside the block among them."""
+    _, smf = mods
+    rows, m = 67, 70
+    d, k = dbs * 2 + max(tail, 70), 2 * kb + tail
+    gen = torch.Generator().manual_seed(dbs + kb)
+    cols = [torch.rand(m, ln, generator=gen).argsort(dim=1)[:, :kk]
+            for ln, kk in zip([dbs, dbs, d - 2 * dbs], (kb, kb, tail))]
+    I = torch.cat(cols, dim=1).to(torch.int16)
+    V = torch.randn(I.shape, generator=gen).to(dtype)
+    clean = I.clone()
+    for r, c in ((0, 0), (5, kb - 1), (33, k - 1), (66, k - 1)):
+        I[r, c] = -3 if r % 2 else 30000  # outside every block
+    coef = torch.randn(m, generator=gen)
+    Vz = V.clone()
+    Vz[I != clean] = 0  # (as in test_row_lengths_at_the_edges)
+    want = to_np(torch.zeros(d, dtype=dtype))
+    oracle.sparse_linear_combination(d, rows, k, dbs, kb, coef.numpy(), to_np(clean), to_np(Vz), want)
+    out = torch.zeros(d, dtype=dtype, device="cuda")
+    smf.LCG(0, 0, 51, d, rows, k, dbs, kb, coef.cuda(), I.cuda(), V.cuda(), out,
+            int(dtype == torch.bfloat16))
+    assert np.array_equal(to_np(out), want)
