@@ -348,7 +348,7 @@ __device__ __forceinline__ uint32_t cell_address(uint32_t w, uint32_t two) {
     return a;
 }
 
-template <typename TV, int G, int RING>
+template <typename TV, int G, int RING, bool LONG>
 __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int64_t k, int m_rows,
                                              const float *coef, const int16_t *I, const TV *V,
                                              int lane) {
@@ -364,12 +364,14 @@ __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int
     // Requests are made in row order and at every round alike (the last row again and again
     // behind the window's end), so that at any time the same number of them is under way and
     // the compiler can wait for the oldest ones alone.  Rows of a round are addressed from its
-    // first one in 32 bits (the host checks that RING rows fit).
-    const uint32_t row_bytes = (uint32_t)k * 2u;
+    // first one in 32 bits, LONG ones (RING of them do not fit) row by row.
+    const uint32_t row_bytes = LONG ? 0 : (uint32_t)k * 2u;
     const int16_t *Ir = I + S.col0;
     const TV *Vr = V + S.col0;
     uint32_t row_at = 0, last_at = 0;
+    int next_row = 0;
     auto aim = [&](int first) {  // the next RING requests are for the rows from `first` on
+        if (LONG) return;
         const int row = first < m_rows ? first : m_rows - 1;
         const int more = m_rows - 1 - row;
         Ir = I + ((int64_t)row * k + S.col0);
@@ -387,7 +389,13 @@ __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int
             v[slot][g] = *reinterpret_cast<const ValueQuad<TV> *>(
                 reinterpret_cast<const char *>(Vr) + (at * kWide));
         }
-        row_at = min(row_at + row_bytes, last_at);
+        if (LONG) {
+            const int64_t on = ++next_row < m_rows ? k : 0;
+            Ir += on;
+            Vr += on;
+        } else {
+            row_at = min(row_at + row_bytes, last_at);
+        }
     };
     uint32_t cell[2][G][4];  // LDS addresses
     float term[2][G][4];
@@ -534,7 +542,7 @@ __device__ __forceinline__ void combine_short_rows(float *acc, const BlockSpan &
 }
 
 // G == 0: rows of any length, all threads, a barrier behind every row
-template <typename TO, typename TV, int G, int WG>
+template <typename TO, typename TV, int G, int WG, bool LONG>
 __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, int kbs,
                                                              int64_t k, int m_rows,
                                                              const float *__restrict__ coef,
@@ -553,8 +561,8 @@ __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, 
     // (expected: with the short rows' code in front of it this path runs 2 % slower)
     if (G > 0 && __builtin_expect(S.kb >= 4, 1)) {
         if (tid < 64)
-            combine_rows<TV, (G > 0 ? G : 1), kRingRows / (G > 0 ? G : 1)>(acc, S, k, m_rows, coef,
-                                                                          I, V, tid);
+            combine_rows<TV, (G > 0 ? G : 1), kRingRows / (G > 0 ? G : 1), LONG>(
+                acc, S, k, m_rows, coef, I, V, tid);
         __syncthreads();
     } else if (G > 0) {
         if (tid < 64) combine_short_rows<TV, kShortRing>(acc, S, k, m_rows, coef, I, V, tid);
@@ -701,19 +709,25 @@ int ma_sparse_linear_combination(int64_t d, int64_t m_rows, int64_t k, int64_t d
     const int lds = (int)(d_block_size * 4);
     if (lds > kLdsBytes) return MA_ERR_LDS;
     hipStream_t s = (hipStream_t)stream;
-    // Rows of up to 512 entries per block: one wave applies them.  1248 blocks of 20480, 1024 rows
-    // of 205 bf16: 360 us against 590 with four waves and a barrier per row.  Longer rows give a
-    // barrier more to do, and a row of more than 2^25 entries does not fit the wave's offsets.
-    const int groups = k <= (1 << 25) ? quad_groups(k_block_size) : 0;
-#define CALL_G(TO, TV, G, WG)                                                                   \
-    if ((rc = allow_lds(sparse_combine_kernel<TO, TV, G, WG>, lds))) return rc;                 \
-    rc = launch_kernel(sparse_combine_kernel<TO, TV, G, WG>, dim3((unsigned)nblocks), WG, lds,  \
-                       s, d, (int)d_block_size, (int)k_block_size, k, (int)m_rows, coef,        \
-                       indices, (const TV *)values, (TO *)out);
+    // Rows of up to 512 entries per block: one wave applies them, against four waves (eight above
+    // 256 entries) and a barrier per row: 1248 blocks of 20480, 1024 rows of 205 bf16: 362 us, 598;
+    // 512 rows of 410: 318, 381; of 512: 317, 395.  Longer rows give a barrier more to do.
+    // Rows of more than 2^25 entries do not fit a round's 32-bit offsets; addressed row by row
+    // the 1024 rows of 205 take 387 us.
+    const int groups = quad_groups(k_block_size) <= 2 ? quad_groups(k_block_size) : 0;
+    const bool is_long = k > (1 << 25);
+    const int threads = groups == 0 ? kWG : kCombineThreads;
+#define CALL_G(TO, TV, ...)                                                                     \
+    if ((rc = allow_lds(sparse_combine_kernel<TO, TV, __VA_ARGS__>, lds))) return rc;           \
+    rc = launch_kernel(sparse_combine_kernel<TO, TV, __VA_ARGS__>, dim3((unsigned)nblocks),     \
+                       threads, lds, s, d, (int)d_block_size, (int)k_block_size, k,             \
+                       (int)m_rows, coef, indices, (const TV *)values, (TO *)out);
 #define CALL(TO, TV)                                                                            \
-    if (groups == 1) { CALL_G(TO, TV, 1, kCombineThreads) }                                     \
-    else if (groups == 2) { CALL_G(TO, TV, 2, kCombineThreads) }                                \
-    else { CALL_G(TO, TV, 0, kWG) }
+    if (groups == 0) { CALL_G(TO, TV, 0, kWG, false) }                                          \
+    else if (is_long && groups == 1) { CALL_G(TO, TV, 1, kCombineThreads, true) }               \
+    else if (is_long) { CALL_G(TO, TV, 2, kCombineThreads, true) }                              \
+    else if (groups == 1) { CALL_G(TO, TV, 1, kCombineThreads, false) }                         \
+    else { CALL_G(TO, TV, 2, kCombineThreads, false) }
     MA_DISPATCH2(out_dtype, values_dtype, CALL)
 #undef CALL
 #undef CALL_G
