@@ -20,6 +20,7 @@ constexpr int kLdsBytes = 160 * 1024;
 constexpr int kRingRows = 32;          // rows the linear combination requests ahead
 constexpr int kShortRing = 16;        // the same for rows of one to three entries
 constexpr int kCombineThreads = 256;  // of a workgroup in which one wave applies the rows
+constexpr int kSmallBlock = 13653;    // coordinates: more than two such blocks fit a CU's LDS
 constexpr int kDotUnroll = 4;          // entries a lane requests ahead in the scalar products
 
 __device__ __forceinline__ float widen(float x) { return x; }
@@ -550,6 +551,7 @@ __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, 
                                                              const TV *__restrict__ V,
                                                              TO *__restrict__ out) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int kRing = WG == 64 ? kRingRows / 2 : kRingRows;
     float *acc = (float *)lds_raw;
     const BlockSpan S = block_span(d, dbs, kbs, k, xcd_item((int)gridDim.x));
     const int tid = threadIdx.x;
@@ -561,8 +563,8 @@ __global__ __launch_bounds__(WG) void sparse_combine_kernel(int64_t d, int dbs, 
     // (expected: with the short rows' code in front of it this path runs 2 % slower)
     if (G > 0 && __builtin_expect(S.kb >= 4, 1)) {
         if (tid < 64)
-            combine_rows<TV, (G > 0 ? G : 1), kRingRows / (G > 0 ? G : 1), LONG>(
-                acc, S, k, m_rows, coef, I, V, tid);
+            combine_rows<TV, (G > 0 ? G : 1), kRing / (G > 0 ? G : 1), LONG>(acc, S, k, m_rows,
+                                                                            coef, I, V, tid);
         __syncthreads();
     } else if (G > 0) {
         if (tid < 64) combine_short_rows<TV, kShortRing>(acc, S, k, m_rows, coef, I, V, tid);
@@ -713,10 +715,12 @@ int ma_sparse_linear_combination(int64_t d, int64_t m_rows, int64_t k, int64_t d
     // 256 entries) and a barrier per row: 1248 blocks of 20480, 1024 rows of 205 bf16: 362 us, 598;
     // 512 rows of 410: 318, 381; of 512: 317, 395.  Longer rows give a barrier more to do.
     // Rows of more than 2^25 entries do not fit a round's 32-bit offsets; addressed row by row
-    // the 1024 rows of 205 take 387 us.
+    // the 1024 rows of 205 take 387 us.  Small blocks, of which the LDS would hold more than two,
+    // are short of waves: one to a workgroup, with half the rows under way (blocks of 512, 256
+    // rows of 5: 591 us; with three idle waves beside it, 833; four waves and barriers, 769).
     const int groups = quad_groups(k_block_size) <= 2 ? quad_groups(k_block_size) : 0;
-    const bool is_long = k > (1 << 25);
-    const int threads = groups == 0 ? kWG : kCombineThreads;
+    const bool is_long = k > (1 << 25), small = d_block_size <= kSmallBlock;
+    const int threads = groups == 0 ? kWG : small && !is_long ? 64 : kCombineThreads;
 #define CALL_G(TO, TV, ...)                                                                     \
     if ((rc = allow_lds(sparse_combine_kernel<TO, TV, __VA_ARGS__>, lds))) return rc;           \
     rc = launch_kernel(sparse_combine_kernel<TO, TV, __VA_ARGS__>, dim3((unsigned)nblocks),     \
@@ -726,6 +730,8 @@ int ma_sparse_linear_combination(int64_t d, int64_t m_rows, int64_t k, int64_t d
     if (groups == 0) { CALL_G(TO, TV, 0, kWG, false) }                                          \
     else if (is_long && groups == 1) { CALL_G(TO, TV, 1, kCombineThreads, true) }               \
     else if (is_long) { CALL_G(TO, TV, 2, kCombineThreads, true) }                              \
+    else if (small && groups == 1) { CALL_G(TO, TV, 1, 64, false) }                             \
+    else if (small) { CALL_G(TO, TV, 2, 64, false) }                                            \
     else if (groups == 1) { CALL_G(TO, TV, 1, kCombineThreads, false) }                         \
     else { CALL_G(TO, TV, 2, kCombineThreads, false) }
     MA_DISPATCH2(out_dtype, values_dtype, CALL)

@@ -272,6 +272,32 @@ def test_scalar_products_take_nothing_from_behind_the_window(mods, dtype, kb, fu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("block", [32, 512])
+def test_linear_combination_of_rows_too_long_for_32_bit_offsets(mods, dtype, block):
+    """Rows of more than 2^25 entries, with a last block of three, against the same sums in the
+    same order by torch, bit for bit."""
+    _, smf = mods
+    m, full = 3, (1 << 25) // block + 5
+    d = k = full * block + 3
+    j = torch.arange(k, device="cuda")
+    lens = torch.where(j < full * block, block, 3)
+    gen = torch.Generator(device="cuda").manual_seed(block)
+    coef = torch.randn(m, generator=gen, device="cuda")
+    I = torch.empty(m, k, dtype=torch.int16, device="cuda")
+    V = torch.empty(m, k, dtype=dtype, device="cuda")
+    acc = torch.zeros(d, device="cuda")
+    for r in range(m):
+        idx = (j % block * 5 + 7 * r) % lens
+        I[r] = idx
+        V[r] = torch.randn(k, generator=gen, device="cuda")
+        pos = j // block * block + idx
+        acc[pos] = acc[pos] + coef[r] * V[r].float()
+    out = torch.zeros(d, dtype=dtype, device="cuda")
+    smf.LCG(0, 0, 51, d, m, k, block, block, coef, I, V, out, int(dtype == torch.bfloat16))
+    assert torch.equal(out, acc.to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("dbs,kb,tail", [(13653, 3, 1), (13653, 137, 2), (13654, 137, 3),
                                          (13654, 2, 2), (4096, 300, 1), (20480, 512, 3)])
 def test_linear_combination_of_short_rows_and_small_blocks(mods, oracle, dtype, dbs, kb, tail):
@@ -297,29 +323,3 @@ def test_linear_combination_of_short_rows_and_small_blocks(mods, oracle, dtype, 
     smf.LCG(0, 0, 51, d, rows, k, dbs, kb, coef.cuda(), I.cuda(), V.cuda(), out,
             int(dtype == torch.bfloat16))
     assert np.array_equal(to_np(out), want)
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("block", [32, 512])
-def test_linear_combination_of_rows_too_long_for_32_bit_offsets(mods, dtype, block):
-    """Rows of more than 2^25 entries, with a last block of three, against the same sums in the
-    same order by torch, bit for bit."""
-    _, smf = mods
-    m, full = 3, (1 << 25) // block + 5
-    d = k = full * block + 3
-    j = torch.arange(k, device="cuda")
-    lens = torch.where(j < full * block, block, 3)
-    gen = torch.Generator(device="cuda").manual_seed(block)
-    coef = torch.randn(m, generator=gen, device="cuda")
-    I = torch.empty(m, k, dtype=torch.int16, device="cuda")
-    V = torch.empty(m, k, dtype=dtype, device="cuda")
-    acc = torch.zeros(d, device="cuda")
-    for r in range(m):
-        idx = (j % block * 5 + 7 * r) % lens
-        I[r] = idx
-        V[r] = torch.randn(k, generator=gen, device="cuda")
-        pos = j // block * block + idx
-        acc[pos] = acc[pos] + coef[r] * V[r].float()
-    out = torch.zeros(d, dtype=dtype, device="cuda")
-    smf.LCG(0, 0, 51, d, m, k, block, block, coef, I, V, out, int(dtype == torch.bfloat16))
-    assert torch.equal(out, acc.to(dtype))
