@@ -275,28 +275,41 @@ __global__ __launch_bounds__(kWG, 8) void sparse_dot_kernel(int64_t d, int dbs, 
         }
     } else {
         stage();
-        for (int r = row_lo + wave; r < row_hi; r += kWaves) {
-            const int64_t first = (int64_t)r * k + S.col0;
-            float acc = 0.0f;
+        // Two rows at a time, their requests without conditions (entries clamped into the row): under
+        // a condition the compiler widens a value right behind its load and waits for it there.
+        // 1220 blocks of 20480, 512 rows of 512 bf16: 420 us with conditions, 240 without.
+        for (int r = row_lo + wave; r < row_hi; r += 2 * kWaves) {
+            const bool two = r + kWaves < row_hi;
+            const int64_t first[2] = {(int64_t)r * k + S.col0,
+                                      (int64_t)(two ? r + kWaves : r) * k + S.col0};
+            float acc[2] = {0.0f, 0.0f};
             for (int j0 = 0; j0 < S.kb; j0 += 64 * kDotUnroll) {
-                int ix[kDotUnroll];
-                TV v[kDotUnroll];
+                int ix[2][kDotUnroll];
+                TV v[2][kDotUnroll];
 #pragma unroll
                 for (int u = 0; u < kDotUnroll; ++u) {
-                    const int j = j0 + u * 64 + lane;
-                    ix[u] = -1;
-                    v[u] = (TV)0;
-                    if (j < S.kb) {
-                        ix[u] = I[first + j];
-                        v[u] = V[first + j];
+                    const int j = min(j0 + u * 64 + lane, S.kb - 1);
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) {
+                        ix[w][u] = I[first[w] + j];
+                        v[w][u] = V[first[w] + j];
                     }
                 }
 #pragma unroll
                 for (int u = 0; u < kDotUnroll; ++u)
-                    if ((unsigned)ix[u] < (unsigned)S.len) acc += widen(v[u]) * widen(gl[ix[u]]);
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) {
+                        const bool counts = j0 + u * 64 + lane < S.kb &&
+                                            (unsigned)ix[w][u] < (unsigned)S.len;
+                        const float t = widen(v[w][u]) * widen(gl[counts ? ix[w][u] : 0]);
+                        acc[w] += counts ? t : 0.0f;
+                    }
             }
-            acc = wave_sum_to_last(acc);
-            if (lane == 63) dst[r] = acc;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                acc[w] = wave_sum_to_last(acc[w]);
+                if (lane == 63 && (w == 0 || two)) dst[r + w * kWaves] = acc[w];
+            }
         }
     }
 }
