@@ -2601,7 +2601,7 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
     constexpr bool kSweep = PASS == 8 || PASS == 9, kSegmented = PASS == 7 || PASS == 9;
     uint32_t *slots = reinterpret_cast<uint32_t *>(P.t[0].ws);
     uint32_t *defer_count = slots + kSpanDeferCount;
-    // (PASS 6) this block gives up: listed for the sweep
+    // (PASS 6 and 7) this block gives up: listed for the sweep
     auto list_deferred = [&](int item) {
         if (threadIdx.x == 0) {
             const uint32_t at = atomicAdd(defer_count, 1u);
@@ -2686,7 +2686,10 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
                            : PASS == 2 ? kUpdate | 1u << kMtError
                                        : 1u << kMtError);
     };
-    auto one = [&](int item) {
+    // (inlined whatever its size: as a call, the compiler's choice for blocks above 20480 elements,
+    // it wants the parameters in memory, 19 KB of scratch a lane: 80 M bf16 parameters in blocks of
+    // 32768, q = 65536, 5.8 ms a step instead of 0.74)
+    auto one = [&](int item) __attribute__((always_inline)) {
         const int ti = find_tensor(P, item);
         const BlockGeo G = make_geo(P, ti, P.t[ti].blk0 + (item - P.t[ti].first_block));
         if (G.n == R::kC * kRound) {

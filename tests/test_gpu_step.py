@@ -948,3 +948,13 @@ def test_logging_steps_of_the_segmented_route(oracle, dtype):
         for key, value in zip(("norm_qe", "norm_g", "norm_u", "norm_e"), got):
             assert value == pytest.approx(want[key], rel=rel, abs=0), key
         assert got[4:] == [want["sparsity_u"], want["sparsity_qe"]]
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.5])
+@pytest.mark.parametrize("spin", [None, "0"], ids=["exchange", "deferred"])
+def test_spanning_route_above_the_hardware_block(oracle, monkeypatch, spin, alpha):
+    """Top-k blocks of more than 20480 elements, which run in kernels of their own."""
+    if spin is not None:
+        monkeypatch.setenv("MA_SPAN_SPIN_LIMIT", spin)
+    _run(oracle, [32768 * 3 + 520, 24576 + 77], torch.bfloat16, 3, 65536, 0.01, alpha, 0.01, 32768, 5,
+         True, zero_step=2, expect_route=True)
