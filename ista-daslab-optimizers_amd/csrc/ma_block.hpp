@@ -1380,6 +1380,11 @@ struct FusedBlock {
     // Q of r2 = (1 - alpha) * Qinv(e1) with statistics of its own.
     uint32_t dcodes[C], dstat[C];  // e1 of the chunk; its min | max << 16 (bf16 bits)
 
+    // Blocks of up to 12288 elements have the registers for the second quantisation element by
+    // element in line, which for q = 8 and 16 costs less than trying 16 and 8 codes a lane
+    // (requantised_alike): 80 M parameters in blocks of 4096, q = 8, 386 us a step against 411.
+    static constexpr bool kDirect = R::kC < kClass2;
+
     __device__ __forceinline__ void quantize_dense(const BlockGeo &G) {
         const int n = FULL ? C * kRound : G.n;
         uint8_t *err = G.D.err + (G.e0 >> 1);
@@ -1445,13 +1450,20 @@ struct FusedBlock {
             dcodes[c] = 0;
             const float mnf = bf2f(mnb);
             const float u = div15(bf2f(mxb) - mnf, d15);
-            if (FULL || off < n) {
-                float cf[8];
-                codes8(x, mnf, u, cf);
+            float cf[kDirect ? 8 : 1];
+            if constexpr (kDirect) {  // (lanes past the end)
 #pragma unroll
-                for (int e = 0; e < kChunk; ++e)
-                    if (!FULL && off + e >= n) cf[e] = 0.0f;
-                dcodes[c] = pack_codes(cf);
+                for (int e = 0; e < kChunk; ++e) cf[e] = 0.0f;
+            }
+            if (FULL || off < n) {
+                float code[8];
+                codes8(x, mnf, u, code);
+#pragma unroll
+                for (int e = 0; e < kChunk; ++e) {
+                    if (!FULL && off + e >= n) code[e] = 0.0f;
+                    if constexpr (kDirect) cf[e] = code[e];
+                }
+                dcodes[c] = pack_codes(code);
             }
             // (packed here and now: left to itself the compiler moves the packing to the update
             // and keeps the floats instead, which costs 42 spilled registers)
@@ -1460,10 +1472,16 @@ struct FusedBlock {
             // (a quantisation block that begins inside the block counts with all its lanes: those
             // past the end hold no elements, but try codes that the others' elements may have)
             const bool begun = FULL || (off & -(1 << q_shift)) < n;
-            if (requantised_alike(mn, mx, mnf, u, begun, mn2b, mx2b)) {
-                codes = dcodes[c];
-            } else {
-                requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
+            bool done = false;
+            if constexpr (kDirect) {
+                done = ql < 4;
+                if (done) requantise_direct(cf, FULL ? kChunk : n - off, mnf, u, mn2b, mx2b, codes);
+            }
+            if (!done) {
+                if (requantised_alike(mn, mx, mnf, u, begun, mn2b, mx2b))
+                    codes = dcodes[c];
+                else
+                    requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
             }
             asm volatile("" : "+v"(codes), "+v"(mn2b), "+v"(mx2b));
             if (FULL || off < n) {
@@ -1497,26 +1515,37 @@ struct FusedBlock {
     // maps to c: the rounding of r2 (2^-9 of it for bf16) would have to reach half a step, i.e.
     // the block's values to lie many times its range away from zero.  So a quantisation block's
     // lanes try the 16 codes between them instead of requantising their 8 elements each (q = 64:
-    // two divisions a lane instead of eight, and no second min / max).  True, for the whole
+    // two divisions a lane instead of eight, and no second min / max; left out for run-time groups
+    // of fewer than 16 lanes, blocks of 12288 at q = 64 take 273 us a step instead of 223; a group
+    // of one lane, q = 8, is faster without: 247 us a step against 260 in blocks of 20480).  True, for the whole
     // wave, if every block maps every code to itself; the statistics of r2 are then r2 at the
     // codes of the block's extremes, 0 and 15.  `counts`: this lane's quantisation block has
     // elements, be they other lanes' alone.
     __device__ __forceinline__ bool requantised_alike(float mn, float mx, float mnf, float u,
                                                       bool counts, uint32_t &mn2b,
                                                       uint32_t &mx2b) const {
-        if (QL == 0 && ql < 16) return false;
-        constexpr int kPer = QL > 0 ? 16 / (QL > 0 ? QL : 1) : 1;  // codes a lane tries
+        if (QL == 0 && ql < 2) return false;
         mn2b = f2bf(kept_value(0.0f, mnf, u));
         mx2b = f2bf(kept_value(15.0f, mnf, u));
         const float m2f = bf2f(mn2b);
         const float u2 = div15(bf2f(mx2b) - m2f, d15);
         bool alike = divisor_is_plain(u) && divisor_is_plain(u2);
         const Divisor dv2 = make_divisor(u2);
+        if constexpr (QL > 0) {
+            constexpr int kPer = 16 / (QL > 0 ? QL : 1);  // codes a lane tries
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const float code = (float)((lane & ((QL > 0 ? QL : 16) - 1)) + i * (QL > 0 ? QL : 16));
-            const float y = kept_value(code, mnf, u) - m2f;
-            alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
+            for (int i = 0; i < kPer; ++i) {
+                const float code = (float)((lane & (QL - 1)) + i * QL);
+                const float y = kept_value(code, mnf, u) - m2f;
+                alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
+            }
+        } else {
+#pragma unroll 1
+            for (int i = lane & (min(ql, 16) - 1); i < 16; i += ql) {
+                const float code = (float)i;
+                const float y = kept_value(code, mnf, u) - m2f;
+                alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
+            }
         }
         if constexpr (!R::kBF16) {
             // (bf16 extremes are their own statistics and get the codes 0 and 15)
@@ -1535,6 +1564,32 @@ struct FusedBlock {
         deq = deq + mnf;
         const float keep = P.keep * deq;
         return to_elem(0.0f + keep);
+    }
+
+    // The second quantisation of a chunk with the codes cf, `valid` (or more) elements of it, whose
+    // quantisation block is not longer than a wave's stretch.
+    __device__ __forceinline__ void requantise_direct(const float (&cf)[8], int valid, float mnf,
+                                                      float u, uint32_t &mn2b, uint32_t &mx2b,
+                                                      uint32_t &codes) const {
+        float r2[8], c2[8];
+        float mn2 = INFINITY, mx2 = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            r2[e] = kept_value(cf[e], mnf, u);
+            if (e < valid) {
+                mn2 = fmin_raw(mn2, r2[e]);
+                mx2 = fmax_raw(mx2, r2[e]);
+            }
+        }
+        group_minmax<QL>(mn2, mx2, ql);
+        mn2b = f2bf(mn2);
+        mx2b = f2bf(mx2);
+        const float m2f = bf2f(mn2b);
+        codes8(r2, m2f, div15(bf2f(mx2b) - m2f, d15), c2);
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e)
+            if (e >= valid) c2[e] = 0.0f;
+        codes = pack_codes(c2);
     }
 
     // The second quantisation element by element: r2 from the codes of the chunk, its statistics,
@@ -2544,10 +2599,19 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
             // compiler (42 spilled registers), the narrow window stage and all elements
             // quantised twice; 1.90 ms so.  (The parameters asked for before the window: the same
             // 1.89 ms and five spilled registers.)
+            // Blocks of up to 12288 elements have the registers for the order of the plain step, and
+            // gain by the narrow stage: 80 M parameters in blocks of 12288, q = 64, 243 us a step
+            // with the wide one, 223 so; in blocks of 4096 390 and 380.
             fb.quantize_dense(G);
-            fb.load_older_rows(G);
-            fb.window_cells(G);
-            fb.load_params(G);
+            if constexpr (R::kC < kClass2) {
+                fb.load_params(G);
+                fb.load_window(G);
+                fb.window_stage(G);
+            } else {
+                fb.load_older_rows(G);
+                fb.window_cells(G);
+                fb.load_params(G);
+            }
             fb.param_stage_dense(G);
         } else if constexpr ((AUX & kAuxQuantErr) != 0) {
             // the quantisation steps the parameters; the window is asked for behind it (with

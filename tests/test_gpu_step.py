@@ -958,3 +958,36 @@ def test_spanning_route_above_the_hardware_block(oracle, monkeypatch, spin, alph
         monkeypatch.setenv("MA_SPAN_SPIN_LIMIT", spin)
     _run(oracle, [32768 * 3 + 520, 24576 + 77], torch.bfloat16, 3, 65536, 0.01, alpha, 0.01, 32768, 5,
          True, zero_step=2, expect_route=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("DB", [4096, 12288, 32768])
+@pytest.mark.parametrize("q", [8, 16, 32, 64])
+def test_densified_second_quantisation_of_run_time_groups(oracle, q, DB, dtype):
+    """The kernels of other block lengths take the quantisation group at run time: one to eight
+    lanes, which try several codes each or requantise their elements; blocks around zero and at
+    30 times their range from it side by side, the last one short."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(q + DB)
+    sizes = [DB + 5 * q + 3, DB - 2 * q + 5, 3 * q + 1]
+    params = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in params]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=DB)
+    gparams = [torch.nn.Parameter(p.clone().cuda()) for p in params]
+    opt = MicroAdam(gparams, m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
+    opt.d_block_size = DB
+    for step in range(3):
+        grads = []
+        for n in sizes:
+            far = torch.arange(n) // q % 80 >= 40 if n > DB // 2 else torch.arange(n) >= 3 * q
+            g = torch.where(far, 0.1 + torch.randn(n, generator=gen) * 0.003,
+                            torch.randn(n, generator=gen) * 0.3)
+            grads.append(g.to(dtype))
+        for p, g in zip(gparams, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        oref.step([to_np(g) for g in grads])
+        for i, p in enumerate(gparams):
+            assert opt._fusable(p, opt.state[p]) == 3
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
