@@ -685,7 +685,7 @@ struct FusedBlock {
 #pragma unroll
                 for (int e = 0; e < kChunk; ++e)
                     if (!FULL && off + e >= n) cf[e] = 0.0f;
-                const uint32_t codes = pack_codes(cf);
+                const uint32_t codes = (LOG || QE) ? pack_codes_apart(cf) : pack_codes(cf);
                 if (FULL || off + kChunk <= n) {
                     *reinterpret_cast<uint32_t *>(err + ((unsigned)off >> 1)) = codes;
                 } else {
@@ -1463,7 +1463,7 @@ struct FusedBlock {
                     if (!FULL && off + e >= n) code[e] = 0.0f;
                     if constexpr (kDirect) cf[e] = code[e];
                 }
-                dcodes[c] = pack_codes(code);
+                dcodes[c] = pack_codes_apart(code);
             }
             // (packed here and now: left to itself the compiler moves the packing to the update
             // and keeps the floats instead, which costs 42 spilled registers)
@@ -1868,15 +1868,33 @@ struct FusedBlock {
     }
 
     // two 16-bit halves, nibble order (e0 e1)(e2 e3) | (e4 e5)(e6 e7), even element high
-    static __device__ __forceinline__ uint32_t pack_codes(const float (&cf)[8]) {
-        float lo = cf[2];
+    static __device__ __forceinline__ void join_codes(const float (&cf)[8], float &lo, float &hi) {
+        lo = cf[2];
         lo = __builtin_fmaf(lo, 16.0f, cf[3]);
         lo = __builtin_fmaf(lo, 16.0f, cf[0]);
         lo = __builtin_fmaf(lo, 16.0f, cf[1]);
-        float hi = cf[6];
+        hi = cf[6];
         hi = __builtin_fmaf(hi, 16.0f, cf[7]);
         hi = __builtin_fmaf(hi, 16.0f, cf[4]);
         hi = __builtin_fmaf(hi, 16.0f, cf[5]);
+    }
+
+    static __device__ __forceinline__ uint32_t pack_codes(const float (&cf)[8]) {
+        float lo, hi;
+        join_codes(cf, lo, hi);
+        return (uint32_t)lo | ((uint32_t)hi << 16);
+    }
+
+    // The same where undefined elements must not spread over the codes they are packed with: they
+    // get code 0, as asymm_block_quant gives it (codes8 has given it to them already for fp32).
+    static __device__ __forceinline__ uint32_t pack_codes_apart(float (&cf)[8]) {
+        float lo, hi;
+        join_codes(cf, lo, hi);
+        if (R::kBF16 && __builtin_amdgcn_ballot_w64(__builtin_isunordered(lo, hi)) != 0) {
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e) cf[e] = fmax_raw(cf[e], 0.0f);
+            join_codes(cf, lo, hi);
+        }
         return (uint32_t)lo | ((uint32_t)hi << 16);
     }
 

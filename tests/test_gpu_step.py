@@ -991,3 +991,30 @@ def test_densified_second_quantisation_of_run_time_groups(oracle, q, DB, dtype):
             assert opt._fusable(p, opt.state[p]) == 3
             assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
             assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q", [64, 128])
+@pytest.mark.parametrize("alpha", [-2, 0.3])
+def test_undefined_elements_leave_their_neighbours_alone(dtype, q, alpha):
+    """Undefined gradients, more of them than a top-k block selects: state and parameters as the
+    op-by-op sequence leaves them, those of the elements packed into the same words included."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(3)
+    d = 20480 * 2 + 4096 + 40
+    start = (torch.randn(d, generator=gen) * 0.02).to(dtype)
+    g = (torch.randn(d, generator=gen) * 0.01).to(dtype)
+    g[torch.randperm(d, generator=gen)[:d // 20]] = float("nan")
+    states = []
+    for fused in (True, False):
+        p = torch.nn.Parameter(start.clone().cuda())
+        opt = MicroAdam([p], m=3, lr=1e-3, quant_block_size=q, alpha=alpha)
+        opt.use_fused = fused
+        for _ in range(2):
+            p.grad = g.clone().cuda()
+            opt.step()
+        st = opt.state[p]
+        states.append([p.data.float().cpu()] + [st[key].float().cpu() for key in
+                      ("error", "min_vals", "max_vals", "quant_err") if key in st])
+    for got, want in zip(*states):
+        assert np.array_equal(got.numpy(), want.numpy(), equal_nan=True)
