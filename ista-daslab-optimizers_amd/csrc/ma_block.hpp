@@ -241,6 +241,11 @@ __device__ __forceinline__ BlockGeo make_geo(const FusedParams &P, int ti, int64
 // which of them they fill and which they consume.
 //   FULL: the block has exactly kRound*C elements, so no chunk needs a bounds check.
 //   QL:   lanes per quantisation block fixed at compile time (4: q = 32, 8: q = 64), 0: any.
+// LDS of the segmented route's exchange: a quadruple per stretch of 512 elements, a pair per
+// quantisation block a top-k block meets
+constexpr int kSegParts = 64;
+constexpr int kSegmentBytes = kSegParts * 16 + (MA_MAX_D_BLOCK / kRowCutStep + 2) * 8;
+
 template <class R, bool FULL, int QL, int AUX = 0>
 struct FusedBlock {
     typedef typename R::elem_t elem_t;
@@ -2385,10 +2390,10 @@ struct FusedBlock {
         }
     }
 
-    // LDS of the exchange, where the selection's histograms were: the extremes of the two parts
-    // of every (wave, chunk), then the extremes of every quantisation block, which
-    // become its (min, step)
-    static constexpr int kSegMax = 32768 / kRowCutStep + 2;
+    // LDS of the exchange, where the selection's histograms were (kSegmentBytes of it): the extremes
+    // of the two parts of every (wave, chunk), then the extremes of every quantisation block,
+    // which become its (min, step)
+    static_assert(kWaves * C * sizeof(float4) <= kSegParts * sizeof(float4), "kSegmentBytes");
     __device__ __forceinline__ float4 *seg_parts() const { return reinterpret_cast<float4 *>(hist); }
     __device__ __forceinline__ float2 *seg_table() const {
         return reinterpret_cast<float2 *>(seg_parts() + kWaves * C);
@@ -2669,12 +2674,12 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
 // (the slot of block 0 of the launch's first tensor), the i-th deferred work item is word
 // kSpanDeferItem of the i-th slot from there (the launch has at most as many work items as
 // there are slots from its first to the end of the workspace).
-// Segmented route (quantisation blocks shorter than the top-k blocks), alpha == 0, no logging:
-// PASS 7 the step, PASS 9 the codes and statistics of the blocks it deferred, listed the same way.
 // (With alpha > 0 the one-pass form was built as well and measured slower than the two passes:
 // its second half needs the registers of the second pass on top of the residual, which costs
 // the third workgroup per CU or spills, and neither pass is short of memory bandwidth by
 // enough to pay for that.)
+// Segmented route (quantisation blocks shorter than the top-k blocks), alpha == 0, no logging:
+// PASS 7 the step, PASS 9 the codes and statistics of the blocks it deferred, listed the same way.
 constexpr int kSpanDeferItem = 4, kSpanDeferCount = 6;
 
 template <class R, int MIN_WAVES, int PASS, int AUX = 0>

@@ -518,9 +518,6 @@ static int fused_check(const ma_tensor *t, const ma_hyper *h, bool dense = false
 }
 
 constexpr int kSpanMaxBlocks = 64;  // top-k blocks one quantisation block may touch
-// LDS the segmented route's exchange takes in the union: a quadruple per stretch of 512 elements,
-// a pair per quantisation block
-constexpr int kSegmentBytes = 64 * 16 + (MA_MAX_D_BLOCK / kRowCutStep + 2) * 8;
 constexpr unsigned kSweepGroups = 256;  // workgroups of the sweep behind a one-pass launch
 
 // Polls a workgroup of the one-pass form spends at most on one neighbour's flag (each a sleep
