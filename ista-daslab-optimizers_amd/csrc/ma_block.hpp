@@ -237,15 +237,15 @@ __device__ __forceinline__ BlockGeo make_geo(const FusedParams &P, int ti, int64
     return G;
 }
 
-// The step of one block, cut into stages.  The register arrays are members; the stages say
-// which of them they fill and which they consume.
-//   FULL: the block has exactly kRound*C elements, so no chunk needs a bounds check.
-//   QL:   lanes per quantisation block fixed at compile time (4: q = 32, 8: q = 64), 0: any.
 // LDS of the segmented route's exchange: a quadruple per stretch of 512 elements, a pair per
 // quantisation block a top-k block meets
 constexpr int kSegParts = 64;
 constexpr int kSegmentBytes = kSegParts * 16 + (MA_MAX_D_BLOCK / kRowCutStep + 2) * 8;
 
+// The step of one block, cut into stages.  The register arrays are members; the stages say
+// which of them they fill and which they consume.
+//   FULL: the block has exactly kRound*C elements, so no chunk needs a bounds check.
+//   QL:   lanes per quantisation block fixed at compile time (4: q = 32, 8: q = 64), 0: any.
 template <class R, bool FULL, int QL, int AUX = 0>
 struct FusedBlock {
     typedef typename R::elem_t elem_t;
