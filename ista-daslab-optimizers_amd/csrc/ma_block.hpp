@@ -1361,13 +1361,7 @@ struct FusedBlock {
                 praw[c].to_float(pv);
                 update8(off, uv);
                 log_update(uv, FULL ? kChunk : n - off);
-                if (apply_decay) {
-#pragma unroll
-                    for (int e = 0; e < kChunk; ++e) {
-                        pv[e] = pv[e] * decay;
-                        if (R::kBF16) pv[e] = bf2f(f2bf(pv[e]));
-                    }
-                }
+                if (apply_decay) decay8(pv, decay);
 #pragma unroll
                 for (int e = 0; e < kChunk; ++e) {
                     const float prod = neg_lr * uv[e];
@@ -1384,11 +1378,6 @@ struct FusedBlock {
     // (for the update, which adds alpha * Qinv(e1)), and the error feedback that is stored is
     // Q of r2 = (1 - alpha) * Qinv(e1) with statistics of its own.
     uint32_t dcodes[C], dstat[C];  // e1 of the chunk; its min | max << 16 (bf16 bits)
-
-    // Blocks of up to 12288 elements have the registers for the second quantisation element by
-    // element in line, which for q = 8 and 16 costs less than trying 16 and 8 codes a lane
-    // (requantised_alike): 80 M parameters in blocks of 4096, q = 8, 386 us a step against 411.
-    static constexpr bool kDirect = R::kC < kClass2;
 
     __device__ __forceinline__ void quantize_dense(const BlockGeo &G) {
         const int n = FULL ? C * kRound : G.n;
@@ -1455,39 +1444,22 @@ struct FusedBlock {
             dcodes[c] = 0;
             const float mnf = bf2f(mnb);
             const float u = div15(bf2f(mxb) - mnf, d15);
-            float cf[kDirect ? 8 : 1];
-            if constexpr (kDirect) {  // (lanes past the end)
-#pragma unroll
-                for (int e = 0; e < kChunk; ++e) cf[e] = 0.0f;
-            }
             if (FULL || off < n) {
                 float code[8];
                 codes8(x, mnf, u, code);
 #pragma unroll
-                for (int e = 0; e < kChunk; ++e) {
+                for (int e = 0; e < kChunk; ++e)
                     if (!FULL && off + e >= n) code[e] = 0.0f;
-                    if constexpr (kDirect) cf[e] = code[e];
-                }
                 dcodes[c] = pack_codes_apart(code);
             }
             // (packed here and now: left to itself the compiler moves the packing to the update
             // and keeps the floats instead, which costs 42 spilled registers)
             asm volatile("" : "+v"(dcodes[c]), "+v"(dstat[c]));
             uint32_t mn2b, mx2b, codes;
-            // (a quantisation block that begins inside the block counts with all its lanes: those
-            // past the end hold no elements, but try codes that the others' elements may have)
-            const bool begun = FULL || (off & -(1 << q_shift)) < n;
-            bool done = false;
-            if constexpr (kDirect) {
-                done = ql < 4;
-                if (done) requantise_direct(cf, FULL ? kChunk : n - off, mnf, u, mn2b, mx2b, codes);
-            }
-            if (!done) {
-                if (requantised_alike(mn, mx, mnf, u, begun, mn2b, mx2b))
-                    codes = dcodes[c];
-                else
-                    requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
-            }
+            if (requantised_alike(mn, mx, mnf, u, FULL || off < n, mn2b, mx2b))
+                codes = dcodes[c];
+            else
+                requantise_chunk(c, off, n, long_q, mn, mx, mnf, u, mn2b, mx2b, codes);
             asm volatile("" : "+v"(codes), "+v"(mn2b), "+v"(mx2b));
             if (FULL || off < n) {
                 if ((lane & (ql - 1)) == 0) {
@@ -1517,41 +1489,26 @@ struct FusedBlock {
 
     // The second quantisation of alpha > 0 maps the 16 values r2(code) = (1 - alpha) * Qinv(code)
     // to codes again, and as r2 is linear in the code up to its rounding, code c nearly always
-    // maps to c: the rounding of r2 (2^-9 of it for bf16) would have to reach half a step, i.e.
-    // the block's values to lie many times its range away from zero.  So a quantisation block's
-    // lanes try the 16 codes between them instead of requantising their 8 elements each (q = 64:
-    // two divisions a lane instead of eight, and no second min / max; left out for run-time groups
-    // of fewer than 16 lanes, blocks of 12288 at q = 64 take 273 us a step instead of 223; a group
-    // of one lane, q = 8, is faster without: 247 us a step against 260 in blocks of 20480).  True, for the whole
-    // wave, if every block maps every code to itself; the statistics of r2 are then r2 at the
-    // codes of the block's extremes, 0 and 15.  `counts`: this lane's quantisation block has
-    // elements, be they other lanes' alone.
+    // maps to c.  r2(c) = A + c B + e_c with |e_c| <= E = 2^-8 M (1 + 2^-7), M the larger magnitude of
+    // r2(0) and r2(15): the rounding of r2, or of its extremes to bf16 statistics (half a unit of
+    // 8-bit significands), and the fp32 operations that form it.  Against the statistics
+    // m2 = r2(0), u2 = (r2(15) - r2(0)) / 15 the value (r2(c) - m2) / u2 lies within
+    // (|e_c| + |e_0| (1 - c/15) + |e_15| c/15) / u2 <= 2 E / u2 of c, so its code is c where
+    // 2 E < u2 / 2, i.e. M (1 + 2^-7) < 4.26 range: asked with a margin of 3 %, the block's range is more
+    // than about a quarter of its largest magnitude.  (Trying the 16 codes between the lanes of a
+    // quantisation block instead took 35 instructions more for every 8 elements of a lane.)  True,
+    // for the whole wave, if that holds for every block; the statistics of r2 are then r2 at the
+    // codes of the block's extremes, 0 and 15.  `counts`: this lane has elements.
     __device__ __forceinline__ bool requantised_alike(float mn, float mx, float mnf, float u,
                                                       bool counts, uint32_t &mn2b,
                                                       uint32_t &mx2b) const {
-        if (QL == 0 && ql < 2) return false;
         mn2b = f2bf(kept_value(0.0f, mnf, u));
         mx2b = f2bf(kept_value(15.0f, mnf, u));
-        const float m2f = bf2f(mn2b);
-        const float u2 = div15(bf2f(mx2b) - m2f, d15);
-        bool alike = divisor_is_plain(u) && divisor_is_plain(u2);
-        const Divisor dv2 = make_divisor(u2);
-        if constexpr (QL > 0) {
-            constexpr int kPer = 16 / (QL > 0 ? QL : 1);  // codes a lane tries
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const float code = (float)((lane & (QL - 1)) + i * QL);
-                const float y = kept_value(code, mnf, u) - m2f;
-                alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
-            }
-        } else {
-#pragma unroll 1
-            for (int i = lane & (min(ql, 16) - 1); i < 16; i += ql) {
-                const float code = (float)i;
-                const float y = kept_value(code, mnf, u) - m2f;
-                alike = alike && floorf(div_shared(y, dv2) + 0.5f) == code;
-            }
-        }
+        const float m2f = bf2f(mn2b), x2f = bf2f(mx2b);
+        const float range2 = x2f - m2f;  // 15 u2
+        // (plain: nothing that enters the bound is subnormal or overflows)
+        bool alike = divisor_is_plain(u) && divisor_is_plain(range2) &&
+                     fmax_raw(__builtin_fabsf(m2f), __builtin_fabsf(x2f)) < range2 * 4.1f;
         if constexpr (!R::kBF16) {
             // (bf16 extremes are their own statistics and get the codes 0 and 15)
             const Divisor dv = make_divisor(u);
@@ -1559,7 +1516,7 @@ struct FusedBlock {
                     div_shared(mx - mnf, dv) + 0.5f >= 15.0f;
         }
         // a range of zero: every code is 0, before and after
-        alike = alike || (u == 0.0f && fabsf(mnf) <= 3.0e38f);
+        alike = alike || (u == 0.0f && __builtin_fabsf(mnf) <= 3.0e38f);
         return __builtin_amdgcn_ballot_w64(counts && !alike) == 0;
     }
 
@@ -1569,32 +1526,6 @@ struct FusedBlock {
         deq = deq + mnf;
         const float keep = P.keep * deq;
         return to_elem(0.0f + keep);
-    }
-
-    // The second quantisation of a chunk with the codes cf, `valid` (or more) elements of it, whose
-    // quantisation block is not longer than a wave's stretch.
-    __device__ __forceinline__ void requantise_direct(const float (&cf)[8], int valid, float mnf,
-                                                      float u, uint32_t &mn2b, uint32_t &mx2b,
-                                                      uint32_t &codes) const {
-        float r2[8], c2[8];
-        float mn2 = INFINITY, mx2 = -INFINITY;
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) {
-            r2[e] = kept_value(cf[e], mnf, u);
-            if (e < valid) {
-                mn2 = fmin_raw(mn2, r2[e]);
-                mx2 = fmax_raw(mx2, r2[e]);
-            }
-        }
-        group_minmax<QL>(mn2, mx2, ql);
-        mn2b = f2bf(mn2);
-        mx2b = f2bf(mx2);
-        const float m2f = bf2f(mn2b);
-        codes8(r2, m2f, div15(bf2f(mx2b) - m2f, d15), c2);
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e)
-            if (e >= valid) c2[e] = 0.0f;
-        codes = pack_codes(c2);
     }
 
     // The second quantisation element by element: r2 from the codes of the chunk, its statistics,
@@ -1643,6 +1574,29 @@ struct FusedBlock {
         }
     }
 
+    // u = rne(Adam + alpha * Qinv(e1)) in place of the Adam direction uv, p += -lr * u, for the 8
+    // elements of chunk c with the codes dcodes[c] against (mnf, u)
+    __device__ __forceinline__ void step8_codes(int c, float mnf, float u, float neg_lr,
+                                                float (&uv)[8], float (&pv)[8]) const {
+        // (nibbles as bytes, one conversion each, as in dequant)
+        uint32_t odd = dcodes[c] & 0x0f0f0f0fu, even = (dcodes[c] >> 4) & 0x0f0f0f0fu;
+        asm volatile("" : "+v"(odd), "+v"(even));
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            const uint32_t code = (((e & 1) ? odd : even) >> (8 * (e >> 1))) & 0xffu;
+            float deq = (float)code * u;
+            deq = deq + mnf;
+            const float add = P.alpha * deq;
+            uv[e] = uv[e] + add;
+            if (e & 1) to_elem2(uv[e - 1], uv[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            const float prod = neg_lr * uv[e];
+            pv[e] = pv[e] + prod;
+        }
+    }
+
     // p = p * decay; u = rne(Adam + alpha * Qinv(e1)); p += -lr * u.  After window_stage.
     __device__ __forceinline__ void param_stage_dense(const BlockGeo &G) {
         const int n = FULL ? C * kRound : G.n;
@@ -1662,21 +1616,9 @@ struct FusedBlock {
                 update8(off, uv);
                 const float mnf = bf2f(dstat[c] & 0xffffu);
                 const float u = div15(bf2f(dstat[c] >> 16) - mnf, d15);
-#pragma unroll
-                for (int e = 0; e < kChunk; ++e) {
-                    if (apply_decay) pv[e] = to_elem(pv[e] * decay);
-                    const uint32_t code = (dcodes[c] >> (8 * (e >> 1) + ((e & 1) ? 0 : 4))) & 15u;
-                    float deq = (float)code * u;
-                    deq = deq + mnf;
-                    const float add = P.alpha * deq;
-                    const float ud = to_elem(uv[e] + add);
-                    const float prod = neg_lr * ud;
-                    pv[e] = pv[e] + prod;
-                    if (FULL || off + e < n) {
-                        log_square(kMtUpdate, ud);
-                        log_zero(kMtUpdateZeros, ud);
-                    }
-                }
+                if (apply_decay) decay8(pv, decay);
+                step8_codes(c, mnf, u, neg_lr, uv, pv);
+                log_update(uv, FULL ? kChunk : n - off);
                 store8(p, off, FULL ? 0x7fffffff : n, true, pv);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1905,6 +1847,26 @@ struct FusedBlock {
 
     static __device__ __forceinline__ float to_elem(float v) {
         return R::kBF16 ? bf2f(f2bf(v)) : v;
+    }
+    // the same of two values, one conversion for both
+    static __device__ __forceinline__ void to_elem2(float &a, float &b) {
+        if (R::kBF16) {
+            const uint32_t w = f2bf_pair(a, b);
+            a = __uint_as_float(w << 16);
+            b = __uint_as_float(w & 0xffff0000u);
+        }
+    }
+    // p = p * decay of 8 parameters (MA:234-235).  Called under a branch that is the same for the
+    // whole workgroup; the empty asm keeps it a branch (as selects it costs four instructions an
+    // element when there is no decay, a fifth of the densified update stage).
+    static __device__ __forceinline__ void decay8(float (&pv)[8], float decay) {
+#pragma unroll
+        for (int e = 0; e < kChunk; e += 2) {
+            pv[e] = pv[e] * decay;
+            pv[e + 1] = pv[e + 1] * decay;
+            to_elem2(pv[e], pv[e + 1]);
+        }
+        asm volatile("");
     }
 
     // ---- pass 1 ------------------------------------------------------------------------------
@@ -2620,8 +2582,9 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
         if constexpr (DENSE) {
             // 1.07 G bf16 parameters, q = 64: 2.67 ms with codes and statistics of e1 left to the
             // compiler (42 spilled registers), the narrow window stage and all elements
-            // quantised twice; 1.90 ms so.  (The parameters asked for before the window: the same
-            // 1.89 ms and five spilled registers.)
+            // quantised twice; 1.87 ms without; 1.69 with the codes of the second quantisation taken
+            // from a bound, decay under a branch and two elements to a conversion (2726 to 2380
+            // vector instructions a wave, whose issue bounds this kernel: floor of its bytes 1.37).
             // Blocks of up to 12288 elements have the registers for the order of the plain step, and
             // gain by the narrow stage: 80 M parameters in blocks of 12288, q = 64, 243 us a step
             // with the wide one, 223 so; in blocks of 4096 390 and 380.
@@ -2952,15 +2915,12 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void window_param_kernel(FusedParam
     auto step8 = [&](int off, const RawChunk<R> &praw, const float (&a1)[8], const float (&a2)[8]) {
         float pv[8];
         praw.to_float(pv);
+        if (apply_decay) FusedBlock<R, false, 0>::decay8(pv, decay);
 #pragma unroll
         for (int e = 0; e < kChunk; ++e) {
             float u = 0.0f;
             if (a1[e] != 0.0f || a2[e] != 0.0f) {
                 u = adam_update<R::kBF16>(a1[e], a2[e], P.W.s1, P.W.s2, P.W.eps);
-            }
-            if (apply_decay) {
-                pv[e] = pv[e] * decay;
-                if (R::kBF16) pv[e] = bf2f(f2bf(pv[e]));
             }
             const float prod = neg_lr * u;
             pv[e] = pv[e] + prod;

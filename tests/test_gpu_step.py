@@ -1018,3 +1018,32 @@ def test_undefined_elements_leave_their_neighbours_alone(dtype, q, alpha):
                       ("error", "min_vals", "max_vals", "quant_err") if key in st])
     for got, want in zip(*states):
         assert np.array_equal(got.numpy(), want.numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q,DB", [(8, 4096), (32, 20480), (64, 20480), (512, 20480)])
+def test_densified_second_quantisation_around_its_bound(oracle, q, DB, dtype):
+    """Blocks from once to nine times their range from zero: the kernels take the second codes to be
+    the first ones where the larger magnitude is below 4.1 times the range (of the rounded
+    statistics), and form them element by element beyond."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(q)
+    d = DB + 7 * q
+    which = torch.arange(d) // q
+    far = torch.linspace(1.0, 9.0, int(which.max()) + 1, dtype=torch.float64)[which].float()
+    sign = torch.where(which % 3 == 0, -1.0, 1.0)
+    width = 2.0 ** (which % 5 - 9).float()
+    params = [(torch.randn(d, generator=gen) * 0.02).to(dtype)]
+    oparams = [to_np(params[0])]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=DB)
+    gp = torch.nn.Parameter(params[0].clone().cuda())
+    opt = MicroAdam([gp], m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
+    opt.d_block_size = DB
+    for step in range(2):
+        g = (sign * width * (far + torch.rand(d, generator=gen) - 0.5)).to(dtype)
+        gp.grad = g.cuda()
+        opt.step()
+        assert opt._fusable(gp, opt.state[gp]) == 3
+        oref.step([to_np(g)])
+        assert_state_equal(opt.state[gp], oref.state[0], f"step {step + 1}")
+        assert np.array_equal(to_np(gp.data), oparams[0]), f"step {step + 1}: parameters"
