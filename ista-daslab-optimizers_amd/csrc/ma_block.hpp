@@ -59,7 +59,7 @@ struct TensorDesc {
     float decay;
     int32_t apply_decay;
     int32_t blk0;         // block of the tensor that its first work item stands for
-    float *ws;            // two-pass route: per-block extremes of the residual;
+    float *ws;            // spanning route: per-block extremes of the residual;
                           // alpha == -2: st['quant_err'] (elements of the data's type);
                           // two-launch form of dense windows: the cache of row cuts (uint16
                           // words) or null; else unused
@@ -78,7 +78,7 @@ struct FusedParams {
     int32_t q_shift;  // log2(quant_block_size)
     int32_t total_items;  // work items (blocks) of the launch
     int32_t short_items;  // of them, at the end: tensors shorter than a top-k block, one item each
-    // two-pass route (quantisation blocks at least as long as the top-k blocks)
+    // spanning route (quantisation blocks at least as long as the top-k blocks)
     int32_t q_span;   // quantisation block length, a multiple of 8
     float alpha;      // share of the dequantised error feedback added to the update
     float keep;       // (float)(1 - alpha): share that stays in the error feedback
@@ -87,7 +87,7 @@ struct FusedParams {
     // the window is window_param_kernel's: the block kernel ends with the quantisation (but not
     // a logging step's) and lists its rows by coordinate where it can
     int32_t win_apart;
-    // one-pass form of the two-pass route: polls a workgroup spends at most on waiting for the
+    // one-pass forms: polls a workgroup spends at most on waiting for the
     // extremes of the blocks that share its quantisation blocks (0: it does not wait at all)
     int32_t spin_limit;
 };
@@ -105,7 +105,7 @@ struct FusedParams {
 //            straight into the parameters, p = p - a, then p = p + Qinv(e) (each rounded to
 //            the parameter's type) before the Adam step.
 constexpr int kAuxLog = 1, kAuxQuantErr = 2;
-constexpr int kSpanWords = 8;  // workspace words per top-k block of the two-pass route
+constexpr int kSpanWords = 8;  // workspace words per top-k block of the spanning route
 constexpr int kRowCutStep = 512;  // coordinates between two cuts of a window row
 constexpr int kHintLongRow = 4 * 512;  // longest block row whose previous threshold is looked up
 
@@ -758,9 +758,15 @@ struct FusedBlock {
     //      and p += -lr * u (MA:304).  The slot cells end up holding the update's bits, 0
     //      where no window row names the coordinate.
     __device__ __forceinline__ void update(const BlockGeo &G) {
-        if (P.L.cell_bytes == 0) {
+        if (P.L.cell_bytes == 0)
             update_by_ranges(G);
-        } else if (wide) {
+        else
+            update_in_cells(G);
+    }
+
+    // the same where the LDS plan has cells (always, on the spanning and the segmented route)
+    __device__ __forceinline__ void update_in_cells(const BlockGeo &G) {
+        if (wide) {
             update_wide(G);
         } else {
             window_stage(G);
@@ -1520,6 +1526,11 @@ struct FusedBlock {
         return __builtin_amdgcn_ballot_w64(counts && !alike) == 0;
     }
 
+    // a value that is the same in every lane, kept in a scalar register from here on
+    static __device__ __forceinline__ float same_in_all(float v) {
+        return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+    }
+
     // r2 of a code: what of Qinv(code) stays in the error feedback, in the element type
     __device__ __forceinline__ float kept_value(float code, float mnf, float u) const {
         float deq = code * u;
@@ -1626,9 +1637,9 @@ struct FusedBlock {
     }
 
     // =========================================================================================
-    // Two-pass route: quantisation blocks of q_span >= block length elements (q_span a
-    // multiple of 8), so a top-k block meets at most two of them and their statistics need
-    // every top-k block they cover.  0 <= alpha < 1 (alpha > 0: MA:296-298, 311-316).
+    // Quantisation blocks of q_span >= block length elements (q_span a multiple of 8), so a
+    // top-k block meets at most two of them and their statistics need every top-k block they
+    // cover.  0 <= alpha < 1 (alpha > 0: MA:296-298, 311-316).  In two passes (logging steps):
     //   pass 1: a = g + Qinv(e), top-k, window row; the residual r goes to the gradient
     //           buffer, its exact min / max per (block, segment) to the workspace
     //   pass 2: statistics of r from the workspace; e1 = Q(r), d1 = Qinv(e1) in registers;
@@ -1641,7 +1652,7 @@ struct FusedBlock {
     // segment 1 the rest.  Workspace: a slot of 8 words per block: min0, max0, min1, max1
     // (floats), then four words the one-pass form uses for its list of deferred blocks.
     //
-    // One-pass form (the same arithmetic, the residual never leaves the registers; the
+    // In one pass (the same arithmetic, the residual never leaves the registers; the
     // workspace starts with the four floats of every block as all-ones words and the rest
     // zero): a workgroup publishes the extremes of its block right after the selection, goes
     // on with what does not need the statistics, and then takes the extremes of the blocks
@@ -1649,7 +1660,7 @@ struct FusedBlock {
     // neighbours, neighbouring blocks are dispatched together, and every workgroup publishes
     // before it waits, so the wait is short; it is bounded all the same (spin_limit polls), and
     // a workgroup that gives up stores its residual in the gradient buffer and lists its block:
-    // a second launch takes the listed blocks through the second pass of the two-pass form.
+    // a second launch takes the listed blocks through the second pass of the two-pass form (alpha > 0: window and parameters too).
     // The old statistics of a quantisation block are overwritten by the block that holds its
     // first element only after that block has seen all blocks of the quantisation block
     // published, i.e. after all of them have read the old statistics.
@@ -1979,32 +1990,47 @@ struct FusedBlock {
     __device__ __forceinline__ void span_publish(const BlockGeo &G, const Span &S) {
         const int n = FULL ? C * kRound : G.n;
         float mn[2] = {INFINITY, INFINITY}, mx[2] = {-INFINITY, -INFINITY};
+        if (FULL && S.bnd == 0x7fffffff) {  // (four blocks in five at q = 100000)
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int off = chunk_off<C>(wave, c, lane);
-            if (FULL || off < n) {
+            for (int c = 0; c < C; ++c) {
                 float x[8];
-                float lmn = INFINITY, lmx = -INFINITY;
 #pragma unroll
                 for (int e = 0; e < kChunk; ++e) x[e] = r.val(c, e);
-                if (FULL) {
-                    minmax8(x, lmn, lmx);
-                } else {
+                minmax8(x, mn[0], mx[0], mn[0], mx[0]);
+            }
+        } else {
 #pragma unroll
-                    for (int e = 0; e < kChunk; ++e) {
-                        if (off + e < n) {
-                            lmn = fmin_raw(lmn, x[e]);
-                            lmx = fmax_raw(lmx, x[e]);
+            for (int c = 0; c < C; ++c) {
+                const int off = chunk_off<C>(wave, c, lane);
+                if (FULL || off < n) {
+                    float x[8];
+                    float lmn = INFINITY, lmx = -INFINITY;
+#pragma unroll
+                    for (int e = 0; e < kChunk; ++e) x[e] = r.val(c, e);
+                    if (FULL) {
+                        minmax8(x, lmn, lmx);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < kChunk; ++e) {
+                            if (off + e < n) {
+                                lmn = fmin_raw(lmn, x[e]);
+                                lmx = fmax_raw(lmx, x[e]);
+                            }
                         }
                     }
+                    const bool second = off >= S.bnd;
+                    mn[0] = fmin_raw(mn[0], second ? INFINITY : lmn);
+                    mx[0] = fmax_raw(mx[0], second ? -INFINITY : lmx);
+                    mn[1] = fmin_raw(mn[1], second ? lmn : INFINITY);
+                    mx[1] = fmax_raw(mx[1], second ? lmx : -INFINITY);
                 }
-                const bool second = off >= S.bnd;
-                mn[0] = fmin_raw(mn[0], second ? INFINITY : lmn);
-                mx[0] = fmax_raw(mx[0], second ? -INFINITY : lmx);
-                mn[1] = fmin_raw(mn[1], second ? lmn : INFINITY);
-                mx[1] = fmax_raw(mx[1], second ? lmx : -INFINITY);
             }
         }
+        publish_extremes(G, mn, mx);
+    }
+
+    __device__ __forceinline__ void publish_extremes(const BlockGeo &G, float (&mn)[2],
+                                                     float (&mx)[2]) {
         wg_minmax2(mn, mx);
         if (tid == 0) {
             // One 64-bit store per segment, past this XCD's L2 (device scope) and without any
@@ -2087,9 +2113,12 @@ struct FusedBlock {
     __device__ __forceinline__ void span_defer(const BlockGeo &G) {
         const int n = FULL ? C * kRound : G.n;
         elem_t *out = reinterpret_cast<elem_t *>(const_cast<void *>(G.D.g)) + G.e0;
+        // (store addresses formed afresh: kept from the loads, they would sit in registers, or in
+        // scratch, up to this branch)
+        const int tid2 = opaque_tid(), lane2 = tid2 & 63, wave2 = tid2 >> 6;
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const int off = chunk_off<C>(wave, c, lane);
+            const int off = chunk_off<C>(wave2, c, lane2);
             if (FULL || off < n) {
                 float x[8];
 #pragma unroll
@@ -2274,6 +2303,103 @@ struct FusedBlock {
             __builtin_amdgcn_sched_barrier(0);
         }
         span_store_statistics(G, S);
+    }
+
+    // alpha > 0, one pass: e1 = Q(r) against the statistics of r, packed into dcodes for the
+    // update, which frees the residual's registers before the parameters are asked for; the error
+    // feedback that is stored is e1's codes taken to those of r2.  That map has 16 entries per
+    // segment, which the lanes of every wave form side by side (lane 16 s + c: segment s, code c);
+    // it nearly always takes every code to itself (see requantised_alike), and then the codes
+    // are stored as they are.
+    __device__ __forceinline__ void span_dense_codes(const BlockGeo &G, const Span &S) {
+        const int n = FULL ? C * kRound : G.n;
+        uint8_t *err = G.D.err + (G.e0 >> 1);
+        const float mn0 = bf2f(sp_mn[0]), mn1 = bf2f(sp_mn[1]);
+        const float u0 = same_in_all(div15(bf2f(sp_mx[0]) - mn0, d15));
+        const float u1 = same_in_all(div15(bf2f(sp_mx[1]) - mn1, d15));
+        uint32_t second_code;
+        bool alike;
+        {
+            const float m20 = bf2f(sp2_mn[0]), m21 = bf2f(sp2_mn[1]);
+            const float v0 = div15(bf2f(sp2_mx[0]) - m20, d15);
+            const float v1 = div15(bf2f(sp2_mx[1]) - m21, d15);
+            const bool second = (lane & 16) != 0;
+            const float r2 = kept_value((float)(lane & 15), second ? mn1 : mn0, second ? u1 : u0);
+            float x[8], cf[8];
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e) x[e] = r2;  // (eight times the same)
+            codes8(x, second ? m21 : m20, second ? v1 : v0, cf);
+            second_code = (uint32_t)cf[0];
+            const bool meant = !second || S.bnd != 0x7fffffff;
+            alike = __builtin_amdgcn_ballot_w64(meant && second_code != (uint32_t)(lane & 15)) == 0;
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int off = chunk_off<C>(wave, c, lane);
+            const bool second = off >= S.bnd;
+            float x[8], cf[8];
+            residual8<true>(c, x);
+            codes8(x, second ? mn1 : mn0, second ? u1 : u0, cf);
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e)
+                if (!FULL && off + e >= n) cf[e] = 0.0f;
+            dcodes[c] = pack_codes_apart(cf);
+            // (packed here and now, as in quantize_dense)
+            asm volatile("" : "+v"(dcodes[c]));
+            uint32_t codes = dcodes[c];
+            if (!alike) {
+                codes = 0;
+#pragma unroll 1
+                for (int i = 0; i < 32; i += 4) {
+                    const uint32_t code = (dcodes[c] >> i) & 15u;
+                    codes |= (uint32_t)__shfl((int)second_code, (int)(code + (second ? 16u : 0u)),
+                                              kWave) << i;
+                }
+            }
+            if (FULL || off < n) {
+                if (FULL || off + kChunk <= n) {
+                    *reinterpret_cast<uint32_t *>(err + ((unsigned)off >> 1)) = codes;
+                } else {
+                    // (the half byte behind an odd last element stays 0, whatever code 0 becomes)
+                    if ((n & 1) != 0) codes &= ~(15u << ((n - 1 - off) * 4));
+                    const int nbytes = (n - off + 1) >> 1;
+                    for (int j = 0; j < nbytes; ++j)
+                        err[(off >> 1) + j] = (uint8_t)(codes >> (8 * j));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        span_store_statistics(G, S);
+    }
+
+    // Its last stage: p = p * decay; u = rne(Adam + alpha * Qinv(e1)); p += -lr * u.  After
+    // window_cells.
+    __device__ __forceinline__ void span_param_stage_codes(const BlockGeo &G, const Span &S) {
+        const int n = FULL ? C * kRound : G.n;
+        const TensorDesc &D = G.D;
+        elem_t *p = reinterpret_cast<elem_t *>(D.p) + G.e0;
+        const float neg_lr = D.neg_lr, decay = D.decay;
+        const bool apply_decay = decay_pending(G);
+        const float mn0 = bf2f(sp_mn[0]), mn1 = bf2f(sp_mn[1]);
+        const float u0 = same_in_all(div15(bf2f(sp_mx[0]) - mn0, d15));
+        const float u1 = same_in_all(div15(bf2f(sp_mx[1]) - mn1, d15));
+        // (store addresses formed afresh, as in param_stage)
+        const int tid2 = opaque_tid(), lane2 = tid2 & 63, wave2 = tid2 >> 6;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int off = chunk_off<C>(wave2, c, lane2);
+            if (FULL || off < n) {
+                const bool second = off >= S.bnd;
+                const float mnf = second ? mn1 : mn0, u = second ? u1 : u0;
+                float pv[8], uv[8];
+                praw[c].to_float(pv);
+                update8(off, uv);
+                if (apply_decay) decay8(pv, decay);
+                step8_codes(c, mnf, u, neg_lr, uv, pv);
+                store8(p, off, FULL ? 0x7fffffff : n, true, pv);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 
     // =========================================================================================
@@ -2624,23 +2750,28 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
     }
 }
 
-// Two-pass route, see FusedBlock; one workgroup per block.
+// Quantisation blocks at least as long as the top-k blocks, see FusedBlock; one workgroup per block.
+// Logging steps take two passes:
 //   alpha > 0:  PASS 1 (residual and its extremes), PASS 2 (everything else)
 //   alpha == 0: PASS 4 (PASS 1 and the parameter update, which does not wait for the
 //               statistics), PASS 3 (codes of the residual)
-//   Logging steps: the first pass leaves |g|^2 (and, as PASS 4, the update's sums) and clears
-//   the components no pass forms; the second leaves the rest.
-// One-pass form of the same route, alpha == 0, no logging: PASS 6 does the whole step of a block,
-// exchanging the extremes of the residual through the workspace; PASS 8 is PASS 3 for the blocks
-// PASS 6 deferred, launched behind it with a fixed number of workgroups.  The deferred blocks are
-// listed: their count is word kSpanDeferCount of the first block slot of the launch's workspace
-// (the slot of block 0 of the launch's first tensor), the i-th deferred work item is word
-// kSpanDeferItem of the i-th slot from there (the launch has at most as many work items as
-// there are slots from its first to the end of the workspace).
-// (With alpha > 0 the one-pass form was built as well and measured slower than the two passes:
-// its second half needs the registers of the second pass on top of the residual, which costs
-// the third workgroup per CU or spills, and neither pass is short of memory bandwidth by
-// enough to pay for that.)
+//   The first pass leaves |g|^2 (and, as PASS 4, the update's sums) and clears the components no
+//   pass forms; the second leaves the rest.
+// All others take one pass, exchanging the extremes of the residual through the workspace, and a
+// second launch of a fixed number of workgroups behind it for the blocks that gave up waiting:
+//   alpha == 0: PASS 6 does the whole step of a block (PASS 8: PASS 3 for the deferred ones)
+//   alpha > 0:  PASS 10 likewise (PASS 11: PASS 2 for the deferred ones, whose window and
+//               parameters PASS 10 has left alone)
+// The deferred blocks are listed: their count is word kSpanDeferCount of the first block slot of
+// the launch's workspace (the slot of block 0 of the launch's first tensor), the i-th deferred work
+// item is word kSpanDeferItem of the i-th slot from there (the launch has at most as many work
+// items as there are slots from its first to the end of the workspace).
+// alpha > 0, 2.8 G bf16 parameters in the Llama-3-8B layer shapes, q = 100000: 5.67 ms a step in two
+// passes (11.4 bytes a parameter: the residual is written and read), 4.90 in one (8.4).  PASS 10 is
+// bound by the issue of its 2640 vector instructions a wave (4.7 ms at 2.4 GHz); what lets it
+// keep three workgroups per CU is that e1 is packed into codes as soon as the statistics are there,
+// so that the residual's registers are free for the window and the parameters (with the residual
+// held through the update: 116 registers or spills, 20 ms for 8 G parameters against 17).
 // Segmented route (quantisation blocks shorter than the top-k blocks), alpha == 0, no logging:
 // PASS 7 the step, PASS 9 the codes and statistics of the blocks it deferred, listed the same way.
 constexpr int kSpanDeferItem = 4, kSpanDeferCount = 6;
@@ -2648,10 +2779,11 @@ constexpr int kSpanDeferItem = 4, kSpanDeferCount = 6;
 template <class R, int MIN_WAVES, int PASS, int AUX = 0>
 __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P) {
     extern __shared__ __align__(16) unsigned char lds[];
-    constexpr bool kSweep = PASS == 8 || PASS == 9, kSegmented = PASS == 7 || PASS == 9;
+    constexpr bool kSweep = PASS == 8 || PASS == 9 || PASS == 11;
+    constexpr bool kSegmented = PASS == 7 || PASS == 9;
     uint32_t *slots = reinterpret_cast<uint32_t *>(P.t[0].ws);
     uint32_t *defer_count = slots + kSpanDeferCount;
-    // (PASS 6 and 7) this block gives up: listed for the sweep
+    // (PASS 6, 7 and 10) this block gives up: listed for the sweep
     auto list_deferred = [&](int item) {
         if (threadIdx.x == 0) {
             const uint32_t at = atomicAdd(defer_count, 1u);
@@ -2696,7 +2828,7 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
                 fb.load_params_window(G);
                 fb.update(G);
             }
-        } else if constexpr (PASS == 2) {
+        } else if constexpr (PASS == 2 || PASS == 11) {
             fb.span_load_row(G);
             fb.load_older_rows(G);
             fb.span_load_residual(G);
@@ -2712,6 +2844,23 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
             fb.span_load_residual(G);
             fb.template span_statistics<false>(G, S);
             fb.span_codes_stage(G, S);
+        } else if constexpr (PASS == 10) {
+            fb.span_load_grad_inputs(G, S);
+            fb.span_dequant(G, S);
+            fb.topk_and_row(G);
+            fb.span_publish(G, S);
+            launder(fb.r);  // (or the residual waits unpacked, in twice its registers)
+            if (!fb.template span_await<true>(G, S)) {
+                launder(fb.r);
+                fb.span_defer(G);  // (window and parameters too are the sweep's then)
+                list_deferred(item);
+                return;
+            }
+            fb.span_dense_codes(G, S);
+            fb.load_older_rows(G);
+            fb.window_cells(G);
+            fb.load_params(G);
+            fb.span_param_stage_codes(G, S);
         } else {  // PASS 6
             fb.span_load_grad_inputs(G, S);
             fb.span_dequant(G, S);
@@ -2727,7 +2876,7 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
                 list_deferred(item);
             }
             fb.load_params_window(G);
-            fb.update(G);
+            fb.update_in_cells(G);
         }
         constexpr unsigned kUnused = 1u << kMtQuantErr | 1u << kMtQuantErrZeros | 3u << 6;
         constexpr unsigned kUpdate = 1u << kMtUpdate | 1u << kMtUpdateZeros;
@@ -3181,18 +3330,21 @@ static int launch_span_one(int pass, unsigned grid, int lds_bytes, hipStream_t s
     case PASS_:                                                                                \
         if (grid == 0) return allow_big_lds(span_step_kernel<R, WAVES_, PASS_, AUX>, LDS_);    \
         return launch_kernel(span_step_kernel<R, WAVES_, PASS_, AUX>, dim3(grid), kWG, LDS_, s, P);
-    switch (pass) {
-        MA_SPAN_CASE(1, kFirst, lds_bytes)
-        MA_SPAN_CASE(2, kFirst, lds_bytes)
-        MA_SPAN_CASE(4, kFirst, lds_bytes)
-        MA_SPAN_CASE(3, kMinWaves, kMiscBytes)  // needs the kSh* words only
-    }
-    if constexpr (AUX == 0) {  // the one-pass form and its sweeps
+    if constexpr (AUX != 0) {  // logging steps
+        switch (pass) {
+            MA_SPAN_CASE(1, kFirst, lds_bytes)
+            MA_SPAN_CASE(2, kFirst, lds_bytes)
+            MA_SPAN_CASE(4, kFirst, lds_bytes)
+            MA_SPAN_CASE(3, kMinWaves, kMiscBytes)  // needs the kSh* words only
+        }
+    } else {  // the one-pass forms and their sweeps
         switch (pass) {
             MA_SPAN_CASE(6, kFirst, lds_bytes)
             MA_SPAN_CASE(8, kMinWaves, kMiscBytes)
             MA_SPAN_CASE(7, kFirst, lds_bytes)
             MA_SPAN_CASE(9, kMinWaves, lds_bytes)
+            MA_SPAN_CASE(10, kFirst, lds_bytes)
+            MA_SPAN_CASE(11, kMinWaves, lds_bytes)
         }
     }
 #undef MA_SPAN_CASE

@@ -134,6 +134,13 @@ __device__ __forceinline__ void minmax8(const float (&x)[8], float &mn, float &m
     mx = fmax_raw(fmax3_raw(fmax3_raw(fmax3_raw(x[0], x[1], x[2]), x[3], x[4]), x[5], x[6]), x[7]);
 }
 
+// the same with the extremes so far: still four each
+__device__ __forceinline__ void minmax8(const float (&x)[8], float mn0, float mx0, float &mn,
+                                        float &mx) {
+    mn = fmin3_raw(fmin3_raw(fmin3_raw(fmin3_raw(mn0, x[0], x[1]), x[2], x[3]), x[4], x[5]), x[6], x[7]);
+    mx = fmax3_raw(fmax3_raw(fmax3_raw(fmax3_raw(mx0, x[0], x[1]), x[2], x[3]), x[4], x[5]), x[6], x[7]);
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_perm(float v) {
     return __int_as_float(

@@ -533,7 +533,7 @@ static int span_spin_limit() {
     return 256;
 }
 
-// the two-pass route: 0 <= alpha < 1, quantisation blocks a multiple of 8 and at least as long
+// the spanning route: 0 <= alpha < 1, quantisation blocks a multiple of 8 and at least as long
 // as the top-k blocks
 static int span_check(const ma_tensor *t, const ma_hyper *h, double alpha) {
     Geometry g;
@@ -890,7 +890,7 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
     //      either steps every tensor or none
     std::vector<PlannedLaunch> plan;
     int64_t items_before = 0;  // work items of the launches laid out so far
-    // the two-pass route's workspace is handed out in the order the tensors are laid out, so the
+    // the spanning route's workspace is handed out in the order the tensors are laid out, so the
     // slots of a launch's tensors follow each other from those of its first tensor
     int64_t ws_off = 0;
     // tensors whose window is too large for the one-pass stage are stepped in two launches
@@ -1008,9 +1008,9 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
 
     // Two rounds over the plan: the first prepares every launch (kernel attributes: all that
     // can fail apart from a launch itself), the second launches.
-    // the one-pass form of the two-pass route (every step but a logging one) starts from a
+    // the one-pass forms (every step but a logging one) start from a
     // cleared workspace: its flags and counts are set as the blocks go
-    const bool one_pass = span && !aux && !(alpha > 0.0);
+    const bool one_pass = span && !aux;
     for (int round = 0; round < 2; ++round)
     for (const PlannedLaunch &L : plan) {
         if (one_pass && round == 1 && &L == &plan.front()) {
@@ -1043,10 +1043,10 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             rc = bf16 ? launch_fused_bf16(L.C, grid, P.L.total, s, P)
                       : launch_fused_f32(L.C, grid, P.L.total, s, P);
         } else {
-            // alpha > 0 and logging steps: two passes; else one pass and the sweep over the
-            // blocks it deferred
-            const int passes[2] = {segmented ? 7 : alpha > 0.0 ? 1 : one_pass ? 6 : 4,
-                                   segmented ? 9 : alpha > 0.0 ? 2 : one_pass ? 8 : 3};
+            // logging steps: two passes; else one pass and the sweep over the blocks it deferred
+            const bool dense_span = alpha > 0.0;
+            const int passes[2] = {segmented ? 7 : one_pass ? (dense_span ? 10 : 6) : dense_span ? 1 : 4,
+                                   segmented ? 9 : one_pass ? (dense_span ? 11 : 8) : dense_span ? 2 : 3};
             for (int i = 0; i < 2 && rc == 0; ++i) {
                 unsigned g2 = grid;
                 if (one_pass && i == 1 && grid > kSweepGroups) g2 = kSweepGroups;

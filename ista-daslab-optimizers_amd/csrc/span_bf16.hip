@@ -1,4 +1,4 @@
-// The two-pass (spanning) step kernels for bf16 data.
+// The spanning (one-pass) and segmented step kernels for bf16 data.
 #include "ma_block.hpp"
 
 namespace ma {

@@ -1047,3 +1047,63 @@ def test_densified_second_quantisation_around_its_bound(oracle, q, DB, dtype):
         oref.step([to_np(g)])
         assert_state_equal(opt.state[gp], oref.state[0], f"step {step + 1}")
         assert np.array_equal(to_np(gp.data), oparams[0]), f"step {step + 1}: parameters"
+
+
+@pytest.mark.parametrize("spin", [None, "0"], ids=["exchange", "deferred"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q,DB", [(24576, 20480), (520, 512), (8192, 4096), (16384, 12288)])
+def test_spanning_second_quantisation(oracle, monkeypatch, spin, q, DB, dtype):
+    """alpha > 0 with long quantisation blocks: blocks around zero, at 3, 30 and 300 times their
+    range from it (where the kept share's codes are not the first ones) and blocks of zeros, tensors
+    with an odd last element; exchanged in one pass, and every block deferred to the sweep."""
+    from ista_daslab_optimizers import MicroAdam
+    if spin is not None:
+        monkeypatch.setenv("MA_SPAN_SPIN_LIMIT", spin)
+    gen = torch.Generator().manual_seed(q)
+    sizes = [6 * q + 77, q // 2 + 1]
+    params = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in params]
+    oref = oracle.OracleMicroAdam(oparams, 3, 1e-3, q, 0.01, 0.3, d_block_size=DB)
+    gparams = [torch.nn.Parameter(p.clone().cuda()) for p in params]
+    opt = MicroAdam(gparams, m=3, lr=1e-3, quant_block_size=q, k_init=0.01, alpha=0.3)
+    opt.d_block_size = DB
+    for step in range(4):
+        grads = []
+        for n in sizes:
+            kind = (torch.arange(n) // q + step // 2) % 5
+            g = torch.tensor([0.0, 0.03, 0.3, 3.0, 0.0])[kind] + torch.randn(n, generator=gen) * 0.003
+            g[kind == 4] = 0.0
+            grads.append(g.to(dtype))
+        for p, g in zip(gparams, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        oref.step([to_np(g) for g in grads])
+        for i, p in enumerate(gparams):
+            assert opt._fusable(p, opt.state[p]) == 2
+            assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_spanning_route_takes_what_the_op_by_op_route_takes(dtype, value):
+    """alpha > 0: infinite and undefined gradients, more of them than a top-k block selects."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(3)
+    d = 20480 * 6 + 4096
+    start = (torch.randn(d, generator=gen) * 0.02).to(dtype)
+    g = (torch.randn(d, generator=gen) * 0.01).to(dtype)
+    g[20480:20480 * 2][torch.randperm(20480, generator=gen)[:1000]] = value
+    states = []
+    for fused in (True, False):
+        p = torch.nn.Parameter(start.clone().cuda())
+        opt = MicroAdam([p], m=3, lr=1e-3, quant_block_size=40960, alpha=0.5)
+        opt.use_fused = fused
+        for _ in range(2):
+            p.grad = g.clone().cuda()
+            opt.step()
+        st = opt.state[p]
+        states.append([p.data.float().cpu()] + [st[key].float().cpu() for key in
+                      ("error", "min_vals", "max_vals")])
+    for got, want in zip(*states):
+        assert np.array_equal(got.numpy(), want.numpy(), equal_nan=True)
