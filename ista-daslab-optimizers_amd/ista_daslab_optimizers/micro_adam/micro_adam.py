@@ -22,7 +22,6 @@ missing library, a missing GPU or a CPU tensor raises.
 """
 import ctypes
 import math
-import operator
 import time
 
 import numpy as np
@@ -32,7 +31,7 @@ import torch.distributed as dist
 import ista_daslab_cuda_micro_adam as _ext_quant
 import ista_daslab_cuda_tools as _ext_tools
 
-from .. import _hip
+from .. import _hip, _step_table
 from ..tools import block_split, get_first_device, get_gpu_mem_usage
 
 try:  # logging is optional here; the reference imports wandb unconditionally (micro_adam.py:5)
@@ -66,6 +65,7 @@ class _Table:
     def __init__(self, entries):
         self.entries = entries
         self.records = (_hip.MaTensor * len(entries))()
+        self.address = ctypes.addressof(self.records)
         self.view = np.frombuffer(self.records, dtype=_TENSOR_RECORD)
         for name in ('error', 'min_vals', 'max_vals', 'I', 'V'):
             self.view[name] = [e.st[name].data_ptr() for e in entries]
@@ -84,59 +84,24 @@ class _Table:
         self.view['index'] = [e.st['index'] for e in es]
 
 
-_dtype_of = operator.attrgetter('dtype')
-_grad_of = operator.attrgetter('grad')
-_index_column = operator.itemgetter('I')
-_row_of = operator.itemgetter('index')
-_address_of = torch.Tensor.data_ptr
-_is_contiguous = torch.Tensor.is_contiguous
-
-
 class _Uniform:
     """A step all of whose tensors went through one table: what the next one needs to refresh the
     table in whole columns.  Rebuilt by the general walk whenever that did not hold."""
-    __slots__ = ('walk', 'params', 'states', 'spans', 'route', 'dtype', 'table')
+    __slots__ = ('walk', 'params', 'states', 'route', 'dtype', 'tag', 'table')
 
     def __init__(self, walk, route, dtype, table):
         self.walk, self.route, self.dtype, self.table = walk, route, dtype, table
+        self.tag = _hip.MA_BF16 if dtype == torch.bfloat16 else _hip.MA_F32
         self.params = [e.p for e in table.entries]
         self.states = [e.st for e in table.entries]
-        self.spans, at = [], 0
-        for group, plist, _ in walk:
-            self.spans.append((group, slice(at, at + len(plist))))
-            at += len(plist)
 
     def refresh(self, default_wd):
         """Writes this step's buffers and hyper-parameters into the table; False, with nothing
         that matters changed, if some tensor's buffers do not admit the table's route this time
         (the conditions of the general walk, tensor by tensor)."""
-        n, params = len(self.params), self.params
-        for (group, span), (_, plist, _) in zip(self.spans, self.walk):
-            if not all(map(operator.is_, plist, params[span])):
-                return False
-        try:
-            grads = list(map(_grad_of, params))
-            dtypes = set(map(_dtype_of, grads))  # (a gradient that is None has no dtype)
-        except AttributeError:
-            return False
-        dtypes.update(map(_dtype_of, params))
-        if len(dtypes) != 1 or self.dtype not in dtypes:
-            return False
-        if set(map(_dtype_of, map(_index_column, self.states))) != {torch.int16}:
-            return False
-        if not (all(map(_is_contiguous, grads)) and all(map(_is_contiguous, params))):
-            return False
-        p = np.fromiter(map(_address_of, params), np.uint64, n)
-        g = np.fromiter(map(_address_of, grads), np.uint64, n)
-        if int(np.bitwise_or.reduce(p | g)) & 15:
-            return False
-        view = self.table.view
-        view['p'], view['g'] = p, g
-        view['index'] = list(map(_row_of, self.states))
-        for group, span in self.spans:
-            view['lr'][span] = group['lr']
-            view['weight_decay'][span] = group.get('weight_decay', default_wd)
-        return True
+        groups = [(plist, group['lr'], group.get('weight_decay', default_wd))
+                  for group, plist, _ in self.walk]
+        return _step_table.refresh(self.table.address, self.params, self.states, groups, self.tag)
 
 
 class _Entry:
@@ -370,8 +335,9 @@ class MicroAdam(torch.optim.Optimizer):
 
         started = time.time()
         logging_step = self._logging_active() and self.steps % self.log_interval == 0
-        # One table for all tensors, as in the last step: 47.7 -> 32.5 us of host time for 30 tensors,
-        # 150 -> 80 for 148 (the walk costs a Python iteration with all its checks per tensor)
+        # One table for all tensors, as in the last step (the walk costs a Python iteration with all
+        # its checks per tensor: 48 us of host time for 30 tensors, 150 for 148; in columns through
+        # the interpreter 33 and 79, natively 16 and 23, of which torch's wrapper of step() is 7)
         walk, same = self._groups(), self._uniform
         if (same is not None and same.walk is walk and self.use_fused and not logging_step
                 and same.refresh(self.weight_decay)):
@@ -500,9 +466,7 @@ class MicroAdam(torch.optim.Optimizer):
             rc = _hip.lib.ma_spanning_step(table.records, n, ctypes.byref(h), alpha, ws_ptr,
                                            ws_len, stream)
             _hip.check(rc, "ma_spanning_step")
-        m = self.m
-        for st in states:  # micro_adam.py:211
-            st['index'] = (st['index'] + 1) % m
+        _step_table.advance(states, self.m)
 
     # ------------------------------------------------------------------ op-by-op route (micro_adam.py:146-328)
     @torch.no_grad()

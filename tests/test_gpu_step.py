@@ -1107,3 +1107,61 @@ def test_spanning_route_takes_what_the_op_by_op_route_takes(dtype, value):
                       ("error", "min_vals", "max_vals")])
     for got, want in zip(*states):
         assert np.array_equal(got.numpy(), want.numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("change", ["nothing", "gradient missing", "gradient strided",
+                                    "gradient unaligned", "parameter replaced", "learning rates",
+                                    "no weight decay", "odd kinds of numbers", "state retyped"])
+def test_table_refresh_takes_what_the_walk_takes(change):
+    """A list that goes through one table, refreshed natively, against the walk over its tensors:
+    the same parameters and states whatever one of the steps brings."""
+    from ista_daslab_optimizers import MicroAdam
+    results = []
+    for walked in (False, True):
+        gen = torch.Generator().manual_seed(11)
+        shapes = [(64, 40), (300,), (128, 96)]
+        params = [torch.nn.Parameter((torch.randn(s, generator=gen) * 0.02).bfloat16().cuda())
+                  for s in shapes]
+        other = torch.nn.Parameter((torch.randn(shapes[1], generator=gen) * 0.02).bfloat16().cuda())
+        opt = MicroAdam([{"params": params[:2]}, {"params": params[2:], "lr": 3e-4}], m=3, lr=1e-3,
+                        quant_block_size=64, weight_decay=0.01)
+        for step in range(5):
+            for group in opt.param_groups:
+                for p in group["params"]:
+                    p.grad = (torch.randn(p.shape, generator=gen) * 0.01).bfloat16().cuda()
+            if step == 3:
+                p = params[2]
+                if change == "gradient missing":
+                    p.grad = None
+                elif change == "gradient strided":
+                    p.grad = p.grad.t().contiguous().t()
+                elif change == "gradient unaligned":
+                    flat = torch.empty(p.numel() + 1, dtype=p.dtype, device="cuda")
+                    p.grad = flat[1:].view(p.shape).copy_(p.grad)
+                elif change == "parameter replaced":
+                    opt.param_groups[0]["params"][1] = other
+                    other.grad = params[1].grad
+                elif change == "learning rates":
+                    opt.param_groups[0]["lr"], opt.param_groups[1]["lr"] = 5e-3, 0
+                elif change == "no weight decay":
+                    opt.param_groups[1]["weight_decay"] = 0
+                    del opt.param_groups[0]["weight_decay"]
+                elif change == "odd kinds of numbers":
+                    opt.param_groups[0]["lr"] = np.float64(2e-3)
+                    opt.param_groups[1]["lr"] = torch.tensor(2e-3)
+                elif change == "state retyped":
+                    st = opt.state[params[0]]
+                    st["I"] = st["I"].to(torch.bfloat16)
+            if walked:
+                opt._uniform = None
+            if change == "gradient strided" and step == 3:
+                with pytest.raises(RuntimeError, match="view size"):  # neither takes it
+                    opt.step()
+                break
+            opt.step()
+        results.append([p.data.float().cpu() for p in params + [other]] +
+                       [opt.state[p][key].float().cpu() for p in params
+                        for key in ("error", "min_vals", "max_vals", "I", "V")] +
+                       [opt.state[p]["index"] for p in params])
+    for got, want in zip(*results):
+        assert torch.equal(got, want) if torch.is_tensor(got) else got == want
