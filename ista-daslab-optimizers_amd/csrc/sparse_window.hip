@@ -72,6 +72,12 @@ struct __attribute__((packed, aligned(2))) IndexQuad {
             uint32_t, __builtin_elementwise_max(__builtin_elementwise_max(t, a), b));
     }
 };
+// two 16-bit numbers, each at most the one in `most`
+__device__ __forceinline__ uint32_t both_at_most(uint32_t w, uint32_t most) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, w), __builtin_bit_cast(u16x2, most)));
+}
 template <typename TV>
 struct ValueQuad;
 template <>
@@ -344,9 +350,15 @@ __global__ __launch_bounds__(kWG) void sparse_dot_reduce_kernel(const float *par
 // atomics.  The accumulators fill the LDS (two 20480-element blocks per CU), so what bounds the
 // kernel is the chain of rows.  ONE wave applies all rows of a block: the LDS operations of a wave
 // execute in program order, so a row needs no barrier behind it, only its own reads; the next
-// row's addresses and terms are formed while those are under way.  The window comes in through a
-// ring of registers, four entries a request.
+// row's addresses and terms are formed, and a row's next request is made, while those are under
+// way.  The window comes in through a ring of registers, four entries a request.  25.6 M coordinates,
+// 1024 rows of 1 %, bf16: 360 us with the requests behind every fourth row and a check of its
+// indices there, 332 in rounds of 32 rows without a branch.  With the LDS left out it still takes
+// 300: what is left is one wave's issue of some 35 instructions a row, 230 cycles.  (LDS float
+// atomics: 193 cycles a wave instruction, where a read and a write of four bytes take 12.)
 typedef __attribute__((address_space(3))) float LdsFloat;
+// read only, at addresses that are the same in all lanes: scalar loads
+typedef __attribute__((address_space(4))) float ConstantFloat;
 
 // LDS address of cell `half` (16 bits) of w: one instruction, as the kernel's dynamic LDS, which
 // the accumulators begin, is all the LDS it has and so begins at address 0
@@ -366,9 +378,9 @@ template <typename TV, int G, int RING, bool LONG>
 __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int64_t k, int m_rows,
                                              const float *coef, const int16_t *I, const TV *V,
                                              int lane) {
-    static_assert(RING <= 64, "a lane holds one coefficient of the ring");
-    constexpr int kStep = 4;  // rows whose indices are checked together
     constexpr uint32_t kWide = sizeof(TV) / 2;
+    constexpr int kStep = 4;  // rows taken together behind the last whole round
+    static_assert(RING % kStep == 0, "the ring in groups of kStep rows");
     // byte offset in a row of the indices of this lane's entries
     uint32_t start[G];
 #pragma unroll
@@ -415,13 +427,18 @@ __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int
     float term[2][G][4];
     uint32_t two = 2;
     asm volatile("" : "+v"(two));
+    uint32_t top = 0;                                         // both halves: largest index so far
+    const uint32_t last = (uint32_t)(S.len - 1) * 0x10001u;  // both halves: largest of the block
     auto prepare = [&](int which, int slot, float c) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            cell[which][g][0] = cell_address<0>(ix[slot][g].w[0], two);
-            cell[which][g][1] = cell_address<1>(ix[slot][g].w[0], two);
-            cell[which][g][2] = cell_address<0>(ix[slot][g].w[1], two);
-            cell[which][g][3] = cell_address<1>(ix[slot][g].w[1], two);
+            top = ix[slot][g].largest(top);
+            const uint32_t w0 = both_at_most(ix[slot][g].w[0], last);
+            const uint32_t w1 = both_at_most(ix[slot][g].w[1], last);
+            cell[which][g][0] = cell_address<0>(w0, two);
+            cell[which][g][1] = cell_address<1>(w0, two);
+            cell[which][g][2] = cell_address<0>(w1, two);
+            cell[which][g][3] = cell_address<1>(w1, two);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 term[which][g][e] = c * v[slot][g].value(e);
@@ -449,69 +466,67 @@ __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int
 #pragma unroll
             for (int e = 0; e < 4; ++e) *(LdsFloat *)(uintptr_t)cell[which][g][e] = x[g][e];
     };
-    // (the first round only requests: a request is made at one place of the code, in one order,
-    // whatever the round)
+    aim(0);
 #pragma unroll
-    for (int u = 0; u < RING; ++u)
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            ix[u][g] = IndexQuad{};
-            v[u][g] = ValueQuad<TV>{};
-        }
-    float next_coef = 0.0f;
-    for (int r0 = -RING; r0 < m_rows; r0 += RING) {
-        const float cs = next_coef;
-        next_coef = coef[r0 + RING + lane < m_rows ? r0 + RING + lane : m_rows - 1];
+    for (int u = 0; u < RING; ++u) {
+        request(u);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // Rounds of RING rows without a branch: whether an index lay outside the block is asked once,
+    // at the end (a branch to another way of taking a row joins this one again, and there the
+    // compiler waits for the whole ring).
+    int r0 = 0;
+    for (; r0 + RING <= m_rows; r0 += RING) {
+        const ConstantFloat *cr = (const ConstantFloat *)(uintptr_t)(coef + r0);
         aim(r0 + RING);
         __builtin_amdgcn_sched_barrier(0);
+        prepare(0, 0, cr[0]);
 #pragma unroll
-        for (int s0 = 0; s0 < RING; s0 += kStep) {
-            const int row = r0 + s0;
-            uint32_t top = 0;
+        for (int u = 0; u < RING; ++u) {
+            read(u & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (u + 1 < RING) prepare((u + 1) & 1, u + 1, cr[u + 1]);
+            // (the row's slot is free: its next request goes out behind the reads too)
+            request(u);
+            __builtin_amdgcn_sched_barrier(0);
+            add_write(u & 1);
+        }
+    }
+    // the window's last rows, fewer than the ring holds
+    const ConstantFloat *cr = (const ConstantFloat *)(uintptr_t)(coef + r0);
 #pragma unroll
-            for (int u = 0; u < kStep; ++u)
-#pragma unroll
-                for (int g = 0; g < G; ++g) top = ix[s0 + u][g].largest(top);
-            const bool stray =
-                (top & 0xffffu) >= (uint32_t)S.len || (top >> 16) >= (uint32_t)S.len;
-            const bool in_block = __builtin_amdgcn_ballot_w64(stray) == 0;
-            auto coef_of = [&](int u) {
-                return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), s0 + u));
-            };
-            if (r0 >= 0 && in_block && row + kStep <= m_rows) {
-                prepare(0, s0, coef_of(0));
-#pragma unroll
-                for (int u = 0; u < kStep; ++u) {
-                    read(u & 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (u + 1 < kStep) prepare((u + 1) & 1, s0 + u + 1, coef_of(u + 1));
-                    __builtin_amdgcn_sched_barrier(0);
-                    add_write(u & 1);
-                }
-            } else if (r0 >= 0 && in_block) {  // the window's last rows
-#pragma unroll
-                for (int u = 0; u < kStep - 1; ++u) {
-                    if (row + u < m_rows) {
-                        prepare(0, s0 + u, coef_of(u));
-                        read(0);
-                        add_write(0);
-                    }
-                }
-            } else if (r0 >= 0) {
-                // an index outside the block, which is skipped: these rows entry by entry
-                for (int r = row; r < row + kStep && r < m_rows; ++r) {
-                    const int64_t first = (int64_t)r * k + S.col0;
-                    for (int j = lane; j < S.kb; j += 64) {
-                        const int i = I[first + j];
-                        const float t = coef[r] * widen(V[first + j]);
-                        if ((unsigned)i < (unsigned)S.len) acc[i] = acc[i] + t;
-                    }
-                }
-            }
+    for (int u0 = 0; u0 < RING; u0 += kStep) {
+        if (r0 + u0 + kStep <= m_rows) {
+            prepare(0, u0, cr[u0]);
 #pragma unroll
             for (int u = 0; u < kStep; ++u) {
-                request(s0 + u);
+                read(u & 1);
                 __builtin_amdgcn_sched_barrier(0);
+                if (u + 1 < kStep) prepare((u + 1) & 1, u0 + u + 1, cr[u0 + u + 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                add_write(u & 1);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kStep - 1; ++u) {
+                if (r0 + u0 + u < m_rows) {
+                    prepare(0, u0 + u, cr[u0 + u]);
+                    read(0);
+                    add_write(0);
+                }
+            }
+        }
+    }
+    const bool stray = (top & 0xffffu) >= (uint32_t)S.len || (top >> 16) >= (uint32_t)S.len;
+    if (__builtin_amdgcn_ballot_w64(stray) != 0) {
+        // an index outside the block, which contributes nothing: all over again, entry by entry
+        for (int i = lane; i < S.len; i += 64) acc[i] = 0.0f;
+        for (int r = 0; r < m_rows; ++r) {
+            const int64_t first = (int64_t)r * k + S.col0;
+            for (int j = lane; j < S.kb; j += 64) {
+                const int i = I[first + j];
+                const float t = coef[r] * widen(V[first + j]);
+                if ((unsigned)i < (unsigned)S.len) acc[i] = acc[i] + t;
             }
         }
     }
@@ -520,7 +535,7 @@ __device__ __forceinline__ void combine_rows(float *acc, const BlockSpan &S, int
 // The same for rows of one to three entries: a lane holds one of them, the lanes behind the last
 // one hold it too and write the same sum.  A last block of at most 300 coordinates has such rows
 // at 1 %; it must not take longer than the others (one dependent trip to memory per row: 706 us
-// for 1249 blocks that take 362 so).
+// for 1249 blocks that took 362 so).
 template <typename TV, int RING>
 __device__ __forceinline__ void combine_short_rows(float *acc, const BlockSpan &S, int64_t k,
                                                    int m_rows, const float *coef,
@@ -725,7 +740,7 @@ int ma_sparse_linear_combination(int64_t d, int64_t m_rows, int64_t k, int64_t d
     if (lds > kLdsBytes) return MA_ERR_LDS;
     hipStream_t s = (hipStream_t)stream;
     // Rows of up to 512 entries per block: one wave applies them, against four waves (eight above
-    // 256 entries) and a barrier per row: 1248 blocks of 20480, 1024 rows of 205 bf16: 362 us, 598;
+    // 256 entries) and a barrier per row: 1248 blocks of 20480, 1024 rows of 205 bf16: 332 us, 598;
     // 512 rows of 410: 318, 381; of 512: 317, 395.  Longer rows give a barrier more to do.
     // Rows of more than 2^25 entries do not fit a round's 32-bit offsets; addressed row by row
     // the 1024 rows of 205 take 387 us.  Small blocks, of which the LDS would hold more than two,
