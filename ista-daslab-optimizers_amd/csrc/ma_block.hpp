@@ -3301,8 +3301,22 @@ static int launch_fused_apart(int C, unsigned grid, int lds_bytes, hipStream_t s
 
 template <class R>
 static int launch_window_param(unsigned grid, int lds_bytes, hipStream_t s, const FusedParams &P) {
-    if (grid == 0) return allow_big_lds(window_param_kernel<R, kWavesThreeWG>, lds_bytes);
-    return launch_kernel(window_param_kernel<R, kWavesThreeWG>, dim3(grid), kWG, lds_bytes, s, P);
+    // bf16: in 64 registers the four workgroups whose LDS fits a CU are resident; with the 66 the
+    // compiler takes by itself there are three.  0.7 G parameters, 20 rows of 5 %, the whole step:
+    // 2.52 ms with three and 2.37 with four.  A launch that three a CU hold at once gains nothing
+    // and pays for the spills (1 M parameters 65.8 and 67.0 us).  fp32 data spills more in 64.
+    constexpr int kAll = 4 * kWG / 256, kUsual = kWavesThreeWG;
+    constexpr unsigned kResident = 3 * 256;
+    if constexpr (R::kBF16) {
+        if (grid == 0) {
+            const int rc = allow_big_lds(window_param_kernel<R, kAll>, lds_bytes);
+            if (rc) return rc;
+        }
+        if (grid > kResident)
+            return launch_kernel(window_param_kernel<R, kAll>, dim3(grid), kWG, lds_bytes, s, P);
+    }
+    if (grid == 0) return allow_big_lds(window_param_kernel<R, kUsual>, lds_bytes);
+    return launch_kernel(window_param_kernel<R, kUsual>, dim3(grid), kWG, lds_bytes, s, P);
 }
 
 template <template <int> class RT>
