@@ -213,6 +213,7 @@ struct RawChunk<RegsF32<C>> {
 // entry e to thread e % kWG, and requested at the start of the block.
 constexpr int kEnt = 5;        // entries per thread at most
 constexpr int kFastRows = 16;  // window rows at most: a coordinate's rows are a 16-bit mask
+constexpr int kLongQueue = 768;  // entries of shared coordinates window_long has room for, 14 bytes each
 
 // Where one top-k block lives: everything a stage needs to address it, copied out of the
 // launch parameters.  Wave-uniform (lives in scalar registers).
@@ -541,7 +542,8 @@ struct FusedBlock {
         const int kb = G.kb;
         bool topk_done = false;
         if constexpr (FULL && R::kBF16) {
-            if (kb <= kWG) {
+            // (not where window_param_kernel takes the window: it wants rows by coordinate)
+            if (kb <= kWG && P.win_apart == 0) {
                 topk_done = hint_topk_bf16(r, kb, hint, cell16, hist, sh, sel_idx, sel_val);
                 if (!topk_done)
                     topk_done = fast_topk_bf16(r, kb, cell16, hist, sh, sel_idx, sel_val);
@@ -558,9 +560,12 @@ struct FusedBlock {
         }
         row_sorted = !topk_done;  // the selections below list their entries by coordinate
         if constexpr (FULL && R::kBF16) {
-            // block rows too long for the candidate lists, where the LDS plan has the cells to
-            // park the block in: threshold and ordered selection from the hint
-            if (kb > kWG && kb <= kHintLongRow && P.L.cell_bytes == 2 &&
+            // block rows too long for the candidate lists, and all that window_param_kernel takes,
+            // where the LDS plan has the cells to park the block in: threshold and ordered
+            // selection from the hint.  (Rows of up to 512 entries as hint_topk_bf16 lists them
+            // sent window_param_kernel through its general form, a barrier a row: 119 M
+            // parameters, 16 rows of 2 %, 590 us a step; 398 so)
+            if ((kb > kWG || P.win_apart != 0) && kb <= kHintLongRow && P.L.cell_bytes == 2 &&
                 P.L.slot_cells >= C * kRound) {
                 topk_done = hint_sorted_topk_bf16(r, kb, hint, cell16, hist, sh, sel_idx, sel_val);
                 launder(r);
@@ -813,39 +818,234 @@ struct FusedBlock {
     }
 
     __device__ __forceinline__ void load_window_wide(const BlockGeo &G) {
+        load_quad(G, tid, wI, wV, w_first, w_row);
+    }
+
+    // the four entries of number t, see wI
+    __device__ __forceinline__ void load_quad(const BlockGeo &G, int t, uint32_t (&qI)[2],
+                                              uint32_t (&qV)[2], int &first, int &of_row) const {
         struct __attribute__((aligned(4))) Pair32 {
             uint32_t x, y;
         };
         const int W = G.kb / 4 + 1;
         const int older = older_rows(G);
-        const int ro = (int)(((float)tid + 0.5f) * __builtin_amdgcn_rcpf((float)W));
-        const int w = tid - ro * W;
-        w_row = -1;
-        w_first = 0;
-        wI[0] = wI[1] = wV[0] = wV[1] = 0;
+        const int ro = (int)(((float)t + 0.5f) * __builtin_amdgcn_rcpf((float)W));
+        const int w = t - ro * W;
+        of_row = -1;
+        first = 0;
+        qI[0] = qI[1] = qV[0] = qV[1] = 0;
         if (ro < older) {
             const int row = (ro < G.D.row || G.D.row >= P.W.rows) ? ro : ro + 1;
             const int64_t e_first = (int64_t)row * G.D.k + G.col0;
             const int a = (int)(e_first & 1);
             const int64_t e_base = e_first - a + 4 * w;
-            w_first = 4 * w - a;
-            w_row = row;
+            first = 4 * w - a;
+            of_row = row;
             const uint16_t *Ip = reinterpret_cast<const uint16_t *>(G.D.I) + e_base;
             const uint16_t *Vp = G.D.V + e_base;
             if (e_base + 4 <= (int64_t)P.W.rows_total * G.D.k) {
                 const Pair32 qi = *reinterpret_cast<const Pair32 *>(Ip);
                 const Pair32 qv = *reinterpret_cast<const Pair32 *>(Vp);
-                wI[0] = qi.x; wI[1] = qi.y; wV[0] = qv.x; wV[1] = qv.y;
+                qI[0] = qi.x; qI[1] = qi.y; qV[0] = qv.x; qV[1] = qv.y;
             } else {  // the last load of the last row may not reach past the arrays
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     if (e_base + j < (int64_t)P.W.rows_total * G.D.k) {
-                        wI[j >> 1] |= (uint32_t)Ip[j] << (16 * (j & 1));
-                        wV[j >> 1] |= (uint32_t)Vp[j] << (16 * (j & 1));
+                        qI[j >> 1] |= (uint32_t)Ip[j] << (16 * (j & 1));
+                        qV[j >> 1] |= (uint32_t)Vp[j] << (16 * (j & 1));
                     }
                 }
             }
         }
+    }
+
+    // =========================================================================================
+    // Window and parameter stage of bf16 blocks, full or not, whose window is too long for the
+    // stage below but has at most two loads of four older entries a thread (15 rows of 1 %, 10 rows
+    // of 2 %).  The steps are those of update_wide_bf16; but the updates go to the coordinate
+    // cells as they are formed, so that nothing is held per entry (a coordinate that one row names
+    // has one reader of its cell, which may overwrite it), the dense parameter stage takes them from
+    // there, and the queue of entries that share coordinates holds as many as the LDS of three
+    // workgroups per CU leaves room for; more of them are taken in turns.
+    // =========================================================================================
+    uint32_t w2I[2], w2V[2];  // the second four entries of a thread
+    int w2_first, w2_row;
+    bool longer;              // this block takes the stage
+
+    __device__ __forceinline__ void load_window_long(const BlockGeo &G) {
+        const int W = G.kb / 4 + 1;
+        longer = row_in_lds && (((uintptr_t)G.D.I | (uintptr_t)G.D.V) & 3) == 0 &&
+                 older_rows(G) * W <= 2 * kWG && G.kb <= kWG && P.W.rows <= 15 &&
+                 P.L.total - P.L.off_union >= kLongQueue * 14;
+        if (longer) {
+            load_quad(G, tid, wI, wV, w_first, w_row);
+            load_quad(G, tid + kWG, w2I, w2V, w2_first, w2_row);
+        }
+    }
+
+    __device__ __forceinline__ void update_long(const BlockGeo &G) {
+        if (!longer || !window_long(G)) {
+            slot_clear = false;
+            window_stage(G);
+        }
+        param_stage(G);
+    }
+
+    // The slot cells end up holding the update's bits.  False, for every thread, if the entries that
+    // share coordinates do not fit the queue in turns either (window_stage then starts afresh).
+    // Ends with a barrier.
+    __device__ __forceinline__ bool window_long(const BlockGeo &G) {
+        const int n = FULL ? C * kRound : G.n;
+        constexpr int kSlots = 9;  // eight entries of older rows, one of this step's row
+        const TensorDesc &D = G.D;
+        const int kb = G.kb;
+        uint32_t *lcount = sh + kShLinks, *qcount = sh + kShCounter;
+        uint32_t *qkey = hist;
+        float *qa1 = reinterpret_cast<float *>(hist + kLongQueue), *qa2 = qa1 + kLongQueue;
+        if (!slot_clear) {
+            __syncthreads();  // the LDS of the selection is reused below
+            for (int i = tid; i < (n + 7) / 8; i += kWG)
+                reinterpret_cast<uint4 *>(cell16)[i] = make_uint4(0, 0, 0, 0);
+        }
+        if (tid < kFastRows) {
+            sh[kShW1 + tid] = __float_as_uint(P.W.w1[tid]);
+            sh[kShW2 + tid] = __float_as_uint(P.W.w2[tid]);
+        }
+        if (tid == 0) *lcount = *qcount = 0;
+        __syncthreads();
+        // entry j of this thread: index and value (bf16 bits); false: none, or nothing to add (+-0
+        // values are skipped; idx < n keeps a corrupt index inside)
+        auto entry = [&](int j, uint32_t &idx, uint32_t &vb) {
+            bool have;
+            if (j < 4) {
+                idx = (wI[(j >> 1) & 1] >> (16 * (j & 1))) & 0xffffu;
+                vb = (wV[(j >> 1) & 1] >> (16 * (j & 1))) & 0xffffu;
+                have = w_row >= 0 && (unsigned)(w_first + j) < (unsigned)kb;
+            } else if (j < 8) {
+                idx = (w2I[(j >> 1) & 1] >> (16 * (j & 1))) & 0xffffu;
+                vb = (w2V[(j >> 1) & 1] >> (16 * (j & 1))) & 0xffffu;
+                have = w2_row >= 0 && (unsigned)(w2_first + j - 4) < (unsigned)kb;
+            } else {
+                have = tid < kb && D.row < P.W.rows;
+                idx = have ? sel_idx[tid] : 0u;
+                vb = have ? sel_val[tid] : 0u;
+            }
+            return have && idx < (uint32_t)n && (vb & 0x7fffu) != 0;
+        };
+        // ---- every entry marks its row in the cell of its coordinate
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) {
+            uint32_t idx, vb;
+            const int row = j < 4 ? w_row : j < 8 ? w2_row : D.row;
+            if (entry(j, idx, vb)) atomicOr(cell32 + (idx >> 1), (1u << row) << ((idx & 1u) * 16));
+        }
+        __syncthreads();
+        // ---- a coordinate named by one row has its update from that entry; the entries of the
+        //      others queue up with their rank among the coordinate's rows
+        auto take = [&](int j, bool singles, uint32_t &shared) {
+            uint32_t idx, vb;
+            const uint32_t row = (uint32_t)(j < 4 ? w_row : j < 8 ? w2_row : D.row);
+            if (!entry(j, idx, vb)) return;
+            const uint32_t mask = cell16[idx];
+            const float v = bf2f(vb);
+            const float vv = v * v;
+            const float a1 = __uint_as_float(sh[kShW1 + row]) * v;
+            const float a2 = __uint_as_float(sh[kShW2 + row]) * vv;
+            if (singles && mask == 1u << row) {
+                const float u =
+                    adam_update<R::kBF16>(0.0f + a1, 0.0f + a2, P.W.s1, P.W.s2, P.W.eps);
+                cell16[idx] = (uint16_t)f2bf(u);
+                return;
+            }
+            shared |= 1u << j;
+            const uint32_t at = atomicAdd(qcount, 1u);
+            if (at < (uint32_t)kLongQueue) {
+                const uint32_t rank = (uint32_t)__popc(mask & ((1u << row) - 1u));
+                qkey[at] = idx | rank << 15 | (uint32_t)__popc(mask) << 19;
+                qa1[at] = a1;
+                qa2[at] = a2;
+            }
+        };
+        uint32_t shared = 0;  // bit j: entry j shares its coordinate
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j) take(j, true, shared);
+        __syncthreads();
+        const uint32_t queued = *qcount;
+        if (queued <= (uint32_t)kLongQueue) {
+            settle_queue(queued);
+            return true;
+        }
+        // Too many for one queue (gradients whose large coordinates persist: in a block that holds
+        // a row of outliers every entry shares its coordinate): the coordinates are taken in 2, 4, ...
+        // turns by their lowest bits.  The marks of a coordinate stay until its turn.
+        uint32_t turns = 2;
+        while (turns * 512u < queued) turns <<= 1;
+#pragma unroll 1
+        for (uint32_t turn = 0; turn < turns; ++turn) {
+            __syncthreads();
+            if (tid == 0) *lcount = *qcount = 0;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kSlots; ++j) {
+                uint32_t idx, vb;
+                uint32_t unused = 0;
+                if (((shared >> j) & 1u) != 0 && entry(j, idx, vb) && (idx & (turns - 1u)) == turn)
+                    take(j, false, unused);
+            }
+            __syncthreads();
+            const uint32_t now = *qcount;
+            if (now > (uint32_t)kLongQueue) return false;
+            settle_queue(now);
+        }
+        return true;
+    }
+
+    // The queued coordinates' updates to their cells, as in update_wide_bf16, with up to two queued
+    // entries a thread.  Ends with a barrier.
+    __device__ __forceinline__ void settle_queue(uint32_t queued) {
+        uint32_t *lcount = sh + kShLinks;
+        const uint32_t *qkey = hist;
+        const float *qa1 = reinterpret_cast<const float *>(hist + kLongQueue), *qa2 = qa1 + kLongQueue;
+        uint16_t *link = reinterpret_cast<uint16_t *>(hist + 3 * kLongQueue);
+        constexpr int kMine = (kLongQueue + kWG - 1) / kWG;
+        uint32_t key[kMine], base[kMine];
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            const uint32_t t = (uint32_t)(tid + i * kWG);
+            key[i] = 0xffffffffu;
+            base[i] = 0;
+            if (t < queued) {
+                key[i] = qkey[t];
+                if (((key[i] >> 15) & 15u) == 0)
+                    cell16[key[i] & 0x7fffu] = (uint16_t)atomicAdd(lcount, key[i] >> 19);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            if (key[i] != 0xffffffffu) {
+                base[i] = cell16[key[i] & 0x7fffu];
+                const uint32_t at = min(base[i] + ((key[i] >> 15) & 15u), (uint32_t)kLongQueue - 1u);
+                link[at] = (uint16_t)(tid + i * kWG);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            if (key[i] != 0xffffffffu && ((key[i] >> 15) & 15u) == 0) {
+                const int terms = (int)(key[i] >> 19);
+                float s1 = 0.0f, s2 = 0.0f;
+                for (int r = 0; r < terms; ++r) {
+                    const uint32_t at = min(base[i] + (uint32_t)r, (uint32_t)kLongQueue - 1u);
+                    const uint32_t q = min((uint32_t)link[at], (uint32_t)kLongQueue - 1u);
+                    s1 = s1 + qa1[q];
+                    s2 = s2 + qa2[q];
+                }
+                const float u = adam_update<R::kBF16>(s1, s2, P.W.s1, P.W.s2, P.W.eps);
+                cell16[key[i] & 0x7fffu] = (uint16_t)f2bf(u);
+            }
+        }
+        __syncthreads();
     }
 
     __device__ __forceinline__ void update_wide(const BlockGeo &G) {
@@ -2692,7 +2892,8 @@ __device__ __forceinline__ int find_tensor(const FusedParams &P, int w) {
 //   WIN: what becomes of the window and the parameters.  kWinFused: everything in this kernel.
 //        kWinApart: nothing; the kernel ends with the quantisation, and window_param_kernel,
 //        launched behind it, forms the update and steps the parameters.
-constexpr int kWinFused = 0, kWinApart = 2;
+//        kWinLong: as kWinFused, by update_long (bf16 data).
+constexpr int kWinFused = 0, kWinLong = 1, kWinApart = 2;
 
 template <class R, int MIN_WAVES, int QL, bool DENSE = false, int WIN = kWinFused, int AUX = 0>
 __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams P) {
@@ -2735,9 +2936,14 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void fused_step_kernel(FusedParams 
         } else {
             // parameters and window entries are asked for before the quantisation, which
             // hides their latency (the selection runs with more registers free without them)
-            if constexpr (WIN != kWinApart) fb.load_params_window(G);
+            if constexpr (WIN == kWinFused) fb.load_params_window(G);
+            if constexpr (WIN == kWinLong) {
+                fb.load_params(G);
+                fb.load_window_long(G);
+            }
             fb.quantize(G);
-            if constexpr (WIN != kWinApart) fb.update(G);
+            if constexpr (WIN == kWinFused) fb.update(G);
+            if constexpr (WIN == kWinLong) fb.update_long(G);
         }
         fb.log_flush(item, 0xffu);
     };
@@ -3299,6 +3505,23 @@ static int launch_fused_apart(int C, unsigned grid, int lds_bytes, hipStream_t s
     return MA_ERR_BLOCK_SIZE;
 }
 
+// the block kernels with the longer one-pass window stage
+template <template <int> class RT>
+static int launch_fused_long(int C, unsigned grid, int lds_bytes, hipStream_t s,
+                             const FusedParams &P) {
+    if (C == kClass2 && P.q_shift == 6)
+        return launch_fused_one<RT<kClass2>, 8, false, kWinLong>(grid, lds_bytes, s, P);
+    if (C == kClass2 && P.q_shift == 5)
+        return launch_fused_one<RT<kClass2>, 4, false, kWinLong>(grid, lds_bytes, s, P);
+    switch (C) {
+        case kClass0: return launch_fused_one<RT<kClass0>, 0, false, kWinLong>(grid, lds_bytes, s, P);
+        case kClass1: return launch_fused_one<RT<kClass1>, 0, false, kWinLong>(grid, lds_bytes, s, P);
+        case kClass2: return launch_fused_one<RT<kClass2>, 0, false, kWinLong>(grid, lds_bytes, s, P);
+        case kClass3: return launch_fused_one<RT<kClass3>, 0, false, kWinLong>(grid, lds_bytes, s, P);
+    }
+    return MA_ERR_BLOCK_SIZE;
+}
+
 template <class R>
 static int launch_window_param(unsigned grid, int lds_bytes, hipStream_t s, const FusedParams &P) {
     // bf16: in 64 registers the four workgroups whose LDS fits a CU are resident; with the 66 the
@@ -3383,6 +3606,8 @@ int launch_fused_f32(int C, unsigned grid, int lds_bytes, hipStream_t s, const F
 int launch_fused_apart_bf16(int C, unsigned grid, int lds_bytes, hipStream_t s,
                             const FusedParams &P);
 int launch_fused_apart_f32(int C, unsigned grid, int lds_bytes, hipStream_t s,
+                           const FusedParams &P);
+int launch_fused_long_bf16(int C, unsigned grid, int lds_bytes, hipStream_t s,
                            const FusedParams &P);
 int launch_window_param_bf16(unsigned grid, int lds_bytes, hipStream_t s, const FusedParams &P);
 int launch_window_param_f32(unsigned grid, int lds_bytes, hipStream_t s, const FusedParams &P);

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kWG) void window_update_kernel(int64_t d, int dbs, 
 // =============================================================================================
 
 
-static inline int align16(int x) { return (x + 15) & ~15; }
+static constexpr int align16(int x) { return (x + 15) & ~15; }
 
 // LDS plan for a block kernel: longest block `dbs_max`, most entries per block row `kb_max`,
 // window length m, bytes per element of the data.
@@ -382,23 +382,45 @@ static LdsMap plan_lds_select_only(int dbs_max, int kb_max, int elem_bytes) {
     L.off_slot = L.off_sel_val + align16(kb_max * 2);
     L.slot_cells = (dbs_max + 7) & ~7;
     L.cell_bytes = 2;
-    if (kb_max <= kWG) {
-        L.off_union = L.off_slot + align16(L.slot_cells * 2);
-        L.hist_log2 = 5;
-        L.total = L.off_union + kHistBytes;
-    } else if (elem_bytes == 2 && kb_max <= kHintLongRow) {
-        // the hinted ordered selection parks the block too; the general selection, which is
+    if (elem_bytes == 2 && kb_max <= kHintLongRow) {
+        // the hinted ordered selection parks the block; the general selection, which is
         // then the exception, makes do with 4 copies of its histogram, and the whole stays
         // within a third of the LDS
         L.off_union = L.off_slot + align16(L.slot_cells * 2);
         L.hist_log2 = 2;
         L.total = L.off_union + ((257 << L.hist_log2) * 4);
+    } else if (kb_max <= kWG) {
+        L.off_union = L.off_slot + align16(L.slot_cells * 2);
+        L.hist_log2 = 5;
+        L.total = L.off_union + kHistBytes;
     } else {
         L.slot_cells = 0;
         L.off_union = L.off_slot;
         L.hist_log2 = 5;
         L.total = L.off_union + kHistBytes;
     }
+    return L;
+}
+
+// LDS plan of a block kernel with the longer one-pass window stage (update_long): the cells, then
+// its queue, where the selection has its lists and histograms before and the ranges of
+// window_stage have their sums.  Three workgroups per CU with rows of up to 410 entries.
+static LdsMap plan_lds_long(int dbs_max, int kb_max) {
+    LdsMap L;
+    memset(&L, 0, sizeof L);
+    L.off_sel_idx = kMiscBytes;
+    L.off_sel_val = L.off_sel_idx + align16(kb_max * 2);
+    L.off_slot = L.off_sel_val + align16(kb_max * 2);
+    L.slot_cells = (dbs_max + 7) & ~7;
+    L.cell_bytes = 2;
+    L.off_union = L.off_slot + align16(L.slot_cells * 2);
+    constexpr int kUnion = align16(kLongQueue * 14);
+    static_assert(kUnion >= kFastTopkBytes && kUnion >= kHintRegBytes, "the selections' lists");
+    L.sub_len = L.z_cap = kUnion / 8;
+    static_assert(kUnion / 8 % 8 == 0, "ranges of whole chunks");
+    L.hist_log2 = 0;
+    while ((257 << (L.hist_log2 + 1)) * 4 <= kUnion && L.hist_log2 < 5) ++L.hist_log2;
+    L.total = L.off_union + kUnion;
     return L;
 }
 
@@ -770,6 +792,22 @@ static bool window_apart(int64_t d, const ma_hyper *h, int elem_bytes) {
     return plan_lds((int)g.dbs, (int)g.k_many, h->m, elem_bytes, true, true).cell_bytes == 0;
 }
 
+// How ma_fused_step (alpha == 0, no logging) takes a tensor's window: in the one-pass stage of the
+// block kernel where it fits (up to 2560 entries a block), in the longer one-pass stage where two
+// loads of four older entries a thread hold it (bf16 data, up to 15 rows), else in a launch of
+// its own.  356 M parameters, 15 rows of 1 % (3075 entries a block):
+// 1.80 ms a step in two launches, 1.16 with the rows there by coordinate, 0.55 in the longer stage;
+// 90 M parameters whose large gradients lie in the same rows at every step: 575, 408, 348 us.
+enum { kOnePass = 0, kApart = 1, kLong = 2, kWindowForms = 3 };
+static int window_form(int64_t d, const ma_hyper *h, int elem_bytes) {
+    if (!window_apart(d, h, elem_bytes)) return kOnePass;
+    const Geometry g = geometry(d, h->d_block_size, h->k_init);
+    if (elem_bytes == 2 && h->m <= 15 && g.k_many <= kWG &&
+        (h->m - 1) * (g.k_many / 4 + 1) <= 2 * kWG)
+        return kLong;
+    return kApart;
+}
+
 // words per window row of the cache of chunk cuts, see the header
 static int64_t row_cut_words(int64_t d, const ma_hyper *h) {
     const Geometry g = geometry(d, h->d_block_size, h->k_init);
@@ -793,9 +831,9 @@ int64_t ma_fused_step_row_cuts(const ma_tensor *tensor, const ma_hyper *hyper) {
 struct PlannedLaunch {
     FusedParams P;
     int C;
-    int kind;  // kWholeStep, or the two launches that share a step: kBlockPart, kWindowPart
+    int kind;  // kWholeStep, kLongStep, or the two launches that share a step: kBlockPart, kWindowPart
 };
-enum { kWholeStep = 0, kBlockPart = 1, kWindowPart = 2 };
+enum { kWholeStep = 0, kBlockPart = 1, kWindowPart = 2, kLongStep = 3 };
 
 // Short tensors (one block of up to 4096 / 12288 elements) have kernels of their own, so that
 // they do not occupy a workgroup sized for the hardware block; but when a call holds few of
@@ -893,22 +931,22 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
     // the spanning route's workspace is handed out in the order the tensors are laid out, so the
     // slots of a launch's tensors follow each other from those of its first tensor
     int64_t ws_off = 0;
-    // tensors whose window is too large for the one-pass stage are stepped in two launches
-    // (block part, window part) of their own, whatever else the call holds: which form a tensor
-    // takes depends on its sizes alone
-    std::vector<char> apart(n_tensors, 0);
+    // tensors whose window is too large for the one-pass stage are stepped in launches of their own
+    // (the longer stage, or block part and window part), whatever else the call holds: which
+    // form a tensor takes depends on its sizes alone
+    std::vector<char> forms(n_tensors, kOnePass);
     if (!span && !dense && !aux)
         for (int i = 0; i < n_tensors; ++i)
-            apart[i] = window_apart(tensors[i].d, h, elem_bytes) ? 1 : 0;
+            forms[i] = (char)window_form(tensors[i].d, h, elem_bytes);
     std::vector<int> order;
     for (int ci = 0; ci < 4; ++ci)
-    for (int form = 0; form < 2; ++form) {
+    for (int form = 0; form < kWindowForms; ++form) {
         // the class's tensors of this form in list order, those shorter than a top-k block (one
         // partial block each: they finish early) behind the others
         order.clear();
         for (int pass = 0; pass < 2; ++pass)
             for (int i = 0; i < n_tensors; ++i) {
-                if (cls[i] != ci || apart[i] != form) continue;
+                if (cls[i] != ci || forms[i] != form) continue;
                 const bool is_short = tensors[i].d < h->d_block_size;
                 if (is_short == (pass == 1)) order.push_back(i);
             }
@@ -942,7 +980,11 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             plan.back().kind = kWholeStep;
             int rc = P.L.total > kLdsLimit ? MA_ERR_LDS : 0;
             if (segmented && P.L.total - P.L.off_union < kSegmentBytes) rc = MA_ERR_LDS;
-            if (!span && !dense && !aux && P.L.cell_bytes == 0) {
+            if (form == kLong) {
+                P.L = plan_lds_long(dbs_max, kb_max);
+                plan.back().kind = kLongStep;
+                if (P.L.total > kLdsLimit) rc = MA_ERR_LDS;
+            } else if (!span && !dense && !aux && P.L.cell_bytes == 0) {
                 // a window too large for the one-pass stage: the block kernel ends with the
                 // quantisation, a second launch over the same blocks forms the update
                 P.win_apart = 1;
@@ -994,7 +1036,7 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             D.blk0 = 0;
             D.ws = span ? reinterpret_cast<float *>(static_cast<char *>(ws) + ws_here)
                    : (aux & kAuxQuantErr) ? static_cast<float *>(t.quant_err)
-                   : apart[i] ? reinterpret_cast<float *>(t.row_cuts)
+                   : forms[i] == kApart ? reinterpret_cast<float *>(t.row_cuts)
                               : nullptr;
             items += nb;
             if (t.d < h->d_block_size) ++short_items;  // (nb == 1, and only short ones follow)
@@ -1036,6 +1078,8 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
         } else if (L.kind == kWindowPart) {
             rc = bf16 ? launch_window_param_bf16(grid, P.L.total, s, P)
                       : launch_window_param_f32(grid, P.L.total, s, P);
+        } else if (L.kind == kLongStep) {
+            rc = launch_fused_long_bf16(L.C, grid, P.L.total, s, P);
         } else if (L.kind == kBlockPart) {
             rc = bf16 ? launch_fused_apart_bf16(L.C, grid, P.L.total, s, P)
                       : launch_fused_apart_f32(L.C, grid, P.L.total, s, P);

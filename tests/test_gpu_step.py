@@ -1165,3 +1165,54 @@ def test_table_refresh_takes_what_the_walk_takes(change):
                        [opt.state[p]["index"] for p in params])
     for got, want in zip(*results):
         assert torch.equal(got, want) if torch.is_tensor(got) else got == want
+
+
+LONG_WINDOW_CASES = [
+    # windows above 2560 entries a block that the longer one-pass stage takes (bf16, up to 15 rows
+    # with two loads of four entries a thread), its last row length that fits and the first that
+    # does not; 16 rows, and rows of up to 512 entries, in the two-launch form; fp32
+    ([20480 * 2 + 17100, 20480 + 9, 18001, 4096], torch.bfloat16, 15, 64, 0.01, 0.01, 20480, 18),
+    ([20480 * 2 + 12000], torch.bfloat16, 10, 32, 0.02, 0.0, 20480, 12),
+    ([20480 * 2 + 333], torch.bfloat16, 9, 64, 0.0249, 0.0, 20480, 11),   # 510 entries, 8 * 128 loads
+    ([20480 * 2 + 333], torch.bfloat16, 10, 64, 0.022, 0.0, 20480, 12),   # 451 entries, 9 * 113
+    ([20480 * 2 + 333], torch.bfloat16, 10, 64, 0.0223, 0.0, 20480, 12),  # 457 entries, 9 * 115
+    ([20480 * 2 + 9001, 20479], torch.bfloat16, 16, 64, 0.02, 0.01, 20480, 18),
+    ([32768 + 8200], torch.bfloat16, 12, 1024, 0.01, 0.0, 32768, 14),
+    ([12288 * 2 + 4096], torch.bfloat16, 15, 128, 0.02, 0.0, 12288, 17),
+    ([20480 + 9001], torch.float32, 15, 64, 0.01, 0.01, 20480, 17),
+]
+
+
+@pytest.mark.parametrize("kind", ["normal", "one row", "ties"])
+@pytest.mark.parametrize("sizes,dtype,m,q,k_init,wd,DB,steps", LONG_WINDOW_CASES)
+def test_longer_windows(oracle, sizes, dtype, m, q, k_init, wd, DB, steps, kind):
+    """kind "one row": the first 1200 coordinates of every other block carry the large gradients
+    at every step, so that all rows of the window name them (more shared entries than the stage's
+    queue holds); "ties": gradients of few magnitudes, zeros among them."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(m)
+    cpu = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in cpu]
+    oref = oracle.OracleMicroAdam(oparams, m, 1e-3, q, k_init, 0.0, weight_decay=wd, d_block_size=DB)
+    params = [torch.nn.Parameter(p.clone().cuda()) for p in cpu]
+    opt = MicroAdam(params, m=m, lr=1e-3, quant_block_size=q, k_init=k_init, weight_decay=wd)
+    opt.d_block_size = DB
+    for step in range(steps):
+        grads = []
+        for n in sizes:
+            g = torch.randn(n, generator=gen) * 1e-2
+            at = torch.arange(n)
+            if kind == "one row":
+                g[(at % DB < 1200) & (at // DB % 2 == 0)] *= 100
+            elif kind == "ties":
+                g = torch.round(g * 200) / 200
+            grads.append(g.to(dtype))
+        for p, g in zip(params, grads):
+            p.grad = g.clone().cuda()
+        opt.step()
+        oref.step([to_np(g) for g in grads])
+        for i, p in enumerate(params):
+            assert opt._fusable(p, opt.state[p]) == 1
+            if step in (0, 1, m - 1, steps - 1):
+                assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
