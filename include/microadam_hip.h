@@ -162,8 +162,8 @@ typedef struct ma_hyper {
  * the parameters: see ma_fused_step_row_cuts.)  The
  * caller advances st['index'] (MA:211) itself.  Conditions (else MA_ERR_NOT_FUSABLE, nothing
  * launched): quant_block_size a power of two in [8, 4096] that divides d_block_size (or
- * d <= d_block_size) and does not exceed d; p and g 16-byte aligned, error 4-byte aligned;
- * d_block_size a multiple of 8 unless d <= d_block_size. */
+ * d <= d_block_size; a tensor may be shorter than a quantisation block); p and g 16-byte aligned,
+ * error 4-byte aligned; d_block_size a multiple of 8 unless d <= d_block_size. */
 int ma_fused_step(const ma_tensor *tensors /* host */, int n_tensors,
                   const ma_hyper *hyper /* host */, void *stream);
 

@@ -528,7 +528,9 @@ static int fused_check(const ma_tensor *t, const ma_hyper *h, bool dense = false
     const int64_t q = h->quant_block_size;
     (void)dense;
     if (q < 8 || q > 4096 || (q & (q - 1)) != 0) return MA_ERR_NOT_FUSABLE;
-    if (t->d < q) return MA_ERR_NOT_FUSABLE;
+    // (a tensor shorter than a quantisation block is one: its lanes past the end hold nothing.  The
+    // vectors of 80 elements among 327 tensors under q = 128, alpha = 0.25, on the spanning route
+    // beside the others: 15.6 ms a step with alpha = -2, 322 us with alpha = 0.25; here 0.13 and 0.08)
     const bool single = t->d <= h->d_block_size;
     if (!single && (g.dbs % q != 0 || g.dbs % 8 != 0)) return MA_ERR_NOT_FUSABLE;
     // the block kernels' LDS plans (with and without densification) must fit the hardware

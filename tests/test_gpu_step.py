@@ -1216,3 +1216,15 @@ def test_longer_windows(oracle, sizes, dtype, m, q, k_init, wd, DB, steps, kind)
             if step in (0, 1, m - 1, steps - 1):
                 assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
             assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.5, -2])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("q", [8, 64, 128, 1024, 4096])
+def test_fused_route_takes_tensors_shorter_than_a_quantisation_block(oracle, q, dtype, alpha):
+    """Beside longer ones, in the same launch; from one element to one less than a block."""
+    sizes = sorted({1, 2, 7, 9, q // 2 - 1, q // 2, q - 7, q - 1, q} - {0}) + [20480 + q]
+    opt = _run(oracle, sizes, dtype, 3, q, 0.01, alpha, 0.01, 20480, 5, True, zero_step=2)
+    assert {opt._fusable(p, opt.state[p]) for p in opt.param_groups[0]["params"]} == \
+        {{0.0: 1, 0.5: 3, -2: 4}[alpha]}
+    assert opt._uniform is not None
