@@ -935,23 +935,19 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
     int64_t ws_off = 0;
     // tensors whose window is too large for the one-pass stage are stepped in launches of their own:
     // the longer stage, or block part and window part
-    // (the longer stage takes every shorter window too: few tensors of the usual form ride along in
-    // its launch, as those of smaller classes do)
+    // (few tensors of a shorter form ride along in the longest one's launches, which take every
+    // window, as those of smaller classes do)
     std::vector<char> forms(n_tensors, kOnePass);
     if (!span && !dense && !aux) {
-        bool any_long = false;
-        int64_t usual_blocks = 0;
+        int64_t blocks_of[kWindowForms] = {0, 0, 0};
         for (int i = 0; i < n_tensors; ++i) {
             forms[i] = (char)window_form(tensors[i].d, h, elem_bytes);
-            any_long = any_long || forms[i] == kLong;
-            if (forms[i] == kOnePass) {
-                const Geometry g = geometry(tensors[i].d, h->d_block_size, h->k_init);
-                usual_blocks += g.n_full + (g.tail > 0 ? 1 : 0);
-            }
+            const Geometry g = geometry(tensors[i].d, h->d_block_size, h->k_init);
+            blocks_of[(int)forms[i]] += g.n_full + (g.tail > 0 ? 1 : 0);
         }
-        if (any_long && usual_blocks <= kMergeBlocks)
-            for (int i = 0; i < n_tensors; ++i)
-                if (forms[i] == kOnePass) forms[i] = kLong;
+        const char longest = blocks_of[kApart] ? kApart : blocks_of[kLong] ? kLong : kOnePass;
+        for (int i = 0; i < n_tensors; ++i)
+            if (blocks_of[(int)forms[i]] <= kMergeBlocks) forms[i] = longest;
     }
     std::vector<int> order;
     for (int ci = 0; ci < 4; ++ci)
