@@ -206,13 +206,13 @@ int ma_fused_step_densified(const ma_tensor *tensors /* host */, int n_tensors,
  *      decoupled weight decay);
  *      alpha > 0: Qinv(e1) stays in registers; window -> Adam direction, + alpha * Qinv(e1);
  *      p update; error = Q((1 - alpha) * Qinv(e1)), min_vals, max_vals.
- * With alpha > 0 these are two kernel passes and r travels from the first to the second in g.
- * With alpha == 0 they are one pass: a workgroup publishes its extremes and takes those of its
+ * These are one kernel pass: a workgroup publishes its extremes and takes those of its
  * neighbours as they arrive; it waits for them a bounded time only (MA_SPAN_SPIN_LIMIT polls
  * per neighbour, an environment variable, default 256, 0 = no wait), and a block that gives
- * up leaves r in g and is taken through step 2 by a second launch.  Either way g may hold r
- * instead of the gradient afterwards (the reference's step destroys p.grad as well,
- * MA:190-316).
+ * up leaves r in g and is taken through step 2 by a second launch (with alpha > 0 including
+ * window and parameters).  (Logging steps take two passes, and r travels from the first to
+ * the second in g.)  Either way g may hold r instead of the gradient afterwards (the
+ * reference's step destroys p.grad as well, MA:190-316).
  * The caller advances st['index'] itself.  Conditions (else MA_ERR_NOT_FUSABLE, nothing
  * launched): 0 <= alpha < 1 (MA:18); quant_block_size a multiple of 8, not below
  * min(d, d_block_size), below 2^30 and covering at most 62 of the tensor's top-k blocks

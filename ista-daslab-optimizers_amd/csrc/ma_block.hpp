@@ -3016,7 +3016,7 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
                 list_deferred(item);
             }
             fb.load_params_window(G);
-            fb.update(G);
+            fb.update_in_cells(G);
         }
     };
     auto run = [&](auto &fb, const BlockGeo &G, int item) {
