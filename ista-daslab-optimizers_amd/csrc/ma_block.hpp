@@ -3126,8 +3126,8 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
 // barrier-separated row steps.  One workgroup per top-k block; it reads the window rows
 // (including the one the block kernel has just written) and the parameters, nothing else.
 //
-// Rows that list their entries by increasing coordinate (as every kernel of this library writes
-// them when a block row has more than 512 entries) are cut at the multiples of 1024
+// Rows that list their entries by increasing coordinate (as the block kernels in front of this one
+// write them) are cut at the multiples of 1024
 // coordinates: chunk ch of a row is the stretch table[row][ch] .. table[row][ch + 1] of its
 // entries.  A wave then owns a chunk: its 1024 pairs of sums live in the wave's own 8 KiB of
 // LDS, it adds the rows' stretches in row order (the LDS operations of one wave execute in

@@ -822,8 +822,8 @@ int64_t ma_fused_step_row_cuts(const ma_tensor *tensor, const ma_hyper *hyper) {
     const int rc = fused_check(tensor, hyper);
     if (rc) return rc;
     const Geometry g = geometry(tensor->d, hyper->d_block_size, hyper->k_init);
-    // only rows of more than 512 entries per block are written in coordinate order, which is
-    // what the cuts describe
+    // kept for rows of more than 512 entries per block; where shorter ones cross the boundaries the
+    // window kernel finds by itself, in one look at every entry
     if (!window_apart(tensor->d, hyper, hyper->dtype == MA_BF16 ? 2 : 4) || g.k_many <= kWG)
         return 0;
     return row_cut_words(tensor->d, hyper);
