@@ -172,7 +172,8 @@ int ma_fused_step(const ma_tensor *tensors /* host */, int n_tensors,
 int ma_fused_step_check(const ma_tensor *tensor /* host */, const ma_hyper *hyper /* host */);
 
 /* ma_fused_step steps tensors whose window has about as many entries as the tensor has
- * coordinates (more than 2560 entries per top-k block, or more than 16 rows) in two launches; the
+ * coordinates (more than 2560 entries per top-k block, or more than 16 rows; bf16 data of up to 15
+ * rows whose older ones make at most 1024 loads of four entries still take one) in two launches; the
  * second walks every window row in stretches of 512 coordinates and must know where each row
  * crosses those boundaries.  With tensor->row_cuts == NULL it finds out by reading all rows at
  * every step.  With a buffer of m x (this function's value) uint16 words, set to 0xffff before
