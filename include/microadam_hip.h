@@ -183,8 +183,8 @@ int ma_fused_step_check(const ma_tensor *tensor /* host */, const ma_hyper *hype
  * (r * blocks + b) * cuts_per_block + c, cuts_per_block = ceil(min(d, d_block_size) / 512) + 1.
  * A row whose first cut is 0xffff is taken as unknown and read in full.  Whoever else rewrites a
  * window row of the tensor (another entry point, a loaded checkpoint) must set that row's
- * words to 0xffff again.  Returns the words per row, 0 if the tensor's step would not use them,
- * negative MA_ERR_* for bad arguments. */
+ * words to 0xffff again.  Returns the words per row, 0 if the tensor's step would not use them
+ * (tensor->row_cuts is not looked at then), negative MA_ERR_* for bad arguments. */
 int64_t ma_fused_step_row_cuts(const ma_tensor *tensor, const ma_hyper *hyper);
 
 

@@ -817,15 +817,18 @@ static int64_t row_cut_words(int64_t d, const ma_hyper *h) {
     return blocks * ((g.dbs + kWinChunk - 1) / kWinChunk + 1);
 }
 
+// Does ma_fused_step use a tensor's cache of chunk cuts?  It is kept for tensors that take two
+// launches by their own sizes, with rows of more than 512 entries per block; where shorter rows cross
+// the boundaries the window kernel finds by itself, in one look at every entry.
+static bool keeps_row_cuts(int64_t d, const ma_hyper *h, int elem_bytes) {
+    return window_apart(d, h, elem_bytes) && geometry(d, h->d_block_size, h->k_init).k_many > kWG;
+}
+
 int64_t ma_fused_step_row_cuts(const ma_tensor *tensor, const ma_hyper *hyper) {
     if (!tensor || !hyper) return MA_ERR_ARG;
     const int rc = fused_check(tensor, hyper);
     if (rc) return rc;
-    const Geometry g = geometry(tensor->d, hyper->d_block_size, hyper->k_init);
-    // kept for rows of more than 512 entries per block; where shorter ones cross the boundaries the
-    // window kernel finds by itself, in one look at every entry
-    if (!window_apart(tensor->d, hyper, hyper->dtype == MA_BF16 ? 2 : 4) || g.k_many <= kWG)
-        return 0;
+    if (!keeps_row_cuts(tensor->d, hyper, hyper->dtype == MA_BF16 ? 2 : 4)) return 0;
     return row_cut_words(tensor->d, hyper);
 }
 
@@ -1047,8 +1050,11 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             D.blk0 = 0;
             D.ws = span ? reinterpret_cast<float *>(static_cast<char *>(ws) + ws_here)
                    : (aux & kAuxQuantErr) ? static_cast<float *>(t.quant_err)
-                   : forms[i] == kApart ? reinterpret_cast<float *>(t.row_cuts)
-                              : nullptr;
+                   // (not of every tensor in the two launches: one that rides along there, or whose
+                   // rows are short, has no cache, whatever its row_cuts points to)
+                   : forms[i] == kApart && keeps_row_cuts(t.d, h, elem_bytes)
+                       ? reinterpret_cast<float *>(t.row_cuts)
+                       : nullptr;
             items += nb;
             if (t.d < h->d_block_size) ++short_items;  // (nb == 1, and only short ones follow)
             if (g.dbs > dbs_max) dbs_max = (int)g.dbs;

@@ -1228,3 +1228,50 @@ def test_fused_route_takes_tensors_shorter_than_a_quantisation_block(oracle, q, 
     assert {opt._fusable(p, opt.state[p]) for p in opt.param_groups[0]["params"]} == \
         {{0.0: 1, 0.5: 3, -2: 4}[alpha]}
     assert opt._uniform is not None
+
+
+@pytest.mark.parametrize("sizes,dtype,m,k_init", [
+    ([20480 * 2 + 9001, 768, 300, 4096], torch.bfloat16, 10, 0.03),  # one tensor with cuts, three beside it
+    ([20480 + 9001, 768, 300, 4096], torch.float32, 10, 0.03),
+    ([20480 * 2 + 9001, 4096], torch.bfloat16, 18, 0.01),            # two launches, short rows: no cuts
+    ([20480 + 9001], torch.float32, 18, 0.01),
+])
+def test_row_cuts_that_no_step_asks_for_are_left_alone(sizes, dtype, m, k_init):
+    """Tensors that ma_fused_step takes in two launches although ma_fused_step_row_cuts answers 0 for
+    them, because they ride along with a longer one or because their rows are short: a row_cuts pointer
+    they come with is neither written nor read, and the step is that without the pointers."""
+    import ctypes
+    from ista_daslab_optimizers import MicroAdam, _hip
+    gen = torch.Generator().manual_seed(m)
+    start = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    opts, lists = [], []
+    for _ in range(2):
+        params = [torch.nn.Parameter(p.clone().cuda()) for p in start]
+        opts.append(MicroAdam(params, m=m, lr=1e-3, quant_block_size=64, k_init=k_init))
+        lists.append(params)
+    guards = {}
+    for step in range(m + 2):
+        grads = [(torch.randn(n, generator=gen) * 1e-2).to(dtype).cuda() for n in sizes]
+        for opt, params in zip(opts, lists):
+            for p, g in zip(params, grads):
+                p.grad = g
+            opt.step()
+        if step == 0:
+            opt, (table,) = opts[0], opts[0]._tables.values()
+            for i, e in enumerate(table.entries):
+                probe, h = opt._probe(e.p, e.st)
+                words = _hip.lib.ma_fused_step_row_cuts(ctypes.byref(probe), ctypes.byref(h))
+                assert (words > 0) == (e.cuts is not None) == (m == 10 and i == 0)
+                if words == 0:
+                    # (longer than the cuts of such a tensor would be: nothing is written past it)
+                    blocks = -(-sizes[i] // 20480)
+                    guards[i] = torch.full((m * blocks * 42,), 0x5555, dtype=torch.int16,
+                                           device="cuda")
+                    table.records[i].row_cuts = guards[i].data_ptr()
+    assert guards and all(torch.all(g == 0x5555) for g in guards.values())
+    (now,) = opts[0]._tables.values()
+    assert now is table and all(table.records[i].row_cuts == g.data_ptr() for i, g in guards.items())
+    for a, b in zip(*lists):
+        assert torch.equal(a.data, b.data)
+        for key in ("error", "min_vals", "max_vals"):
+            assert torch.equal(opts[0].state[a][key], opts[1].state[b][key]), key
