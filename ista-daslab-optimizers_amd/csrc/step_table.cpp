@@ -93,7 +93,22 @@ PyObject *refresh(PyObject *, PyObject *args) {
     Py_RETURN_TRUE;
 }
 
-// advance(states, m): state['index'] = (state['index'] + 1) % m (micro_adam.py:211)
+// (value + 1) % m as the interpreter forms it, for ring positions that are not plain integers
+PyObject *advanced(PyObject *value, long m) {
+    Py_INCREF(value);
+    PyObject *one = PyLong_FromLong(1), *length = PyLong_FromLong(m);
+    PyObject *sum = one && length ? PyNumber_Add(value, one) : nullptr;
+    PyObject *next = sum ? PyNumber_Remainder(sum, length) : nullptr;
+    Py_XDECREF(one);
+    Py_XDECREF(length);
+    Py_XDECREF(sum);
+    Py_DECREF(value);
+    return next;
+}
+
+// advance(states, m): state['index'] = (state['index'] + 1) % m (micro_adam.py:211), whatever kind of
+// number the position is: the step has been launched, and what it took must not fail here (a
+// framework that re-types optimizer state may have made a float or a tensor of it).
 PyObject *advance(PyObject *, PyObject *args) {
     PyObject *states;
     long m;
@@ -109,9 +124,10 @@ PyObject *advance(PyObject *, PyObject *args) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_KeyError, "index");
             return nullptr;
         }
-        const long row = PyLong_AsLong(index);
-        if (row == -1 && PyErr_Occurred()) return nullptr;
-        PyObject *next = PyLong_FromLong((row + 1) % m);
+        const long row = PyLong_CheckExact(index) ? PyLong_AsLong(index) : -1;
+        if (row == -1) PyErr_Clear();
+        PyObject *next =
+            row >= 0 && row < m ? PyLong_FromLong((row + 1) % m) : advanced(index, m);
         if (!next) return nullptr;
         const int rc = PyDict_SetItem(st, key_index, next);
         Py_DECREF(next);

@@ -123,6 +123,25 @@ def test_row_cuts_query():
     assert _hip.lib.ma_fused_step_row_cuts(None, None) == _hip.MA_ERR_ARG
 
 
+def test_ring_positions_of_every_kind_move_on():
+    """Behind a launch: plain integers, and what a framework that re-types optimizer state makes of
+    them, as (index + 1) % m of the interpreter; nothing stops half-way through the list."""
+    import numpy as np
+    from ista_daslab_optimizers import _step_table
+    m = 3
+    positions = [0, 2, 1.0, 2.0, True, np.int64(2), np.float32(1), torch.tensor(2), torch.tensor(1.0), -1,
+                 7, 2 ** 70]
+    states = [{"index": i} for i in positions]
+    _step_table.advance(states, m)
+    for st, i in zip(states, positions):
+        want = (i + 1) % m
+        assert type(st["index"]) is type(want) and st["index"] == want, i
+    with pytest.raises(KeyError):
+        _step_table.advance([{}], m)
+    with pytest.raises(ValueError):
+        _step_table.advance([], 0)
+
+
 def test_logged_step_argument_checks():
     """Host-only: the size of the per-block buffer a logging step needs, and the refusals that
     come before any launch."""

@@ -1275,3 +1275,29 @@ def test_row_cuts_that_no_step_asks_for_are_left_alone(sizes, dtype, m, k_init):
         assert torch.equal(a.data, b.data)
         for key in ("error", "min_vals", "max_vals"):
             assert torch.equal(opts[0].state[a][key], opts[1].state[b][key]), key
+
+
+@pytest.mark.parametrize("kind", [float, np.int64, lambda i: torch.tensor(float(i))],
+                         ids=["float", "numpy", "tensor"])
+def test_ring_positions_of_another_kind_step_as_before(kind):
+    """A ring position that something re-typed between two steps: the list goes through the walk, and
+    all positions have moved on behind it."""
+    from ista_daslab_optimizers import MicroAdam
+    lists, opts = [], []
+    for _ in range(2):
+        gen = torch.Generator().manual_seed(5)
+        lists.append([torch.nn.Parameter((torch.randn(n, generator=gen) * 0.02).cuda())
+                      for n in (500, 3000, 64)])
+        opts.append(MicroAdam(lists[-1], m=3, lr=1e-3, quant_block_size=64))
+    for step in range(5):
+        grads = [torch.randn(p.numel(), generator=gen).cuda() for p in lists[0]]
+        for opt, params in zip(opts, lists):
+            for p, g in zip(params, grads):
+                p.grad = g
+            if opt is opts[0] and step == 2:
+                st = opt.state[params[1]]
+                st["index"] = kind(st["index"])
+            opt.step()
+    for a, b in zip(*lists):
+        assert torch.equal(a.data, b.data)
+        assert opts[0].state[a]["index"] == opts[1].state[b]["index"] == 2
