@@ -75,6 +75,7 @@ PyObject *refresh(PyObject *, PyObject *args) {
                     Py_RETURN_FALSE;
                 const long row = PyLong_AsLong(index);
                 if (row == -1 && PyErr_Occurred()) return nullptr;
+                if (row != static_cast<int32_t>(row)) Py_RETURN_FALSE;  // (refused by the walk)
                 void *pp = p.data_ptr(), *gp = g.data_ptr();
                 if (((reinterpret_cast<uintptr_t>(pp) | reinterpret_cast<uintptr_t>(gp)) & 15) != 0)
                     Py_RETURN_FALSE;

@@ -1301,3 +1301,19 @@ def test_ring_positions_of_another_kind_step_as_before(kind):
     for a, b in zip(*lists):
         assert torch.equal(a.data, b.data)
         assert opts[0].state[a]["index"] == opts[1].state[b]["index"] == 2
+
+
+def test_ring_positions_outside_32_bits_are_refused():
+    """2^32 + 1 in a list that goes through one table: refused in front of the launch, not taken for
+    row 1."""
+    from ista_daslab_optimizers import MicroAdam
+    p = torch.nn.Parameter(torch.ones(500, device="cuda"))
+    opt = MicroAdam([p], m=3, lr=1e-3, quant_block_size=64)
+    for _ in range(2):
+        p.grad = torch.ones_like(p)
+        opt.step()
+    opt.state[p]["index"] = 2 ** 32 + 1
+    before = p.data.clone()
+    with pytest.raises(OverflowError):
+        opt.step()
+    assert torch.equal(p.data, before) and opt.state[p]["index"] == 2 ** 32 + 1
