@@ -31,8 +31,15 @@ import torch.distributed as dist
 import ista_daslab_cuda_micro_adam as _ext_quant
 import ista_daslab_cuda_tools as _ext_tools
 
-from .. import _hip, _step_table
+from .. import _hip
 from ..tools import block_split, get_first_device, get_gpu_mem_usage
+
+try:
+    from .. import _step_table
+except ImportError as e:  # missing, or built for another interpreter or torch
+    raise ImportError("the extension _step_table cannot be loaded: build it with `make -B -C "
+                      "ista-daslab-optimizers_amd/csrc table PYTHON=<this interpreter>` "
+                      f"(a C++ compiler and this interpreter's torch). {e}") from e
 
 try:  # logging is optional here; the reference imports wandb unconditionally (micro_adam.py:5)
     import wandb

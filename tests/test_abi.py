@@ -187,3 +187,22 @@ def test_spanning_step_check_and_workspace():
     # too small a workspace is refused before anything is launched
     rc = _hip.lib.ma_spanning_step(arr, 2, ctypes.byref(h), 0.5, 0x10000, 16, None)
     assert rc == -1  # MA_ERR_ARG
+
+
+def test_the_c_library_builds_without_an_interpreter():
+    """`make` for the C ABI alone asks no Python and compiles nothing against torch."""
+    import subprocess
+    out = subprocess.run(["make", "-n", "-B", "PYTHON=/nonexistent/python", "-C",
+                          os.path.join(ROOT, "ista-daslab-optimizers_amd", "csrc")],
+                         capture_output=True, text=True)
+    assert out.returncode == 0 and "libmicroadam_hip.so" in out.stdout
+    assert "step_table" not in out.stdout and "/nonexistent" not in out.stdout + out.stderr
+
+
+def test_missing_step_table_says_how_to_build_it():
+    import subprocess
+    import sys
+    code = ("import sys; sys.path.insert(0, %r); sys.modules['ista_daslab_optimizers._step_table'] = None\n"
+            "import ista_daslab_optimizers" % os.path.join(ROOT, "ista-daslab-optimizers_amd"))
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert out.returncode != 0 and "make -B -C ista-daslab-optimizers_amd/csrc table" in out.stderr
