@@ -116,7 +116,8 @@ def test_row_cuts_query():
     assert words(20480 * 2, 20, 0.05) == 2 * 41
     # the window of the 7B configuration fits the one-pass stage
     assert words(20480 * 2 + 4096, 10, 0.01) == 0
-    # two launches, but rows of at most 512 entries are not listed by coordinate
+    # two launches, but where rows of at most 512 entries cross the boundaries the second one finds
+    # by itself
     assert words(20480 * 2, 20, 0.01) == 0
     # a tensor shorter than a top-k block: one block, ceil(d / 512) + 1 cuts
     assert words(16384, 20, 0.05) == 33

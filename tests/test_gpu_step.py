@@ -76,8 +76,8 @@ CASES = [
     ([20480 * 2 + 4096, 20480], torch.bfloat16, 20, 64, 0.05, 0.0, 0.01, 20480, 22),
     ([20480 + 8192], torch.bfloat16, 24, 32, 0.05, 0.0, 0.0, 20480, 26),
     ([20480 * 2 + 8192], torch.float32, 20, 32, 0.05, 0.0, 0.0, 20480, 22),
-    # more rows than the one-pass stage takes, but short block rows (1 %), which the fast
-    # selections do not list by coordinate: two launches, the window kernel's general form
+    # more rows than the one-pass stage takes, but short block rows (1 %): two launches, without a
+    # cache of chunk cuts (rows out of order: test_window_kernel_over_rows_out_of_order)
     ([20480 * 2 + 8192, 4096], torch.bfloat16, 18, 64, 0.01, 0.0, 0.0, 20480, 21),
     # a fifth of every block selected: a row has about 100 entries per 512 coordinates, more
     # than the window kernel's 64 lanes take in one go
@@ -100,7 +100,7 @@ def test_step_matches_oracle(oracle, sizes, dtype, m, q, k_init, alpha, wd, DB, 
 
 
 GENERAL_CASES = [
-    # alpha > 0, odd quantisation blocks, d < q: only the op-by-op route applies
+    # alpha > 0 or d < q with odd quantisation blocks: only the op-by-op route applies
     ([4100, 33], torch.bfloat16, 3, 1000, 0.01, 0.5, 0.0, 1024, 7),
     ([999], torch.float32, 2, 100, 0.03, 0.25, 0.01, 400, 5),
     ([20480 * 3 + 77], torch.bfloat16, 4, 100001, 0.01, 0.5, 0.0, 20480, 6),
@@ -137,7 +137,7 @@ def test_step_quant_err_route(oracle, sizes, dtype, m, q, k_init, alpha, wd, DB,
 
 
 SPANNING_CASES = [
-    # quantisation blocks at least as long as the top-k blocks: two-pass route
+    # quantisation blocks at least as long as the top-k blocks: spanning route
     ([20480 * 5 + 77], torch.bfloat16, 10, 100000, 0.01, 0.5, 0.0, 20480, 12),
     ([20480 * 12 + 4096, 4096, 1000], torch.bfloat16, 4, 24576, 0.01, 0.3, 0.01, 20480, 8),
     ([5000, 3000], torch.float32, 3, 2048, 0.02, 0.25, 0.0, 1024, 6),
@@ -146,7 +146,7 @@ SPANNING_CASES = [
     # alpha == 0 with long quantisation blocks (the reference's documented quant_block_size)
     ([20480 * 5 + 77, 4096], torch.bfloat16, 10, 100000, 0.01, 0.0, 0.0, 20480, 12),
     ([5000, 3000], torch.float32, 3, 2048, 0.02, 0.0, 0.01, 1024, 6),
-    ([50, 20], torch.bfloat16, 3, 64, 0.1, 0.0, 0.0, 20480, 4),       # d < q
+    ([50, 20], torch.bfloat16, 3, 64, 0.1, 0.0, 0.0, 20480, 4),       # d < q: the fused route
 ]
 
 
@@ -857,6 +857,7 @@ def test_spanning_route_takes_short_vectors(oracle, q, dtype, alpha):
 @pytest.mark.parametrize("sizes,dtype,m,k_init", [
     ([20480 * 2 + 8192], torch.bfloat16, 20, 0.03),        # partial block: 246 entries
     ([20480 + 4096, 20480], torch.float32, 20, 0.025),     # 512 entries a block
+    ([20480 * 2], torch.bfloat16, 20, 0.01),               # full blocks of 205 entries
 ])
 def test_logging_steps_write_dense_windows_rows_by_coordinate(sizes, dtype, m, k_init):
     """Windows that the ordinary step takes in two launches: the second one counts on block rows
@@ -876,7 +877,6 @@ def test_logging_steps_write_dense_windows_rows_by_coordinate(sizes, dtype, m, k
         for p in params:
             st = opt.state[p]
             row, many = st["I"][step % m].long().cpu(), st["k_block_size_many"]
-            # (full bf16 blocks of at most 512 entries are not listed by coordinate by any step)
             for part in row.split(many):
                 assert torch.all(part[1:] > part[:-1]), (step, len(part))
 
@@ -1317,3 +1317,105 @@ def test_ring_positions_outside_32_bits_are_refused():
     with pytest.raises(OverflowError):
         opt.step()
     assert torch.equal(p.data, before) and opt.state[p]["index"] == 2 ** 32 + 1
+
+
+RIDING_CASES = [
+    # a tensor that takes two launches by its sizes, and short ones of a single-launch form beside it
+    ([20480 * 2 + 9001, 768, 300], torch.bfloat16, 10, 0.03),
+    ([20480 + 9001, 768, 300], torch.float32, 10, 0.03),
+    ([20480 * 2 + 9001, 768, 300], torch.bfloat16, 16, 0.03),
+    ([20480 + 9001, 768, 300], torch.float32, 16, 0.03),
+    # both single-launch forms beside it, one of them in a full block of a smaller class when alone
+    ([20480 + 9001, 12288, 12000, 4096, 5001], torch.bfloat16, 15, 0.02),
+    # more short tensors than a launch holds: the second launch has short ones alone
+    ([20480 + 9001] + [300 + i for i in range(170)], torch.bfloat16, 10, 0.03),
+]
+
+
+@pytest.mark.parametrize("sizes,dtype,m,k_init", RIDING_CASES)
+def test_short_tensors_beside_dense_windows(oracle, sizes, dtype, m, k_init):
+    """They ride along in the two launches of the longer tensor.  Without its gradient in one step
+    they take their own form, whose rows are in no particular order, and ride along again over those
+    rows afterwards."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(m)
+    cpu = [(torch.randn(n, generator=gen) * 0.02).to(dtype) for n in sizes]
+    oparams = [to_np(p) for p in cpu]
+    oref = oracle.OracleMicroAdam(oparams, m, 1e-3, 64, k_init, 0.0, weight_decay=0.01, d_block_size=20480)
+    params = [torch.nn.Parameter(p.clone().cuda()) for p in cpu]
+    opt = MicroAdam(params, m=m, lr=1e-3, quant_block_size=64, k_init=k_init, weight_decay=0.01)
+    for step in range(m + 4):
+        grads = [(torch.randn(n, generator=gen) * 1e-2).to(dtype) for n in sizes]
+        for p, g in zip(params, grads):
+            p.grad = g.clone().cuda()
+        if step in (3, m + 1):
+            params[0].grad = grads[0] = None
+        opt.step()
+        oref.step([None if g is None else to_np(g) for g in grads])
+        for i, p in enumerate(params):
+            assert opt._entries[p].route == 1
+            if step in (0, 3, 4, m + 1, m + 2, m + 3):
+                assert_state_equal(opt.state[p], oref.state[i], f"step {step + 1} tensor {i}")
+            assert np.array_equal(to_np(p.data), oparams[i]), (step, i)
+
+
+@pytest.mark.parametrize("why", ["one turn", "odd address"])
+@pytest.mark.parametrize("n", [20480 * 2 + 17100, 18001])
+def test_longer_windows_that_fall_back_to_ranges(oracle, n, why):
+    """Windows of the longer one-pass stage that it gives up.  "one turn": the large gradients lie on
+    every 16th coordinate, the same ones at every step, so that all 3000 entries that share a
+    coordinate fall into one turn of its queue; "odd address": the window begins on an odd entry."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(n)
+    m, dtype = 15, torch.bfloat16
+    start = (torch.randn(n, generator=gen) * 0.02).to(dtype)
+    oparams = [to_np(start)]
+    oref = oracle.OracleMicroAdam(oparams, m, 1e-3, 64, 0.01, 0.0, weight_decay=0.01, d_block_size=20480)
+    p = torch.nn.Parameter(start.clone().cuda())
+    opt = MicroAdam([p], m=m, lr=1e-3, quant_block_size=64, weight_decay=0.01)
+    for step in range(m + 3):
+        g = torch.randn(n, generator=gen) * 1e-2
+        if why == "one turn":
+            at = torch.arange(n)
+            g[(at % 20480 % 16 == 0) & (at % 20480 < 16 * 200)] *= 100
+        p.grad = g.to(dtype).cuda()
+        opt.step()
+        oref.step([to_np(g.to(dtype))])
+        st = opt.state[p]
+        if step == 0 and why == "odd address":
+            for key in ("I", "V"):
+                flat = torch.empty(st[key].numel() + 1, dtype=st[key].dtype, device="cuda")
+                st[key] = flat[1:].view(st[key].shape).copy_(st[key])
+                assert st[key].data_ptr() % 4 == 2
+            opt._tables.clear()
+            opt._uniform = None
+        assert opt._entries[p].route == 1
+        assert_state_equal(st, oref.state[0], f"step {step + 1}")
+        assert np.array_equal(to_np(p.data), oparams[0]), step
+
+
+def test_window_kernel_over_rows_out_of_order(oracle):
+    """Two launches over a window with rows that are not listed by coordinate, as a checkpoint may hold
+    them: the window kernel's general form."""
+    from ista_daslab_optimizers import MicroAdam
+    gen = torch.Generator().manual_seed(18)
+    n, m, dtype = 20480 * 2 + 8192, 18, torch.bfloat16
+    start = (torch.randn(n, generator=gen) * 0.02).to(dtype)
+    oparams = [to_np(start)]
+    oref = oracle.OracleMicroAdam(oparams, m, 1e-3, 64, 0.01, 0.0, d_block_size=20480)
+    p = torch.nn.Parameter(start.clone().cuda())
+    opt = MicroAdam([p], m=m, lr=1e-3, quant_block_size=64)
+    for step in range(m + 3):
+        g = (torch.randn(n, generator=gen) * 1e-2).to(dtype)
+        p.grad = g.cuda()
+        opt.step()
+        oref.step([to_np(g)])
+        st = opt.state[p]
+        assert opt._entries[p].route == 1 and opt._entries[p].cuts is None
+        assert_state_equal(st, oref.state[0], f"step {step + 1}")
+        assert np.array_equal(to_np(p.data), oparams[0]), step
+        if step % 5 == 1:  # this step's row of every block, backwards
+            many = st["k_block_size_many"]
+            for key in ("I", "V"):
+                row = st[key][step % m]
+                row.copy_(torch.cat([part.flip(0) for part in row.split(many)]))
