@@ -845,6 +845,12 @@ enum { kWholeStep = 0, kBlockPart = 1, kWindowPart = 2, kLongStep = 3 };
 // them next to longer tensors, a launch of their own costs more than that: up to this many
 // blocks of a smaller class ride along in the call's largest class instead.
 constexpr int64_t kMergeBlocks = 768;
+// Tensors of the longer one-pass window stage beside ones that take two launches: they gain by a
+// launch of their own sooner, as the two launches cost a block about twice as much.  One tensor of
+// 40960 and n of 12000 elements, 15 rows of 2 %, in the longer stage's launch and riding along:
+// n = 128 65 and 53 us a step, 256 94 and 99, 400 123 and 146, 700 179 and 239; n of 14000, 10 rows of
+// 3 %: 128 62 and 44, 256 96 and 88, 400 130 and 133.
+constexpr int64_t kMergeLongBlocks = 256;
 
 // Blocks (work items) a list of tensors makes; -1 for a tensor without elements.
 static int64_t count_blocks(const ma_tensor *tensors, int n_tensors, const ma_hyper *h) {
@@ -948,9 +954,14 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
             const Geometry g = geometry(tensors[i].d, h->d_block_size, h->k_init);
             blocks_of[(int)forms[i]] += g.n_full + (g.tail > 0 ? 1 : 0);
         }
-        const char longest = blocks_of[kApart] ? kApart : blocks_of[kLong] ? kLong : kOnePass;
-        for (int i = 0; i < n_tensors; ++i)
-            if (blocks_of[(int)forms[i]] <= kMergeBlocks) forms[i] = longest;
+        // where each form's tensors go: the longer stage's stay unless a longer form has them ride
+        char rides[kWindowForms] = {kOnePass, kApart, kLong};
+        if (blocks_of[kApart] && blocks_of[kLong] <= kMergeLongBlocks) rides[kLong] = kApart;
+        if (blocks_of[kOnePass] <= kMergeBlocks) {
+            if (blocks_of[kLong]) rides[kOnePass] = rides[kLong];
+            else if (blocks_of[kApart]) rides[kOnePass] = kApart;
+        }
+        for (int i = 0; i < n_tensors; ++i) forms[i] = rides[(int)forms[i]];
     }
     std::vector<int> order;
     for (int ci = 0; ci < 4; ++ci)

@@ -1329,6 +1329,8 @@ RIDING_CASES = [
     ([20480 + 9001, 12288, 12000, 4096, 5001], torch.bfloat16, 15, 0.02),
     # more short tensors than a launch holds: the second launch has short ones alone
     ([20480 + 9001] + [300 + i for i in range(170)], torch.bfloat16, 10, 0.03),
+    # more tensors of the longer one-pass stage than ride along: the shortest ride along with them
+    ([20480 + 9001] + [8600] * 257 + [300, 301, 4096], torch.bfloat16, 15, 0.02),
 ]
 
 
