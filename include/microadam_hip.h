@@ -159,7 +159,7 @@ typedef struct ma_hyper {
  * top-k block: a = g + Qinv(e); block top-k -> I[index], V[index]; residual -> new min/max
  * and 4-bit codes; window -> Adam direction; p update (with decoupled weight decay).  (Tensors
  * whose window is about as dense as the tensor take two launches, the second for the window and
- * the parameters: see ma_fused_step_row_cuts.)  The
+ * the parameters: see ma_fused_step_row_cuts; a few shorter ones of the list ride along in them.)  The
  * caller advances st['index'] (MA:211) itself.  Conditions (else MA_ERR_NOT_FUSABLE, nothing
  * launched): quant_block_size a power of two in [8, 4096] that divides d_block_size (or
  * d <= d_block_size; a tensor may be shorter than a quantisation block); p and g 16-byte aligned,

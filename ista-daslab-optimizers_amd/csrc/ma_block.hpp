@@ -1860,7 +1860,8 @@ struct FusedBlock {
     // neighbours, neighbouring blocks are dispatched together, and every workgroup publishes
     // before it waits, so the wait is short; it is bounded all the same (spin_limit polls), and
     // a workgroup that gives up stores its residual in the gradient buffer and lists its block:
-    // a second launch takes the listed blocks through the second pass of the two-pass form (alpha > 0: window and parameters too).
+    // a second launch takes the listed blocks through the second pass of the two-pass form (alpha > 0:
+    // window and parameters too).
     // The old statistics of a quantisation block are overwritten by the block that holds its
     // first element only after that block has seen all blocks of the quantisation block
     // published, i.e. after all of them have read the old statistics.
@@ -2190,7 +2191,9 @@ struct FusedBlock {
     __device__ __forceinline__ void span_publish(const BlockGeo &G, const Span &S) {
         const int n = FULL ? C * kRound : G.n;
         float mn[2] = {INFINITY, INFINITY}, mx[2] = {-INFINITY, -INFINITY};
-        if (FULL && S.bnd == 0x7fffffff) {  // (four blocks in five at q = 100000)
+        // (four blocks in five at q = 100000, without a choice an element; the alpha == 0 kernel, which
+        // waits for memory, takes the same time either way)
+        if (FULL && S.bnd == 0x7fffffff) {
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 float x[8];
@@ -3127,13 +3130,12 @@ __global__ __launch_bounds__(kWG, MIN_WAVES) void span_step_kernel(FusedParams P
 // (including the one the block kernel has just written) and the parameters, nothing else.
 //
 // Rows that list their entries by increasing coordinate (as the block kernels in front of this one
-// write them) are cut at the multiples of 1024
-// coordinates: chunk ch of a row is the stretch table[row][ch] .. table[row][ch + 1] of its
-// entries.  A wave then owns a chunk: its 1024 pairs of sums live in the wave's own 8 KiB of
-// LDS, it adds the rows' stretches in row order (the LDS operations of one wave execute in
-// program order and a row names a coordinate once, so no barrier is needed and every sum is
-// formed in row order, as compute_microadam_update forms it), and lane l steps the 16
-// parameters at 16 l of the chunk.
+// write them) are cut at the multiples of 512 coordinates: chunk ch of a row is the stretch
+// table[row][ch] .. table[row][ch + 1] of its entries.  A wave then owns a chunk: its 512 pairs of
+// sums live in the wave's own 4 KiB of LDS, it adds the rows' stretches in row order (the LDS
+// operations of one wave execute in program order and a row names a coordinate once, so no barrier
+// is needed and every sum is formed in row order, as compute_microadam_update forms it), and lane l
+// steps the 8 parameters at 8 l of the chunk.
 // A block in which some row is not in increasing order, or holds an index outside the block,
 // takes the general form instead: coordinate ranges of 4096 with a barrier after every row.
 //   LDS: the kSh* words | table: rows x (chunks + 1) int32 at L.off_slot, row stride

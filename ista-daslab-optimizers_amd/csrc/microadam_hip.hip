@@ -944,8 +944,8 @@ static int step_impl(const ma_tensor *tensors, int n_tensors, const ma_hyper *h,
     int64_t ws_off = 0;
     // tensors whose window is too large for the one-pass stage are stepped in launches of their own:
     // the longer stage, or block part and window part
-    // (few tensors of a shorter form ride along in the longest one's launches, which take every
-    // window, as those of smaller classes do)
+    // (few tensors of a shorter form ride along in a longer one's launches, which take every window,
+    // as those of smaller classes do)
     std::vector<char> forms(n_tensors, kOnePass);
     if (!span && !dense && !aux) {
         int64_t blocks_of[kWindowForms] = {0, 0, 0};
